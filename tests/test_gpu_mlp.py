@@ -58,6 +58,30 @@ def test_forward_and_grad_match_oracle(ctx):
     assert np.array_equal(g, g2.cpu().numpy())
 
 
+@pytest.mark.parametrize("batch", [1, 31, 32, 33, 300, 32 * 256 - 1, 32 * 256 + 1, 32 * 512 + 45])
+def test_grad_at_tile_edges(ctx, batch):
+    """Batches around the gradient kernel's 32-sample tiles and around the
+    point (256 tiles) from which a wave takes several tiles.  A term of the
+    gradient passes through about 250 rounded operations (three 32-term layers
+    forward and back, the sum over a tile and over the partials), each 6e-8
+    relative: 1.5e-5, times about 4 for cancellation among the terms."""
+    rng = np.random.default_rng(batch)
+    p = (rng.normal(0, 0.3, MR.NP)).astype(np.float32)
+    X = rng.uniform(-1, 1, (batch, MR.NF)).astype(np.float32)
+    T = rng.normal(0, 1, (batch, MR.NC)).astype(np.float32)
+    Mk = (rng.uniform(0, 1, (batch, MR.NC)) > 0.2).astype(np.float32)
+    Mk[0, 0] = 1
+    disp = D.Dispatcher(ctx, params=p)
+    Xd, Td, Md = (torch.from_numpy(a).cuda() for a in (X, T, Mk))
+    announce("grad tile edges", batch)
+    loss, g = disp.grad(Xd, Td, Md)
+    loss_ref, g_ref = MR.grad(p, X, T, Mk)
+    assert abs(float(loss.item()) - loss_ref) <= 6e-5 * abs(loss_ref)
+    assert np.abs(g.cpu().numpy() - g_ref).max() <= 6e-5 * np.abs(g_ref).max()
+    _, g2 = disp.grad(Xd, Td, Md)
+    assert torch.equal(g, g2)
+
+
 def test_training_reduces_loss(ctx):
     """Fit a smooth teacher function of the features with the HIP Adam steps."""
     rng = np.random.default_rng(5)

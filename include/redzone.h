@@ -70,7 +70,7 @@ typedef struct rz_ctx rz_ctx;
 /* Launch shape.  A step is wg_size * items pairs; the removal list is cut into
  * slices of whole steps, one workgroup (or queue item) per slice. */
 typedef struct rz_tile_config {
-  int32_t wg_size;     /* 256 or 512 */
+  int32_t wg_size;     /* 256 or 512 (variants 5 and 7 also 1024) */
   int32_t items;       /* items per thread per step: 2, 4, 8, 16 (variants 0/1); 4 or 8 (variant 2, batches) */
   int32_t max_slices;  /* variants 0/1/3/4/6: upper bound on slices (workgroups of the move step);
                           batches: queues in use, 1, 2 or 4 (any other value: one per XCD, 8); 16: 8 queues
@@ -87,7 +87,10 @@ typedef struct rz_tile_config {
                           5 = dense form: head writes grouped by destination bin, then one scatter per bin
                               (for k/n of several percent and up),
                           6 = variant 4 in one launch: mark workgroups first, move slices after them wait for
-                              the marks (same LDS limit and fallback as variant 4) */
+                              the marks (same LDS limit and fallback as variant 4),
+                          7 = one launch of independent workgroups, for k up to 2^17 (wg_size 256 or 512 with
+                              1, 2 or 4 items, or 1024 with 1 or 2; a slice is one step and max_slices is not
+                              used; with premarked tails or RZ_COOPERATIVE: 256 x 4 of variant 4 or 1) */
   int32_t slice_steps; /* variant 2 and batches: steps per slice (0 = 4); variant 5: log2 of the target
                           number of destination bins, 5..10 (0 = 9); variant 6: log2 of the removals
                           each mark workgroup takes, 8..16 (0 = 12) */
@@ -99,7 +102,7 @@ typedef struct rz_tile_config {
  * ceil(k/32) words with bit r-(n-k) set for every removal r >= n-k and no
  * other bit; the call skips the mark step and leaves the bitmap zero.  cfg may
  * be null (the tuned table); shapes whose single launch includes the mark
- * (variants 1-3 and 6) run as variant 4.  RZ_SORTED is ignored and RZ_STATS counts
+ * (variants 1-3, 6 and 7) run as variant 4.  RZ_SORTED is ignored and RZ_STATS counts
  * no tail removals (the marks were not made here).  Has no counterpart in the
  * reference: its phase 1 always scans the list (redzone.hxx:698-707). */
 rz_status rz_remove_premarked(rz_ctx* ctx, void* d_data, int64_t n, uint32_t elem_bytes, int32_t* d_removals,
@@ -111,7 +114,9 @@ rz_status rz_remove_premarked(rz_ctx* ctx, void* d_data, int64_t n, uint32_t ele
  * combined list, usually < n) are removed as by rz_remove on n + g items.  The
  * new length is n + g - k.  When g >= k and every removal is below n, the red
  * zone lies inside the appended items, so every removal is a plain move of an
- * added item into its hole. */
+ * added item into its hole.  Added items that fall into the red zone are read
+ * from d_add where the launch form allows it and then never written to the
+ * list's end, which is scratch like every red zone. */
 rz_status rz_add_remove(rz_ctx* ctx, void* d_data, int64_t n, int64_t capacity, uint32_t elem_bytes,
                         const void* d_add, int64_t g, int32_t* d_removals, int64_t k, uint32_t flags, void* stream);
 /* In-place gather by a preserve list (paper p.14, eq. 3): A'[i] = A[P[i]] for

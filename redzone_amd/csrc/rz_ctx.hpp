@@ -150,9 +150,15 @@ inline int log2_floor(int64_t v) {
 rz_tile_config default_config(uint32_t esz, int64_t n, int64_t k);
 
 // launchers (one per translation unit)
-// ext_bits: a caller-owned tail bitmap (with kFlagPremarked: already marked)
+// ext_bits: a caller-owned tail bitmap (with kFlagPremarked: already marked).
+// add, split: red-zone items from `split` on are read from add (only where
+// reads_added_in_place says so).
 rz_status launch_plain(rz_ctx* ctx, void* data, int64_t n, uint32_t esz, int32_t* R, int64_t k, uint32_t flags,
-                       const rz_tile_config& cfg, hipStream_t s, uint32_t* ext_bits = nullptr);
+                       const rz_tile_config& cfg, hipStream_t s, uint32_t* ext_bits = nullptr,
+                       const void* add = nullptr, uint32_t split = 0xffffffffu);
+// whether a call of this shape can read red-zone items from outside the list
+// (the fused and the direct forms, which never write the red zone)
+bool reads_added_in_place(const rz_ctx* ctx, const rz_tile_config& cfg, int64_t k, uint32_t flags);
 rz_status launch_mark_removals(rz_ctx* ctx, const int32_t* R, int64_t n, int64_t k, uint32_t* bits, hipStream_t s);
 // rz_remove_sized: the one-launch fused shape for up to k_cap removals (false
 // when none fits), and its launch with n and k read from d_n, d_k on the device

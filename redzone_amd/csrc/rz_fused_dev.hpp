@@ -31,6 +31,17 @@
 
 namespace rz {
 
+// The red zone as a removal reads it: items [0, split) are the list's own tail,
+// the others are still where the caller appends from (rz_add_remove), so an
+// added item goes from there to its hole and is never written to the list's end.
+template <typename T>
+struct RedZone {
+  const T* tail;    // A + sZ
+  const T* add;     // item p >= split is add[p - split]
+  uint32_t split;   // k or more: the whole red zone is in the list
+  __device__ __forceinline__ T operator[](uint32_t p) const { return p < split ? tail[p] : add[p - split]; }
+};
+
 constexpr uint64_t kStAgg = 1ull << 62, kStIncl = 2ull << 62, kStCount = (1ull << 62) - 1;
 
 // COH: read the tail bitmap with coherent loads (it was marked in the same
@@ -44,7 +55,8 @@ __device__ __forceinline__ void move_pair_core(T* __restrict__ A, const int32_t*
                                                uint64_t* __restrict__ st, uint64_t* __restrict__ slots,
                                                uint32_t slot_cap, uint32_t* __restrict__ ctrl, int stats, int early,
                                                uint32_t slice, uint32_t backoff, uint32_t tag,
-                                               uint64_t* __restrict__ my_stamps) {
+                                               uint64_t* __restrict__ my_stamps, const T* add = nullptr,
+                                               uint32_t split = 0xffffffffu) {
   constexpr int NW = WG / kWave;
   constexpr int E = MoveShared<WG, IPT>::E;
   constexpr int PER = (E + kWave - 1) / kWave;
@@ -54,7 +66,7 @@ __device__ __forceinline__ void move_pair_core(T* __restrict__ A, const int32_t*
   uint32_t* s_off = sh.off;
   const int tid = threadIdx.x, lane = lane_id(), wave = tid / kWave;
   const uint32_t a = slice * L, b = min(a + L, k);
-  T* __restrict__ Z = A + sZ;
+  const RedZone<T> Z{A + sZ, add, split};
 
   // one step's loads: R and the red zone, and the bitmap words (coherent
   // loads are made after the step's other loads, below)

@@ -190,15 +190,33 @@ rz_status rz_add_remove(rz_ctx* ctx, void* d_data, int64_t n, int64_t capacity, 
   if (m >= (1ll << 31) || k < 0 || k > m) return RZ_EINVAL;
   if (g > 0) {
     const char* add = (const char*)d_add;
-    char* dst = (char*)d_data + (size_t)n * elem_bytes;
-    const size_t bytes = (size_t)g * elem_bytes;
+    char* list = (char*)d_data;
+    char* dst = list + (size_t)n * elem_bytes;
+    const size_t bytes = (size_t)g * elem_bytes, head = (size_t)(m - k) * elem_bytes;
     if (add < dst + bytes && dst < add + bytes) return RZ_EINVAL;  // the added items may not overlap their slot
-    int prev = -1;
-    (void)hipGetDevice(&prev);
-    if (prev != ctx->device) (void)hipSetDevice(ctx->device);
-    const hipError_t e = hipMemcpyAsync(dst, add, bytes, hipMemcpyDeviceToDevice, (hipStream_t)stream);
-    if (prev >= 0 && prev != ctx->device) (void)hipSetDevice(prev);
-    if (e != hipSuccess) return RZ_EHIP;
+    std::lock_guard<std::mutex> lock(ctx->mu);
+    DeviceGuard guard(ctx->device);
+    hipStream_t s = (hipStream_t)stream;
+    // The added items that fall into the red zone go from d_add straight to
+    // their holes: the red zone is scratch afterwards, so writing them there
+    // first is a copy (and a launch) for nothing.  Not if a hole could be
+    // written over an added item not yet read, or if the items are not
+    // aligned as the kernels load them.
+    const uintptr_t align = elem_bytes > 8 ? 16 : elem_bytes;
+    const rz_tile_config cfg = k > 0 && k < m ? ctx->table[esz_index(elem_bytes)][log2_floor(k)] : rz_tile_config{};
+    const bool direct = k > 0 && k < m && d_removals && (uintptr_t)d_data % align == 0 &&
+                        (uintptr_t)d_removals % 4 == 0 && (uintptr_t)d_add % align == 0 &&
+                        !(add < list + head && list < add + bytes) && reads_added_in_place(ctx, cfg, k, flags);
+    const int64_t copied = !direct ? g : g > k ? g - k : 0;  // added items that stay where they are appended
+    if (copied > 0)
+      RZ_HIP(hipMemcpyAsync(dst, add, (size_t)copied * elem_bytes, hipMemcpyDeviceToDevice, s));
+    if (direct) {
+      rz_status st;
+      if ((flags & RZ_VALIDATE) && (st = launch_validate(ctx, d_removals, m, k, flags, s)) != RZ_OK) return st;
+      st = launch_plain(ctx, d_data, m, elem_bytes, d_removals, k, flags, cfg, s, nullptr,
+                        add + (size_t)copied * elem_bytes, (uint32_t)(g < k ? k - g : 0));
+      return st != RZ_OK ? st : finish_call(ctx, flags, s);
+    }
   }
   return rz_remove(ctx, d_data, m, elem_bytes, d_removals, k, flags, stream);
 }

@@ -27,12 +27,16 @@
 // structure, redzone.hxx:626-941); (2) the persistent work-queue kernel of
 // rz_batch.hip with a single list; (3) one ordered launch, roles by workgroup
 // id; (4) mark, then one kernel that moves and pairs orphans through a
-// decoupled look-back and per-rank exchange words (rz_move_pair).
+// decoupled look-back and per-rank exchange words (rz_move_pair); (6) the same
+// in one launch; (7) one launch of independent workgroups for small k
+// (rz_direct).
 //
 // Contract violations (duplicates, out-of-range indices) never cause an
 // out-of-bounds access: marks are taken only for indices inside the tail,
 // moves only into holes below n-k, and pairing stops at the smaller orphan
 // total (a mismatch sets an error bit in the control block).
+#include <type_traits>
+
 #include "../../include/redzone_device.h"
 #include "rz_fused_dev.hpp"
 #include "rz_redzone_dev.hpp"
@@ -108,7 +112,8 @@ __device__ __forceinline__ void move_pair_body(T* __restrict__ A, const int32_t*
                                                uint64_t* __restrict__ mstatus, uint64_t* __restrict__ slots,
                                                uint32_t slot_cap, uint32_t* __restrict__ ctrl, int stats,
                                                int early, uint32_t slice, uint32_t backoff,
-                                               uint32_t* __restrict__ err_out, uint64_t* __restrict__ stamps) {
+                                               uint32_t* __restrict__ err_out, uint64_t* __restrict__ stamps,
+                                               const T* __restrict__ add = nullptr, uint32_t split = 0xffffffffu) {
   const int tid = threadIdx.x;
   // RZ_PROFILE: thread 0 stamps the wall clock at each stage boundary
   uint64_t* const my_stamps = stamps ? stamps + (size_t)blockIdx.x * kStampsPerGroup : nullptr;
@@ -120,7 +125,7 @@ __device__ __forceinline__ void move_pair_body(T* __restrict__ A, const int32_t*
     for (uint32_t w = slice * WG + tid; w < (uint32_t)kMaxSlices; w += ns * WG) other[w] = 0ull;
   }
   move_pair_core<T, WG, IPT, COH, COH>(A, R, k, sZ, L, ns, bits, st, slots, slot_cap, ctrl, stats, early, slice,
-                                       backoff, epoch, my_stamps);
+                                       backoff, epoch, my_stamps, add, split);
   // the last workgroup to leave (all of them have read the epoch by then)
   // starts the next call's epoch.  With err_out, it also hands the call's
   // error bits to the caller's word: every bit a workgroup sets is set by its
@@ -145,9 +150,10 @@ __global__ __launch_bounds__(WG) void rz_move_pair(T* __restrict__ A, const int3
                                                     uint32_t* __restrict__ bits, uint64_t* __restrict__ mstatus,
                                                     uint64_t* __restrict__ slots, uint32_t slot_cap,
                                                     uint32_t* __restrict__ ctrl, int stats, int early,
-                                                    uint32_t* __restrict__ err_out, uint64_t* __restrict__ stamps) {
+                                                    uint32_t* __restrict__ err_out, uint64_t* __restrict__ stamps,
+                                                    const T* __restrict__ add, uint32_t split) {
   move_pair_body<T, WG, IPT, false>(A, R, k, sZ, L, ns, bits, mstatus, slots, slot_cap, ctrl, stats, early,
-                                    blockIdx.x, 0u, err_out, stamps);
+                                    blockIdx.x, 0u, err_out, stamps, add, split);
 }
 
 // Variant 6: the mark step in the same launch.  Workgroups [0, nm) each mark
@@ -208,13 +214,14 @@ __global__ __launch_bounds__(WG) void rz_mark_move_pair(T* __restrict__ A, const
                                                          uint32_t* __restrict__ ctrl, int stats, uint32_t nm,
                                                          uint32_t tile, uint32_t backoff, int sorted, int early,
                                                          uint32_t* __restrict__ err_out,
-                                                         uint64_t* __restrict__ stamps) {
+                                                         uint64_t* __restrict__ stamps, const T* __restrict__ add,
+                                                         uint32_t split) {
   if (blockIdx.x < nm) {
     mark_group_body<WG>(R, k, sZ, bits, ctrl, stats, nm, tile, sorted, stamps);
     return;
   }
   move_pair_body<T, WG, IPT, true>(A, R, k, sZ, L, ns, bits, mstatus, slots, slot_cap, ctrl, stats, early,
-                                   blockIdx.x - nm, backoff, err_out, stamps);
+                                   blockIdx.x - nm, backoff, err_out, stamps, add, split);
 }
 
 // The one-launch form with n and k read from device memory (rz_remove_sized;
@@ -257,6 +264,147 @@ __global__ __launch_bounds__(WG) void rz_mark_move_pair_sized(T* __restrict__ A,
   if (slice >= ns) return;
   move_pair_body<T, WG, IPT, true>(A, R, uk, sZ, L, ns, bits, mstatus, slots, uk / 2 + 1, ctrl, stats, early, slice,
                                    backoff, nullptr, nullptr);
+}
+
+// ---------------------------------------------------------------------------
+// direct form (variant 7): one launch whose workgroups never wait for each
+// other.  Every workgroup reads all of R and builds two k-bit maps in LDS:
+// pair i's source is dead (an LDS atomicOr per red-zone removal), pair i's
+// destination is a hole (a ballot).  These give every pair's class and, with
+// a prefix sum over the words, every orphan's global rank, so the workgroup
+// moves its own slice of pairs and, for the t-th dest orphan, selects the
+// t-th source orphan's bit itself.  No scratch, no look-back, no exchange and
+// no epoch.  It reads R once per workgroup: (k / slice) * 4k bytes from the
+// caches, which is what bounds its k.
+// Below that it is bound by latency: R, the maps, one prefix sum, the moves,
+// where the one-launch fused form pays eight device-scope round trips (marks,
+// two done counters, ready word, bitmap, look-back, exchange, exit count).
+// Back-to-back calls from Python on MI355X, this form (512 x 1) against the
+// tuned fused shape, 4- and 16-byte items alike, us: k = 2^14 at k/n = 1% 7.2
+// (the caller's own rate) against 8.5, at 50% 7.3 against 12.5; k = 2^14.5
+// 8.2 against 8.5 and 7.5 against 13.1; k = 2^15.5 (1024 x 1) 11.2 against
+// 8.8 and 10.1 against 13.5.  So the tuned table has it up to 2^15 removals.
+// ---------------------------------------------------------------------------
+constexpr uint32_t kDirectMaxK = 1u << 17;  // 24 bytes of LDS per 64 removals: 48 KiB
+
+// position of the r-th set bit of m (r below its count)
+__device__ __forceinline__ uint32_t select_bit(uint64_t m, uint32_t r) {
+  uint32_t pos = 0;
+#pragma unroll
+  for (int sh = 32; sh >= 1; sh >>= 1) {
+    const uint32_t c = (uint32_t)__popcll(m & ((1ull << sh) - 1));
+    if (r >= c) {
+      r -= c;
+      pos += sh;
+      m >>= sh;
+    }
+  }
+  return pos;
+}
+
+template <typename T, int WG, int IPT>
+__global__ __launch_bounds__(WG) void rz_direct(T* __restrict__ A, const int32_t* __restrict__ R, uint32_t k,
+                                                 uint32_t sZ, const T* __restrict__ add, uint32_t split,
+                                                 uint32_t* __restrict__ ctrl, int stats) {
+  extern __shared__ uint64_t s_direct[];
+  __shared__ uint64_t s_tmp[WG / kWave + 1];
+  const uint32_t W = (k + 63u) >> 6;
+  uint64_t* const hole = s_direct;       // bit i: R[i] is a hole in the head
+  uint64_t* const dead = hole + W;       // bit i: red-zone item i was removed
+  uint64_t* const pre = dead + W;        // orphans before a word: dest | source << 32
+  const uint32_t tid = threadIdx.x;
+  const RedZone<T> Z{A + sZ, add, split};
+  const uint32_t base = blockIdx.x * (WG * IPT);
+  // this slice's pairs, loaded ahead of the maps
+  uint32_t d[IPT];
+  T z[IPT];
+#pragma unroll
+  for (int j = 0; j < IPT; ++j) {
+    const uint32_t p = base + j * WG + tid;
+    d[j] = sZ;  // no destination
+    z[j] = T();
+    if (p < k) {
+      d[j] = (uint32_t)R[p];
+      z[j] = Z[p];
+    }
+  }
+  for (uint32_t w = tid; w < W; w += WG) dead[w] = 0ull;
+  __syncthreads();
+  // The maps, U words of 64 removals per wave and round: lane u collects word
+  // u's ballot, so a round stores its hole words at once.  A wave64
+  // instruction takes four cycles of its SIMD and every workgroup does this
+  // for all of R, so the instructions per word bound the form from 2^14
+  // removals up (k = 2^16 at k/n = 1%: 512 threads 13.6 us a call, 18.1 with a
+  // bounds check and a one-lane store per word).
+  constexpr uint32_t U = 16;
+  auto round = [&](uint32_t c0, auto whole) {
+    uint32_t r[U];
+#pragma unroll
+    for (uint32_t u = 0; u < U; ++u) {
+      const uint32_t i = c0 + u * WG + tid;
+      r[u] = decltype(whole)::value || i < k ? (uint32_t)R[i] : 0xffffffffu;  // in neither zone
+    }
+    uint64_t words = 0;
+#pragma unroll
+    for (uint32_t u = 0; u < U; ++u) {
+      const uint64_t m = ballot(r[u] < sZ);
+      if ((uint32_t)lane_id() == u) words = m;
+      const uint32_t q = r[u] - sZ;  // wraps to >= 2^31 > k below the red zone
+      if (q < k) atomicOr((uint32_t*)dead + (q >> 5), 1u << (q & 31));
+    }
+    const uint32_t w = (c0 + (tid & ~63u)) / 64u + (uint32_t)lane_id() * (WG / 64);
+    if ((uint32_t)lane_id() < U && w < W) hole[w] = words;
+  };
+  uint32_t c0 = 0;
+  for (; c0 + WG * U <= k; c0 += WG * U) round(c0, std::true_type{});
+  if (c0 < k) round(c0, std::false_type{});
+  __syncthreads();
+  auto sources = [&](uint32_t w) {  // source orphans of word w (bits past k are none)
+    const uint64_t valid = w == W - 1 && (k & 63u) ? (1ull << (k & 63u)) - 1 : ~0ull;
+    return ~(hole[w] | dead[w]) & valid;
+  };
+  auto dests = [&](uint32_t w) { return hole[w] & dead[w]; };
+  const uint32_t per = (W + WG - 1) / WG, w0 = tid * per, w1 = min(w0 + per, W);
+  uint64_t sum = 0, tails = 0;
+  for (uint32_t w = w0; w < w1; ++w) {
+    sum += (uint64_t)__popcll(dests(w)) | (uint64_t)__popcll(sources(w)) << 32;
+    tails += (uint64_t)__popcll(dead[w]);
+  }
+  uint64_t total;
+  uint64_t ex = block_excl_scan<WG>(sum, s_tmp, &total);
+  for (uint32_t w = w0; w < w1; ++w) {
+    pre[w] = ex;
+    ex += (uint64_t)__popcll(dests(w)) | (uint64_t)__popcll(sources(w)) << 32;
+  }
+  const uint32_t tot_d = (uint32_t)total, tot_s = (uint32_t)(total >> 32);
+  if (blockIdx.x == 0) {
+    if (tid == 0 && tot_d != tot_s) or_relaxed(&ctrl[kCtrlError], kErrOrphanMismatch);
+    if (stats) {
+      tails = wave_sum(tails);
+      if (lane_id() == 0 && tails) add_relaxed((uint64_t*)&ctrl[kCtrlStatTail], tails);
+      if (tid == 0) st_relaxed((uint64_t*)&ctrl[kCtrlStatOrphans], (uint64_t)min(tot_d, tot_s));
+    }
+  }
+  __syncthreads();
+  // the dest orphans' sources first: a load after the moves would wait for them to drain
+#pragma unroll
+  for (int j = 0; j < IPT; ++j) {
+    const uint32_t p = base + j * WG + tid, w = p >> 6;
+    if (p >= k || d[j] >= sZ || !((dead[w] >> (p & 63u)) & 1ull)) {
+      if (p >= k) d[j] = sZ;
+      continue;
+    }
+    const uint32_t t = (uint32_t)pre[w] + (uint32_t)__popcll(dests(w) & ((1ull << (p & 63u)) - 1));
+    if (t >= tot_s) {  // only with an invalid removal list
+      d[j] = sZ;
+      continue;
+    }
+    const uint32_t ws = (uint32_t)upper_row((int)W, t, [&](int q) { return (uint32_t)(pre[q] >> 32); });
+    z[j] = Z[ws * 64u + select_bit(sources(ws), t - (uint32_t)(pre[ws] >> 32))];
+  }
+#pragma unroll
+  for (int j = 0; j < IPT; ++j)
+    if (d[j] < sZ) A[d[j]] = z[j];
 }
 
 // ---------------------------------------------------------------------------
@@ -408,12 +556,12 @@ template <typename T>
 static bool dispatch_move_pair(int wg, int ipt, hipStream_t s, T* A, const int32_t* R, uint32_t k, uint32_t sZ,
                                uint32_t L, uint32_t ns, uint32_t* bits, uint64_t* mstatus, uint64_t* slots,
                                uint32_t slot_cap, uint32_t* ctrl, int stats, int early, uint32_t* err_out = nullptr,
-                               uint64_t* stamps = nullptr) {
+                               uint64_t* stamps = nullptr, const T* add = nullptr, uint32_t split = 0xffffffffu) {
   const size_t lds = (size_t)L * 4;
 #define RZ_MP_CASE(W, I)                                                                                     \
   if (wg == W && ipt == I) {                                                                                 \
     hipLaunchKernelGGL((rz_move_pair<T, W, I>), dim3(ns), dim3(W), lds, s, A, R, k, sZ, L, ns, bits, mstatus, \
-                       slots, slot_cap, ctrl, stats, early, err_out, stamps);                                \
+                       slots, slot_cap, ctrl, stats, early, err_out, stamps, add, split);                    \
     return true;                                                                                             \
   }
   RZ_MP_CASE(256, 2) RZ_MP_CASE(256, 4) RZ_MP_CASE(256, 8) RZ_MP_CASE(256, 16)
@@ -421,6 +569,27 @@ static bool dispatch_move_pair(int wg, int ipt, hipStream_t s, T* A, const int32
 #undef RZ_MP_CASE
   return false;
 }
+
+template <typename T>
+static bool dispatch_direct(int wg, int ipt, hipStream_t s, T* A, const int32_t* R, uint32_t k, uint32_t sZ,
+                            const T* add, uint32_t split, uint32_t* ctrl, int stats) {
+  const size_t lds = (size_t)((k + 63) / 64) * 24;
+  const uint32_t grid = (k + wg * ipt - 1) / (wg * ipt);
+#define RZ_DIRECT_CASE(W, I)                                                                                   \
+  if (wg == W && ipt == I) {                                                                                   \
+    hipLaunchKernelGGL((rz_direct<T, W, I>), dim3(grid), dim3(W), lds, s, A, R, k, sZ, add, split, ctrl, stats); \
+    return true;                                                                                               \
+  }
+  RZ_DIRECT_CASE(256, 1) RZ_DIRECT_CASE(256, 2) RZ_DIRECT_CASE(256, 4)
+  RZ_DIRECT_CASE(512, 1) RZ_DIRECT_CASE(512, 2) RZ_DIRECT_CASE(512, 4)
+  RZ_DIRECT_CASE(1024, 1) RZ_DIRECT_CASE(1024, 2)
+#undef RZ_DIRECT_CASE
+  return false;
+}
+
+// The one-launch fused shape of lists the direct form would run (tuned for k
+// up to 2^14; it covers any k a fused form can).
+constexpr rz_tile_config kSmallFused = {256, 4, 512, 6, 12, 1};
 
 static int clamp_tile_log(int tile_log) {
   return tile_log == 0 ? kFusedMarkTileLog : (tile_log < 8 ? 8 : (tile_log > 16 ? 16 : tile_log));
@@ -436,7 +605,8 @@ template <typename T>
 static bool dispatch_mark_move_pair(int wg, int ipt, hipStream_t s, T* A, const int32_t* R, uint32_t k, uint32_t sZ,
                                     uint32_t L, uint32_t ns, uint32_t* bits, uint64_t* mstatus, uint64_t* slots,
                                     uint32_t slot_cap, uint32_t* ctrl, int stats, int tile_log, int sorted,
-                                    int early, uint32_t* err_out = nullptr, uint64_t* stamps = nullptr) {
+                                    int early, uint32_t* err_out = nullptr, uint64_t* stamps = nullptr,
+                                    const T* add = nullptr, uint32_t split = 0xffffffffu) {
   const uint32_t bo = kMarkWaitBackoff;
   const size_t lds = (size_t)L * 4;
   tile_log = clamp_tile_log(tile_log);
@@ -445,7 +615,8 @@ static bool dispatch_mark_move_pair(int wg, int ipt, hipStream_t s, T* A, const 
 #define RZ_MMP_CASE(W, I)                                                                                      \
   if (wg == W && ipt == I) {                                                                                   \
     hipLaunchKernelGGL((rz_mark_move_pair<T, W, I>), dim3(nm + ns), dim3(W), lds, s, A, R, k, sZ, L, ns, bits, \
-                       mstatus, slots, slot_cap, ctrl, stats, nm, tile, bo, sorted, early, err_out, stamps);   \
+                       mstatus, slots, slot_cap, ctrl, stats, nm, tile, bo, sorted, early, err_out, stamps,    \
+                       add, split);                                                                            \
     return true;                                                                                               \
   }
   RZ_MMP_CASE(256, 2) RZ_MMP_CASE(256, 4) RZ_MMP_CASE(256, 8) RZ_MMP_CASE(256, 16)
@@ -500,12 +671,25 @@ static rz_status dispatch_coop(int wg, int ipt, rz_ctx* ctx, T* A, int32_t* R, i
 
 template <typename T>
 static rz_status plain_impl(rz_ctx* ctx, T* A, int64_t n, int32_t* R, int64_t k, uint32_t flags,
-                            const rz_tile_config& cfg, bool coop, hipStream_t s, uint32_t* ext_bits) {
+                            const rz_tile_config& cfg, bool coop, hipStream_t s, uint32_t* ext_bits, const T* add,
+                            uint32_t split) {
   const uint32_t sZ = (uint32_t)(n - k);
   uint32_t L, ns;
   slice_shape(k, cfg, kMaxSlices, &L, &ns);
   rz_status st;
   ctx->stamp_groups = 0;  // stage stamps only from a fused call with RZ_PROFILE
+  if (cfg.variant == 7 && !coop) {
+    uint32_t* ctrl = (uint32_t*)ctx->ctrl.ptr;
+    const int stats = (flags & RZ_STATS) ? 1 : 0;
+    if (stats && (st = fill_u32(ctrl + kCtrlStatTail, 0u, 2, s)) != RZ_OK) return st;
+    if ((st = prof_mark(ctx, flags, 0, s)) != RZ_OK) return st;
+    if ((st = prof_mark(ctx, flags, 1, s)) != RZ_OK) return st;
+    if (!dispatch_direct<T>(cfg.wg_size, cfg.items, s, A, R, (uint32_t)k, sZ, add, split, ctrl, stats))
+      return RZ_EINVAL;
+    RZ_HIP(hipGetLastError());
+    if ((st = prof_mark(ctx, flags, 2, s)) != RZ_OK) return st;
+    return prof_mark(ctx, flags, 3, s);
+  }
   if (!ext_bits && (st = ensure(ctx, ctx->tail_bits, (size_t)((k + 63) / 64) * 8, s)) != RZ_OK) return st;
   if ((st = ensure(ctx, ctx->counts, (size_t)ns * 8, s)) != RZ_OK) return st;
   int32_t* Rd = R;
@@ -578,7 +762,7 @@ static rz_status plain_impl(rz_ctx* ctx, T* A, int64_t n, int32_t* R, int64_t k,
     if (!dispatch_mark_move_pair<T>(cfg.wg_size, cfg.items, s, A, R, (uint32_t)k, sZ, L, ns, bits,
                                     (uint64_t*)ctx->mstatus.ptr, (uint64_t*)ctx->slots.ptr, (uint32_t)(k / 2 + 1),
                                     ctrl, stats, cfg.slice_steps, (flags & RZ_SORTED) ? 1 : 0,
-                                    (flags & RZ_ANY_PAIRING) ? 1 : 0, nullptr, stamps))
+                                    (flags & RZ_ANY_PAIRING) ? 1 : 0, nullptr, stamps, add, split))
       return RZ_EINVAL;
     RZ_HIP(hipGetLastError());
     if ((st = prof_mark(ctx, flags, 2, s)) != RZ_OK) return st;
@@ -587,7 +771,7 @@ static rz_status plain_impl(rz_ctx* ctx, T* A, int64_t n, int32_t* R, int64_t k,
   if (fused) {
     if (!dispatch_move_pair<T>(cfg.wg_size, cfg.items, s, A, R, (uint32_t)k, sZ, L, ns, bits,
                                (uint64_t*)ctx->mstatus.ptr, (uint64_t*)ctx->slots.ptr, (uint32_t)(k / 2 + 1), ctrl,
-                               stats, (flags & RZ_ANY_PAIRING) ? 1 : 0, nullptr, stamps))
+                               stats, (flags & RZ_ANY_PAIRING) ? 1 : 0, nullptr, stamps, add, split))
       return RZ_EINVAL;
     RZ_HIP(hipGetLastError());
     if ((st = prof_mark(ctx, flags, 2, s)) != RZ_OK) return st;
@@ -680,24 +864,54 @@ static bool plain_shape_ok(const rz_ctx* ctx, const rz_tile_config& cfg, uint32_
       return wg_ok && (cfg.items == 2 || cfg.items == 4 || cfg.items == 8 || cfg.items == 16);
     case 2: return wg_ok && (cfg.items == 4 || cfg.items == 8);
     case 5: return dense_shape_ok(ctx, cfg, esz, n, k, flags);
+    case 7:
+      return k <= (int64_t)kDirectMaxK &&
+             (cfg.items == 1 || cfg.items == 2 ? wg_ok || cfg.wg_size == 1024 : wg_ok && cfg.items == 4);
     default: return false;
   }
 }
 
-rz_status launch_plain(rz_ctx* ctx, void* data, int64_t n, uint32_t esz, int32_t* R, int64_t k, uint32_t flags,
-                       const rz_tile_config& cfg_in, hipStream_t s, uint32_t* ext_bits) {
-  rz_tile_config cfg = cfg_in;
+// The launch shape a call runs for a given one: the forms that take no marks
+// from outside or have no cooperative launch run another.
+static rz_tile_config effective_shape(const rz_tile_config& in, uint32_t flags) {
+  rz_tile_config cfg = in;
   const bool premarked = (flags & kFlagPremarked) != 0;
+  // the direct form marks in LDS and has neither a premarked nor a cooperative shape
+  if (cfg.variant == 7 && (premarked || (flags & RZ_COOPERATIVE))) cfg = kSmallFused;
   // the single-launch forms include their own mark step: with the marks set
   // by the caller, run their shape as the two-kernel fused form
   if (premarked && ((cfg.variant >= 1 && cfg.variant <= 3) || cfg.variant == 6)) cfg.variant = 4;
+  return cfg;
+}
+
+bool reads_added_in_place(const rz_ctx* ctx, const rz_tile_config& in, int64_t k, uint32_t flags) {
+  const rz_tile_config cfg = effective_shape(in, flags);
+  if (flags & RZ_COOPERATIVE) return false;
+  if (cfg.variant == 7) return true;
+  if ((cfg.variant != 4 && cfg.variant != 6) || cfg.wg_size < 1 || cfg.items < 1) return false;
+  uint32_t L, ns;
+  slice_shape(k, cfg, kMaxSlices, &L, &ns);
+  return fused_fits(ctx, cfg, L);
+}
+
+rz_status launch_plain(rz_ctx* ctx, void* data, int64_t n, uint32_t esz, int32_t* R, int64_t k, uint32_t flags,
+                       const rz_tile_config& cfg_in, hipStream_t s, uint32_t* ext_bits, const void* add,
+                       uint32_t split) {
+  const rz_tile_config cfg = effective_shape(cfg_in, flags);
+  const bool premarked = (flags & kFlagPremarked) != 0;
+  if (cfg_in.variant == 7 && !plain_shape_ok(ctx, cfg_in, esz, n, k, flags)) return RZ_EINVAL;
   if (!plain_shape_ok(ctx, cfg, esz, n, k, flags)) return RZ_EINVAL;
   if (cfg.variant == 2) return launch_queue_single(ctx, data, n, esz, R, k, flags, cfg, s);
   const bool coop = !premarked && (cfg.variant == 1 || (flags & RZ_COOPERATIVE));
   switch (esz) {
-    case 4: return plain_impl<uint32_t>(ctx, (uint32_t*)data, n, R, k, flags, cfg, coop, s, ext_bits);
-    case 8: return plain_impl<uint64_t>(ctx, (uint64_t*)data, n, R, k, flags, cfg, coop, s, ext_bits);
-    case 16: return plain_impl<uint4>(ctx, (uint4*)data, n, R, k, flags, cfg, coop, s, ext_bits);
+    case 4:
+      return plain_impl<uint32_t>(ctx, (uint32_t*)data, n, R, k, flags, cfg, coop, s, ext_bits, (const uint32_t*)add,
+                                  split);
+    case 8:
+      return plain_impl<uint64_t>(ctx, (uint64_t*)data, n, R, k, flags, cfg, coop, s, ext_bits, (const uint64_t*)add,
+                                  split);
+    case 16:
+      return plain_impl<uint4>(ctx, (uint4*)data, n, R, k, flags, cfg, coop, s, ext_bits, (const uint4*)add, split);
     default: return RZ_EINVAL;
   }
 }
@@ -710,6 +924,7 @@ rz_status launch_plain(rz_ctx* ctx, void* data, int64_t n, uint32_t esz, int32_t
 // up to kMaxSlices slices.  false when no fused shape fits k_cap.
 bool sized_shape(const rz_ctx* ctx, uint32_t esz, int64_t k_cap, rz_tile_config* out) {
   rz_tile_config c = ctx->table[esz_index(esz)][log2_floor(k_cap)];
+  if (c.variant == 7) c = kSmallFused;  // the direct form takes its sizes from the host
   uint32_t L, ns;
   const bool tuned = (c.variant == 4 || c.variant == 6) && (c.wg_size == 256 || c.wg_size == 512) &&
                      (c.items == 2 || c.items == 4 || c.items == 8 || c.items == 16);

@@ -95,6 +95,7 @@ static const rz_tile_config kCandidates[] = {
     {512, 4, 512, 6, 10, 1},  {512, 4, 512, 6, 12, 1},  {256, 4, 1024, 6, 11, 1},
     {1024, 8, 1024, 5, 11, 2}, {1024, 8, 1024, 5, 12, 2}, {1024, 4, 1024, 5, 11, 2}, {512, 8, 2048, 5, 11, 2},  // dense
     {1024, 8, 1024, 5, 11, 0},
+    {512, 1, 0, 7, 0, 1},     {1024, 1, 0, 7, 0, 1},                                                        // direct
 };
 
 static const rz_tile_config kBatchCandidates[] = {

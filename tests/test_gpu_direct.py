@@ -1,0 +1,120 @@
+"""The direct form (variant 7: independent workgroups, maps of all pairs in
+LDS) and the added items that rz_add_remove reads in place, against the CPU
+oracle: bit-exact survivors at the edges of words, steps, slices and of the
+form's range."""
+import numpy as np
+import pytest
+import torch
+
+import redzone_amd as rz
+from redzone_amd import workloads as W
+from tests.parity import announce, expected_canonical, first_mismatch, gpu_remove_parity
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [(256, 1), (256, 2), (256, 4), (512, 1), (512, 2), (512, 4), (1024, 1), (1024, 2)]
+MAX_K = 1 << 17
+
+
+@pytest.mark.parametrize("esz", [4, 8, 16])
+@pytest.mark.parametrize("k", [1, 63, 64, 65, 255, 256, 1023, 1025, 4096, 4097, 16384 + 1])
+def test_direct_edges(ctx, oracle, esz, k):
+    for pattern, n in (("uniform", 40 * k + 7), ("uniform", 2 * k + 1), ("tail_heavy", 3 * k + 5),
+                       ("clustered", k + k // 3 + 2)):
+        A = W.payload(esz, n, seed=k)
+        R = W.removals(pattern, n, k, seed=k + 1)
+        want = expected_canonical(oracle, A.numpy(), R.numpy())
+        for wg, it in SHAPES:
+            announce("direct", esz, k, pattern, wg, it)
+            gpu_remove_parity(ctx, oracle, A, R, config=rz.TileConfig(wg, it, 0, 7, 0, 1), want=want)
+
+
+@pytest.mark.parametrize("k", [MAX_K - 1, MAX_K, MAX_K + 1])
+def test_direct_range_end(ctx, oracle, k):
+    """The largest k of the form, and one above it (refused)."""
+    n = 2 * k + 11
+    A = W.payload(4, n, seed=5)
+    R = W.uniform_removals(n, k, seed=6)
+    for wg, it in ((256, 4), (1024, 1)):
+        announce("direct end", k, wg, it)
+        if k > MAX_K:
+            with pytest.raises(rz.RedzoneError):
+                ctx.remove(A.cuda(), R.cuda(), config=rz.TileConfig(wg, it, 0, 7, 0, 1))
+        else:
+            gpu_remove_parity(ctx, oracle, A, R, config=rz.TileConfig(wg, it, 0, 7, 0, 1))
+
+
+def test_direct_flags(ctx, oracle):
+    n, k = 50000, 20001
+    A, R = W.payload(8, n, seed=7), torch.sort(W.uniform_removals(n, k, seed=8)).values.contiguous()
+    cfg = rz.TileConfig(512, 2, 0, 7, 0, 1)
+    want = expected_canonical(oracle, A.numpy(), R.numpy())
+    sz = n - k
+    dead = np.zeros(k, bool)
+    dead[R.numpy()[R.numpy() >= sz] - sz] = True
+    for flags in (0, rz.RZ_PRESERVE_REMOVALS, rz.RZ_SORTED, rz.RZ_VALIDATE | rz.RZ_SORTED, rz.RZ_ANY_PAIRING,
+                  rz.RZ_STATS, rz.RZ_PROFILE, rz.RZ_COOPERATIVE):
+        announce("direct flags", flags)
+        _, dR = gpu_remove_parity(ctx, oracle, A, R, config=cfg, flags=flags, want=want)
+        if flags & rz.RZ_PRESERVE_REMOVALS:
+            assert torch.equal(dR.cpu(), R)
+        if flags & rz.RZ_STATS:
+            st = ctx.last_stats()
+            assert st.tail_removals == int(dead.sum())
+            assert st.orphan_pairs == int((dead & (R.numpy() < sz)).sum())
+    dup = R.clone()
+    dup[0] = dup[k - 1]  # the last tail item twice: one source more than holes
+    dA, dR = A.cuda(), dup.cuda()
+    announce("direct mismatch")
+    with pytest.raises(rz.RedzoneError):
+        ctx.remove(dA, dR, config=cfg, flags=rz.RZ_STATS)
+    gpu_remove_parity(ctx, oracle, A, R, config=cfg, want=want)
+    announce("direct premarked")
+    bits = torch.zeros((k + 31) // 32, dtype=torch.int32, device="cuda")
+    dA, dR = A.cuda(), R.cuda()
+    ctx.mark_removals(dR, n, bits)
+    ctx.remove_premarked(dA, dR, bits, config=cfg)
+    assert first_mismatch(dA.cpu().numpy()[:sz], want[:sz]) < 0 and int(bits.abs().sum()) == 0
+    for bad in (rz.TileConfig(1024, 4, 0, 7, 0, 1), rz.TileConfig(256, 8, 0, 7, 0, 1), rz.TileConfig(128, 1, 0, 7, 0, 1)):
+        with pytest.raises(rz.RedzoneError):
+            ctx.remove(dA, dR, config=bad)
+
+
+@pytest.mark.parametrize("esz", [4, 8, 16])
+@pytest.mark.parametrize("k,variant", [(300, 7), (5000, 7), (70001, 6), (70001, 4), (70001, 0)])
+def test_add_remove_sources(oracle, esz, k, variant):
+    """Added items read where the caller has them (fused and direct forms) or
+    copied first (the others; unaligned items; items inside the list)."""
+    ctx = rz.Context(0)
+    b = k.bit_length() - 1
+    ctx.set_table(esz, b, rz.TileConfig(256, 4, 512, variant, 12 if variant == 6 else 0, 1))
+    n = 3 * k + 17
+    for g in (1, k // 2, k, k + 1, 2 * k):
+        m = n + g
+        full = W.payload(esz, m, seed=g)
+        R = W.uniform_removals(m, k, seed=g + 1)
+        want = expected_canonical(oracle, full.numpy(), R.numpy())
+        announce("add sources", esz, k, variant, g)
+        cap = torch.zeros((m + 3,) + tuple(full.shape[1:]), dtype=torch.int32, device="cuda")
+        cap[:n] = full[:n].cuda()
+        guard = cap[m:].clone()
+        add = full[n:].cuda()
+        assert ctx.add_remove(cap, n, add, R.cuda()) == m - k
+        assert first_mismatch(cap[: m - k].cpu().numpy(), want[: m - k]) < 0
+        assert torch.equal(cap[m:], guard)
+        if esz > 4:  # items at an address the kernels cannot load them from
+            raw = torch.empty(add.numel() + 1, dtype=torch.int32, device="cuda")
+            off = raw[1:].view(add.shape)
+            off.copy_(add)
+            cap[:n] = full[:n].cuda()
+            assert ctx.add_remove(cap, n, off, R.cuda()) == m - k
+            assert first_mismatch(cap[: m - k].cpu().numpy(), want[: m - k]) < 0
+        if g <= n:  # the added items are a part of the list itself
+            cap[:n] = full[:n].cuda()
+            src = full.clone()
+            src[n:] = full[:g]
+            want2 = expected_canonical(oracle, src.numpy(), R.numpy())
+            assert ctx.add_remove(cap, n, cap[:g], R.cuda()) == m - k
+            assert first_mismatch(cap[: m - k].cpu().numpy(), want2[: m - k]) < 0
+    assert ctx.check_errors() == 0
+    ctx.close()

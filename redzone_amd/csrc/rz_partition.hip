@@ -371,9 +371,9 @@ constexpr int kPartWG = 256, kPartIPT = 16;
 // Bucketed marks, two kernels: the removals r in a window [base, base + m)
 // set bit r - base of an m-bit bitmap that is zero on entry (the partition's
 // n-bit bitmap: base 0, m = n; the dense form's tail bitmap: base n - k,
-// m = k).  Bins of 2^blog positions (2^15 to 2^19, so that a window has 256 to
-// 1,024 bins).
-// rz_part_append: a workgroup takes 1,024 x IPT removals, counts them per bin in
+// m = k).  Bins of 2^blog positions (2^15 to 2^20, so that a window has 256 to
+// 512 bins, fewer when it is small).
+// rz_part_append: a workgroup takes 1,024 x IPT removals at a time, counts them per bin in
 // LDS, reserves room in each bin's entry list (2^blog entries, a bin's
 // positions) with one atomic per bin, sorts them by bin in LDS and writes them
 // out bin by bin, so consecutive threads write consecutive words.
@@ -385,70 +385,89 @@ constexpr int kPartWG = 256, kPartIPT = 16;
 // No scans and no epoch launch: two launches where a count / scan / entries /
 // bits pipeline took five.
 // ---------------------------------------------------------------------------
-constexpr uint32_t kPartMinBinLog = 15, kPartMaxBinLog = 19;  // 4 to 64 KiB LDS bitmaps
-constexpr uint32_t kPartMaxBins = 1024;                       // lists of up to 2^29 items
+constexpr uint32_t kPartMinBinLog = 15, kPartMaxBinLog = 20;  // 4 to 128 KiB LDS bitmaps
+constexpr uint32_t kPartMaxBins = 1024;
+constexpr int64_t kPartMaxWindow = (int64_t)1 << 29;  // entry lists of 2 GiB
 constexpr uint32_t kAppWG = 1024;
-// removals per thread: the bigger the stage (dynamic LDS, 4 bytes a removal),
-// the longer each bin's runs of consecutive words and the fewer count atomics
-constexpr int kAppIPT = 16, kAppIPTSmall = 8;
+// Removals per thread of a tile (dynamic LDS, 4 bytes a removal).  A bigger
+// tile writes longer runs of consecutive words per bin: a run's two ends share
+// their lines with runs of other workgroups, so 32-word runs cost 45 us of the
+// 180 that 2^26 removals take, and 128-word runs 15.  A smaller one gives the
+// chip more workgroups, but each costs its own scan and reservation.  One
+// kernel at k/n = 1/4, us for 8 / 16 / 32 removals per thread: k = 600,000
+// 8.6 / 10.8 / -; 2^22 20.0 / 17.2 / -; 2^24 56.5 / 47.1 / 42.9; 2^26
+// 226 / 191 / 162 (the next tile's loads issued ahead).  With 256 bins instead of
+// 512 there the entries' reader (rz_part_bits) took 73 us instead of 93.
+constexpr int kAppIPT = 16, kAppIPTSmall = 8, kAppIPTBig = 32;
+constexpr int64_t kAppSmallK = (int64_t)1 << 21, kAppBigK = (int64_t)1 << 24;
 
+// A workgroup takes tiles blockIdx, blockIdx + grid, ...
 template <int IPT>
 __global__ __launch_bounds__(1024) void rz_part_append(const int32_t* __restrict__ R, uint32_t k, uint32_t base,
-                                                        uint32_t m, uint32_t blog, uint32_t nbins,
+                                                        uint32_t m, uint32_t blog, uint32_t nbins, uint32_t ntiles,
                                                         uint32_t* __restrict__ ent, uint32_t* __restrict__ cur,
                                                         uint64_t* __restrict__ stat) {
   constexpr uint32_t kAppS = kAppWG * IPT;
-  __shared__ uint32_t s_cnt[kPartMaxBins], s_lbase[kPartMaxBins], s_gbase[kPartMaxBins];
+  __shared__ uint32_t s_cnt[kPartMaxBins], s_lbase[kPartMaxBins];
   __shared__ uint32_t s_tmp[kAppWG / kWave + 1];
   extern __shared__ __align__(16) unsigned char dyn[];
   uint32_t* s_stage = (uint32_t*)dyn;
   const uint32_t tid = threadIdx.x;
-  const uint32_t a = blockIdx.x * kAppS, b = min(a + kAppS, k);
-  for (uint32_t w = tid; w < nbins; w += kAppWG) s_cnt[w] = 0u;
   if (stat && blockIdx.x == 0 && tid == 0) st_relaxed(stat, (uint64_t)0);
-  __syncthreads();
-  uint32_t r[IPT];
+  uint32_t next[IPT];
+  auto load = [&](uint32_t tile) {  // all loads of a tile in flight together
+    const int32_t* Rt = R + (size_t)tile * kAppS;
+    const uint32_t left = k - tile * kAppS;
 #pragma unroll
-  for (int j = 0; j < IPT; ++j) {  // all loads first (a use inside this loop would wait for each one)
-    const uint32_t i = a + j * kAppWG + tid;
-    r[j] = i < b ? (uint32_t)R[i] : 0xffffffffu;
-  }
-  // positions in the window; 0xffffffff (>= m) for none (0xffffffff - base >= 2^31 > m)
+    for (int j = 0; j < IPT; ++j) next[j] = j * kAppWG + tid < left ? (uint32_t)Rt[j * kAppWG + tid] : 0xffffffffu;
+  };
+  load(blockIdx.x);
+  for (uint32_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+    for (uint32_t w = tid; w < nbins; w += kAppWG) s_cnt[w] = 0u;
+    __syncthreads();
+    // positions in the window; 0xffffffff (>= m) for none (0xffffffff - base >= 2^31 > m)
+    uint32_t r[IPT], rank[IPT / 2];  // two ranks (below 2^15) to a register: IPT 32 leaves none to spare
 #pragma unroll
-  for (int j = 0; j < IPT; ++j) {
-    const uint32_t p = r[j] - base;
-    r[j] = p < m ? p : 0xffffffffu;
-  }
-  // a wave whose removals share one bin (a run) counts them with one atomic
+    for (int j = 0; j < IPT; ++j) {
+      const uint32_t p = next[j] - base;
+      r[j] = p < m ? p : 0xffffffffu;
+    }
+    // count and rank in one pass: the count's atomic returns the rank (a wave
+    // whose removals share one bin, a run, takes one atomic)
 #pragma unroll
-  for (int j = 0; j < IPT; ++j) lds_bin_count(s_cnt, r[j] >> blog, r[j] < m);
-  __syncthreads();
-  // exclusive prefix over the bins (one bin per thread), then room in each bin's list
-  uint32_t total;
-  const uint32_t c = tid < nbins ? s_cnt[tid] : 0u;
-  const uint32_t ex = block_excl_scan<kAppWG>(c, s_tmp, &total);
-  // the reservation's atomics stay in flight while the removals are staged:
-  // only the write-out below needs their results
-  uint32_t gb = 0u;
-  if (tid < nbins) {
-    s_lbase[tid] = ex;
-    if (c) gb = add_relaxed(&cur[tid], c);
-    s_cnt[tid] = 0u;
-  }
-  __syncthreads();
+    for (int j = 0; j < IPT; j += 2) {
+      rank[j / 2] = lds_bin_add(s_cnt, r[j] >> blog, r[j] < m);
+      rank[j / 2] |= lds_bin_add(s_cnt, r[j + 1] >> blog, r[j + 1] < m) << 16;
+    }
+    __syncthreads();
+    // exclusive prefix over the bins (one bin per thread), then room in each bin's list
+    uint32_t total;
+    const uint32_t c = tid < nbins ? s_cnt[tid] : 0u;
+    const uint32_t ex = block_excl_scan<kAppWG>(c, s_tmp, &total);
+    // the reservation's atomics stay in flight while the removals are staged:
+    // only the write-out below needs their results
+    uint32_t gb = 0u;
+    if (tid < nbins) {
+      s_lbase[tid] = ex;
+      if (c) gb = add_relaxed(&cur[tid], c);
+    }
+    __syncthreads();
+    uint32_t bl = blog;
+    asm volatile("" : "+s"(bl));  // the bins are computed again: IPT of them kept from above would not fit in registers
 #pragma unroll
-  for (int j = 0; j < IPT; ++j) {
-    const uint32_t bz = r[j] >> blog;
-    const uint32_t rank = lds_bin_add(s_cnt, bz, r[j] < m);
-    if (r[j] < m) s_stage[s_lbase[bz] + rank] = r[j];
-  }
-  if (tid < nbins) s_gbase[tid] = gb;
-  __syncthreads();
-  for (uint32_t t = tid; t < total; t += kAppWG) {
-    const uint32_t v = s_stage[t];
-    const uint32_t bz = v >> blog;
-    const uint32_t g = s_gbase[bz] + (t - s_lbase[bz]);
-    if (g < (1u << blog)) ent[((size_t)bz << blog) + g] = v;  // more only with duplicate removals
+    for (int j = 0; j < IPT; ++j)
+      if (r[j] < m) s_stage[s_lbase[r[j] >> bl] + ((rank[j / 2] >> 16 * (j & 1)) & 0xffffu)] = r[j];
+    if (tid < nbins) s_cnt[tid] = gb - ex;  // a staged entry's place in its bin's list, less its place in the stage
+    // the next tile's loads go out ahead of this tile's stores: a wait for them never waits for the stores
+    if (tile + gridDim.x < ntiles) load(tile + gridDim.x);
+    __syncthreads();
+    for (uint32_t t = tid; t < total; t += kAppWG) {
+      const uint32_t v = s_stage[t];
+      const uint32_t bz = v >> blog;
+      const uint32_t g = s_cnt[bz] + t;
+      if (g < (1u << blog)) ent[((size_t)bz << blog) + g] = v;  // more only with duplicate removals
+    }
+    __syncthreads();
   }
 }
 
@@ -513,40 +532,56 @@ __global__ __launch_bounds__(1024) void rz_part_bits(const uint32_t* __restrict_
   }
 }
 
-bool bucket_marks_fit(int64_t m) { return m > 0 && m <= ((int64_t)kPartMaxBins << kPartMaxBinLog); }
+bool bucket_marks_fit(int64_t m) { return m > 0 && m <= kPartMaxWindow; }
+
+template <int IPT>
+static rz_status append_launch(rz_ctx* ctx, const int32_t* R, int64_t k, uint32_t base, int64_t m, uint32_t blog,
+                               uint32_t nbins, uint32_t* ent, uint32_t* cur, uint64_t* stat, hipStream_t s) {
+  constexpr size_t lds = (size_t)4 * kAppWG * IPT;
+  static std::atomic<uint64_t> attr_mask{0};
+  const int dev = ctx->device;
+  if (dev < 0 || dev >= 64 || !(attr_mask.load(std::memory_order_relaxed) & (1ull << dev))) {
+    RZ_HIP(hipFuncSetAttribute((const void*)rz_part_append<IPT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    if (dev >= 0 && dev < 64) attr_mask.fetch_or(1ull << dev, std::memory_order_relaxed);
+  }
+  const uint32_t tiles = (uint32_t)((k + kAppWG * IPT - 1) / (kAppWG * IPT));
+  // the big tile's LDS leaves one workgroup per CU, which then keeps its next tile's loads in flight
+  const uint32_t grid = IPT == kAppIPTBig && tiles > (uint32_t)ctx->cu_count ? (uint32_t)ctx->cu_count : tiles;
+  hipLaunchKernelGGL(rz_part_append<IPT>, dim3(grid), dim3(kAppWG), lds, s, R, (uint32_t)k, base, (uint32_t)m, blog,
+                     nbins, tiles, ent, cur, stat);
+  RZ_HIP(hipGetLastError());
+  return RZ_OK;
+}
 
 rz_status bucket_marks(rz_ctx* ctx, const int32_t* R, int64_t k, uint32_t base, int64_t m, uint32_t* bits,
                        uint32_t* epoch_ctrl, uint64_t* stat, hipStream_t s) {
   if (!bucket_marks_fit(m) || k < 1 || k > INT32_MAX) return RZ_EINVAL;
+  // the device gives a workgroup the big tile (and its bins' bitmaps) or the small one only
+  const bool big = (size_t)4 * kAppWG * kAppIPTBig + 16384 <= (size_t)ctx->lds_max && k >= kAppBigK;
+  const uint32_t max_blog = big ? kPartMaxBinLog : kPartMaxBinLog - 1;
   uint32_t blog = kPartMinBinLog;
-  while (blog < kPartMaxBinLog && (m >> blog) > 512) ++blog;
+  while (blog < max_blog && (m >> blog) > (big ? 256 : 512)) ++blog;
   const uint32_t nbins = (uint32_t)((m + (1ll << blog) - 1) >> blog);
   rz_status st;
   if ((st = ensure(ctx, ctx->pent, (size_t)nbins << (blog + 2), s)) != RZ_OK) return st;
   if ((st = ensure(ctx, ctx->pcur, (size_t)nbins * 8, s)) != RZ_OK) return st;  // counts, then done counters
-  constexpr size_t lds_max = (size_t)4 << (kPartMaxBinLog - 5);
   const size_t lds_bits = (size_t)4 << (blog - 5);
-  // the big stage where the device gives a workgroup its LDS (plus about 12 KiB static)
-  constexpr size_t lds_app = (size_t)4 * kAppWG * kAppIPT, lds_app_small = (size_t)4 * kAppWG * kAppIPTSmall;
-  const bool big = lds_app + 16384 <= (size_t)ctx->lds_max;
   static std::atomic<uint64_t> attr_mask{0};
   const int dev = ctx->device;
   if (dev < 0 || dev >= 64 || !(attr_mask.load(std::memory_order_relaxed) & (1ull << dev))) {
-    RZ_HIP(hipFuncSetAttribute((const void*)rz_part_bits, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_max));
-    if (big)
-      RZ_HIP(hipFuncSetAttribute((const void*)rz_part_append<kAppIPT>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                 (int)lds_app));
+    const size_t want = (size_t)4 << (kPartMaxBinLog - 5), most = want + 1024 <= (size_t)ctx->lds_max ? want : want / 2;
+    RZ_HIP(hipFuncSetAttribute((const void*)rz_part_bits, hipFuncAttributeMaxDynamicSharedMemorySize, (int)most));
     if (dev >= 0 && dev < 64) attr_mask.fetch_or(1ull << dev, std::memory_order_relaxed);
   }
   uint32_t* cur = (uint32_t*)ctx->pcur.ptr;
   uint32_t* ent = (uint32_t*)ctx->pent.ptr;
   if (big)
-    hipLaunchKernelGGL(rz_part_append<kAppIPT>, dim3((uint32_t)((k + kAppWG * kAppIPT - 1) / (kAppWG * kAppIPT))),
-                       dim3(kAppWG), lds_app, s, R, (uint32_t)k, base, (uint32_t)m, blog, nbins, ent, cur, stat);
+    st = append_launch<kAppIPTBig>(ctx, R, k, base, m, blog, nbins, ent, cur, stat, s);
+  else if (k >= kAppSmallK && (size_t)4 * kAppWG * kAppIPT + 16384 <= (size_t)ctx->lds_max)
+    st = append_launch<kAppIPT>(ctx, R, k, base, m, blog, nbins, ent, cur, stat, s);
   else
-    hipLaunchKernelGGL(rz_part_append<kAppIPTSmall>,
-                       dim3((uint32_t)((k + kAppWG * kAppIPTSmall - 1) / (kAppWG * kAppIPTSmall))), dim3(kAppWG),
-                       lds_app_small, s, R, (uint32_t)k, base, (uint32_t)m, blog, nbins, ent, cur, stat);
+    st = append_launch<kAppIPTSmall>(ctx, R, k, base, m, blog, nbins, ent, cur, stat, s);
+  if (st != RZ_OK) return st;
   uint32_t G = ((uint32_t)ctx->cu_count + nbins - 1) / nbins;  // about one workgroup per CU
   G = G < 1 ? 1 : (G > 16 ? 16 : G);
   hipLaunchKernelGGL(rz_part_bits, dim3(nbins * G), dim3(1024), lds_bits, s, (const uint32_t*)ent, cur, cur + nbins,

@@ -47,6 +47,16 @@ def test_partition_ragged(ctx, oracle):
         _run(ctx, oracle, A, R)
 
 
+@pytest.mark.parametrize("n,k", [((1 << 20) + 3, (1 << 19) + 1), ((1 << 22) + 5, (1 << 21) - 1), ((1 << 22) + 5, 1 << 21),
+                                 ((1 << 25) + 9, (1 << 24) - 1), ((1 << 25) + 9, (1 << 24) + 32769)])
+@pytest.mark.parametrize("pattern", ["uniform", "clustered"])
+def test_partition_mark_tiles(ctx, oracle, n, k, pattern):
+    """Removal counts on both sides of the mark kernel's tile sizes (8, 16 and
+    32 removals per thread; the last in several rounds per workgroup)."""
+    announce("mark tiles", n, k, pattern)
+    _run(ctx, oracle, W.index_payload(n), W.removals(pattern, n, k, seed=k))
+
+
 def test_partition_unaligned_list(ctx, oracle):
     """A list that starts one item into a buffer is not 16-byte aligned: the
     scalar tile kernel handles it."""

@@ -92,7 +92,8 @@ typedef struct rz_tile_config {
                               1, 2 or 4 items, or 1024 with 1 or 2; a slice is one step and max_slices is not
                               used; with premarked tails or RZ_COOPERATIVE: 256 x 4 of variant 4 or 1) */
   int32_t slice_steps; /* variant 2 and batches: steps per slice (0 = 4); variant 5: log2 of the target
-                          number of destination bins, 5..10 (0 = 9); variant 6: log2 of the removals
+                          number of destination bins, 3..12 (0 = 10; a bin is at least 512 KiB of the list,
+                          1 MiB for 16-byte items); variant 6: log2 of the removals
                           each mark workgroup takes, 8..16 (0 = 12) */
   int32_t chunk;       /* variant 2 and batches: queue items taken per ticket (0 = 1) */
 } rz_tile_config;

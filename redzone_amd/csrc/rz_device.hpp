@@ -46,17 +46,44 @@ __device__ __forceinline__ uint32_t lds_bin_add(uint32_t* cnt, uint32_t bin, boo
   }
   return active ? atomicAdd(&cnt[bin], 1u) : 0u;
 }
-// Count only (no ranks), grouped the same way.
-__device__ __forceinline__ void lds_bin_count(uint32_t* cnt, uint32_t bin, bool active) {
-  const uint64_t act = ballot(active);
-  if (!act) return;
-  const int leader = __builtin_ctzll(act);
-  const uint32_t lb = (uint32_t)__builtin_amdgcn_readlane((int)bin, leader);
-  if (ballot(active && bin == lb) == act) {
-    if (lane_id() == leader) atomicAdd(&cnt[lb], (uint32_t)__popcll(act));
-  } else if (active) {
-    atomicAdd(&cnt[bin], 1u);
+// The same for IPT bins per lane, every lane taking part.  A wave without a
+// run in any of its rows takes IPT plain atomics, all in flight together.
+template <int IPT>
+__device__ __forceinline__ void lds_bin_ranks(uint32_t* cnt, const uint32_t (&bin)[IPT], uint32_t (&rank)[IPT]) {
+  bool run = false;
+#pragma unroll
+  for (int q = 0; q < IPT; ++q)
+    run |= ballot(bin[q] != (uint32_t)__builtin_amdgcn_readfirstlane((int)bin[q])) == 0ull;
+  if (!run) {
+#pragma unroll
+    for (int q = 0; q < IPT; ++q) rank[q] = atomicAdd(&cnt[bin[q]], 1u);
+  } else {
+#pragma unroll
+    for (int q = 0; q < IPT; ++q) rank[q] = lds_bin_add(cnt, bin[q], true);
   }
+}
+
+// Keeps the instructions of the two sides apart (a fully unrolled loop would
+// otherwise hold all of its values in registers at once).
+__device__ __forceinline__ void sched_fence() { __builtin_amdgcn_sched_barrier(0); }
+
+// The thread's index, computed anew: index arithmetic on it is not kept in
+// registers from one round of a loop to the next.
+__device__ __forceinline__ uint32_t fresh_tid() {
+  uint32_t t = threadIdx.x;
+  asm volatile("" : "+v"(t));
+  return t;
+}
+
+// The value is in its register here: a load it comes from has been waited for,
+// and none of the stores issued since that load.
+__device__ __forceinline__ void arrived(uint32_t& v) { asm volatile("" : "+v"(v)); }
+__device__ __forceinline__ void arrived(uint64_t& v) { asm volatile("" : "+v"(v)); }
+__device__ __forceinline__ void arrived(uint4& v) {
+  arrived(v.x);
+  arrived(v.y);
+  arrived(v.z);
+  arrived(v.w);
 }
 
 __device__ __forceinline__ uint32_t ld_relaxed(const uint32_t* p) {

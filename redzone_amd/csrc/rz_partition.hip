@@ -391,53 +391,77 @@ constexpr int64_t kPartMaxWindow = (int64_t)1 << 29;  // entry lists of 2 GiB
 constexpr uint32_t kAppWG = 1024;
 // Removals per thread of a tile (dynamic LDS, 4 bytes a removal).  A bigger
 // tile writes longer runs of consecutive words per bin: a run's two ends share
-// their lines with runs of other workgroups, so 32-word runs cost 45 us of the
-// 180 that 2^26 removals take, and 128-word runs 15.  A smaller one gives the
+// their lines with runs of other workgroups, so 32-word runs cost 45 of the
+// 180 us that 2^26 removals took, and 128-word runs 15.  A smaller one gives the
 // chip more workgroups, but each costs its own scan and reservation.  One
 // kernel at k/n = 1/4, us for 8 / 16 / 32 removals per thread: k = 600,000
 // 8.6 / 10.8 / -; 2^22 20.0 / 17.2 / -; 2^24 56.5 / 47.1 / 42.9; 2^26
-// 226 / 191 / 162 (the next tile's loads issued ahead).  With 256 bins instead of
-// 512 there the entries' reader (rz_part_bits) took 73 us instead of 93.
+// 226 / 191 / 162.  At 2^26 the entries' reader (rz_part_bits) took 73 us with
+// 256 bins, 93 with 512.
+// The waves' instructions and the waits count as much: one atomic for count
+// and rank, no branch per removal, and a wait for the next tile's loads that
+// is not one for this tile's stores took the last from 163 to 140 us (3.8 TB/s
+// of removals in and entries out).
 constexpr int kAppIPT = 16, kAppIPTSmall = 8, kAppIPTBig = 32;
 constexpr int64_t kAppSmallK = (int64_t)1 << 21, kAppBigK = (int64_t)1 << 24;
 
-// A workgroup takes tiles blockIdx, blockIdx + grid, ...
-template <int IPT>
+// A workgroup takes tiles blockIdx, blockIdx + grid, ...  ALL: the window is the
+// whole list, so every removal of a valid list falls into a bin and nothing
+// branches on it.
+template <int IPT, bool ALL>
 __global__ __launch_bounds__(1024) void rz_part_append(const int32_t* __restrict__ R, uint32_t k, uint32_t base,
                                                         uint32_t m, uint32_t blog, uint32_t nbins, uint32_t ntiles,
                                                         uint32_t* __restrict__ ent, uint32_t* __restrict__ cur,
                                                         uint64_t* __restrict__ stat) {
   constexpr uint32_t kAppS = kAppWG * IPT;
-  __shared__ uint32_t s_cnt[kPartMaxBins], s_lbase[kPartMaxBins];
+  __shared__ uint32_t s_cnt[kPartMaxBins + 1], s_lbase[kPartMaxBins + 1];
   __shared__ uint32_t s_tmp[kAppWG / kWave + 1];
   extern __shared__ __align__(16) unsigned char dyn[];
   uint32_t* s_stage = (uint32_t*)dyn;
   const uint32_t tid = threadIdx.x;
   if (stat && blockIdx.x == 0 && tid == 0) st_relaxed(stat, (uint64_t)0);
   uint32_t next[IPT];
-  auto load = [&](uint32_t tile) {  // all loads of a tile in flight together
+  auto load = [&](uint32_t tile) {  // all loads of a tile in flight together; past the end the last removal again
     const int32_t* Rt = R + (size_t)tile * kAppS;
-    const uint32_t left = k - tile * kAppS;
-#pragma unroll
-    for (int j = 0; j < IPT; ++j) next[j] = j * kAppWG + tid < left ? (uint32_t)Rt[j * kAppWG + tid] : 0xffffffffu;
-  };
-  load(blockIdx.x);
-  for (uint32_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-    for (uint32_t w = tid; w < nbins; w += kAppWG) s_cnt[w] = 0u;
-    __syncthreads();
-    // positions in the window; 0xffffffff (>= m) for none (0xffffffff - base >= 2^31 > m)
-    uint32_t r[IPT], rank[IPT / 2];  // two ranks (below 2^15) to a register: IPT 32 leaves none to spare
+    const uint32_t last = k - tile * kAppS - 1, t = fresh_tid();
 #pragma unroll
     for (int j = 0; j < IPT; ++j) {
-      const uint32_t p = next[j] - base;
-      r[j] = p < m ? p : 0xffffffffu;
+      next[j] = (uint32_t)Rt[min(j * kAppWG + t, last)];
+      if (j % 4 == 3) sched_fence();
     }
-    // count and rank in one pass: the count's atomic returns the rank (a wave
-    // whose removals share one bin, a run, takes one atomic)
+  };
+  auto wait_loads = [&]() {
 #pragma unroll
-    for (int j = 0; j < IPT; j += 2) {
-      rank[j / 2] = lds_bin_add(s_cnt, r[j] >> blog, r[j] < m);
-      rank[j / 2] |= lds_bin_add(s_cnt, r[j + 1] >> blog, r[j + 1] < m) << 16;
+    for (int j = 0; j < IPT; ++j) arrived(next[j]);
+  };
+  load(blockIdx.x);
+  wait_loads();
+  for (uint32_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+    for (uint32_t w = tid; w <= nbins; w += kAppWG) s_cnt[w] = 0u;
+    __syncthreads();
+    // positions in the window, bin nbins for none
+    uint32_t r[IPT], rank[IPT / 2];  // two ranks (below 2^15) to a register: 32 removals leave none to spare
+    const uint32_t left = k - tile * kAppS, t0 = fresh_tid();
+#pragma unroll
+    for (int j = 0; j < IPT; ++j) {
+      r[j] = next[j] - base;
+      if (j * kAppWG + t0 >= left || r[j] >= m) r[j] = 0xffffffffu;
+    }
+    // count and rank in one pass: the count's atomic returns the rank
+#pragma unroll
+    for (int h = 0; h < IPT; h += 8) {
+      uint32_t bin[8], rk[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) bin[j] = ALL ? min(r[h + j] >> blog, nbins) : r[h + j] >> blog;
+      if constexpr (ALL) {
+        lds_bin_ranks<8>(s_cnt, bin, rk);
+      } else {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) rk[j] = lds_bin_add(s_cnt, bin[j], r[h + j] < m);
+      }
+#pragma unroll
+      for (int j = 0; j < 8; j += 2) rank[(h + j) / 2] = rk[j] | rk[j + 1] << 16;
+      sched_fence();
     }
     __syncthreads();
     // exclusive prefix over the bins (one bin per thread), then room in each bin's list
@@ -447,27 +471,44 @@ __global__ __launch_bounds__(1024) void rz_part_append(const int32_t* __restrict
     // the reservation's atomics stay in flight while the removals are staged:
     // only the write-out below needs their results
     uint32_t gb = 0u;
-    if (tid < nbins) {
-      s_lbase[tid] = ex;
-      if (c) gb = add_relaxed(&cur[tid], c);
-    }
+    if (tid < nbins) s_lbase[tid] = ex;
+    if (tid == 0) s_lbase[nbins] = total;  // removals outside the window come last
+    if (c) gb = add_relaxed(&cur[tid], c);
     __syncthreads();
     uint32_t bl = blog;
     asm volatile("" : "+s"(bl));  // the bins are computed again: IPT of them kept from above would not fit in registers
 #pragma unroll
-    for (int j = 0; j < IPT; ++j)
-      if (r[j] < m) s_stage[s_lbase[r[j] >> bl] + ((rank[j / 2] >> 16 * (j & 1)) & 0xffffu)] = r[j];
-    if (tid < nbins) s_cnt[tid] = gb - ex;  // a staged entry's place in its bin's list, less its place in the stage
-    // the next tile's loads go out ahead of this tile's stores: a wait for them never waits for the stores
-    if (tile + gridDim.x < ntiles) load(tile + gridDim.x);
-    __syncthreads();
-    for (uint32_t t = tid; t < total; t += kAppWG) {
-      const uint32_t v = s_stage[t];
-      const uint32_t bz = v >> blog;
-      const uint32_t g = s_cnt[bz] + t;
-      if (g < (1u << blog)) ent[((size_t)bz << blog) + g] = v;  // more only with duplicate removals
+    for (int j = 0; j < IPT; ++j) {
+      if (ALL || r[j] < m)
+        s_stage[s_lbase[min(r[j] >> bl, nbins)] + ((rank[j / 2] >> 16 * (j & 1)) & 0xffffu)] = r[j];
+      if (j % 8 == 7) sched_fence();
     }
+    if (tid < nbins) s_cnt[tid] = gb - ex;  // a staged entry's place in its bin's list, less its place in the stage
+    // the next tile's loads go out ahead of this tile's stores, and the wait
+    // for them behind IPT stores, whatever the tile holds, is one for the
+    // loads alone
+    const bool more = tile + gridDim.x < ntiles;
+    if (more) load(tile + gridDim.x);
     __syncthreads();
+    if (ALL && more) {
+      const uint32_t t1 = fresh_tid();
+#pragma unroll
+      for (int j = 0; j < IPT; ++j) {
+        const uint32_t t = j * kAppWG + t1, v = s_stage[t], bz = min(v >> blog, nbins), g = s_cnt[bz] + t;
+        // a place past the bin's list only with duplicate removals, none only with indices out of range
+        ent[t < total && g < (1u << blog) ? ((size_t)bz << blog) + g : (size_t)nbins << blog] = v;
+        if (j % 4 == 3) sched_fence();
+      }
+      wait_loads();
+      __syncthreads();
+    } else {
+      for (uint32_t t = tid; t < total; t += kAppWG) {
+        const uint32_t v = s_stage[t], bz = v >> blog, g = s_cnt[bz] + t;
+        if (g < (1u << blog)) ent[((size_t)bz << blog) + g] = v;
+      }
+      if (more) wait_loads();
+      __syncthreads();
+    }
   }
 }
 
@@ -534,20 +575,20 @@ __global__ __launch_bounds__(1024) void rz_part_bits(const uint32_t* __restrict_
 
 bool bucket_marks_fit(int64_t m) { return m > 0 && m <= kPartMaxWindow; }
 
-template <int IPT>
+template <int IPT, bool ALL>
 static rz_status append_launch(rz_ctx* ctx, const int32_t* R, int64_t k, uint32_t base, int64_t m, uint32_t blog,
                                uint32_t nbins, uint32_t* ent, uint32_t* cur, uint64_t* stat, hipStream_t s) {
   constexpr size_t lds = (size_t)4 * kAppWG * IPT;
   static std::atomic<uint64_t> attr_mask{0};
   const int dev = ctx->device;
   if (dev < 0 || dev >= 64 || !(attr_mask.load(std::memory_order_relaxed) & (1ull << dev))) {
-    RZ_HIP(hipFuncSetAttribute((const void*)rz_part_append<IPT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    RZ_HIP(hipFuncSetAttribute((const void*)rz_part_append<IPT, ALL>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     if (dev >= 0 && dev < 64) attr_mask.fetch_or(1ull << dev, std::memory_order_relaxed);
   }
   const uint32_t tiles = (uint32_t)((k + kAppWG * IPT - 1) / (kAppWG * IPT));
   // the big tile's LDS leaves one workgroup per CU, which then keeps its next tile's loads in flight
   const uint32_t grid = IPT == kAppIPTBig && tiles > (uint32_t)ctx->cu_count ? (uint32_t)ctx->cu_count : tiles;
-  hipLaunchKernelGGL(rz_part_append<IPT>, dim3(grid), dim3(kAppWG), lds, s, R, (uint32_t)k, base, (uint32_t)m, blog,
+  hipLaunchKernelGGL((rz_part_append<IPT, ALL>), dim3(grid), dim3(kAppWG), lds, s, R, (uint32_t)k, base, (uint32_t)m, blog,
                      nbins, tiles, ent, cur, stat);
   RZ_HIP(hipGetLastError());
   return RZ_OK;
@@ -563,7 +604,7 @@ rz_status bucket_marks(rz_ctx* ctx, const int32_t* R, int64_t k, uint32_t base, 
   while (blog < max_blog && (m >> blog) > (big ? 256 : 512)) ++blog;
   const uint32_t nbins = (uint32_t)((m + (1ll << blog) - 1) >> blog);
   rz_status st;
-  if ((st = ensure(ctx, ctx->pent, (size_t)nbins << (blog + 2), s)) != RZ_OK) return st;
+  if ((st = ensure(ctx, ctx->pent, ((size_t)nbins << (blog + 2)) + 4, s)) != RZ_OK) return st;
   if ((st = ensure(ctx, ctx->pcur, (size_t)nbins * 8, s)) != RZ_OK) return st;  // counts, then done counters
   const size_t lds_bits = (size_t)4 << (blog - 5);
   static std::atomic<uint64_t> attr_mask{0};
@@ -575,12 +616,13 @@ rz_status bucket_marks(rz_ctx* ctx, const int32_t* R, int64_t k, uint32_t base, 
   }
   uint32_t* cur = (uint32_t*)ctx->pcur.ptr;
   uint32_t* ent = (uint32_t*)ctx->pent.ptr;
-  if (big)
-    st = append_launch<kAppIPTBig>(ctx, R, k, base, m, blog, nbins, ent, cur, stat, s);
-  else if (k >= kAppSmallK && (size_t)4 * kAppWG * kAppIPT + 16384 <= (size_t)ctx->lds_max)
-    st = append_launch<kAppIPT>(ctx, R, k, base, m, blog, nbins, ent, cur, stat, s);
-  else
-    st = append_launch<kAppIPTSmall>(ctx, R, k, base, m, blog, nbins, ent, cur, stat, s);
+  const bool all = epoch_ctrl != nullptr;  // the partition: base 0, m = n
+  const bool mid = k >= kAppSmallK && (size_t)4 * kAppWG * kAppIPT + 16384 <= (size_t)ctx->lds_max;
+#define RZ_APPEND(I)                                                                       \
+  (all ? append_launch<I, true>(ctx, R, k, base, m, blog, nbins, ent, cur, stat, s)        \
+       : append_launch<I, false>(ctx, R, k, base, m, blog, nbins, ent, cur, stat, s))
+  st = big ? RZ_APPEND(kAppIPTBig) : mid ? RZ_APPEND(kAppIPT) : RZ_APPEND(kAppIPTSmall);
+#undef RZ_APPEND
   if (st != RZ_OK) return st;
   uint32_t G = ((uint32_t)ctx->cu_count + nbins - 1) / nbins;  // about one workgroup per CU
   G = G < 1 ? 1 : (G > 16 ? 16 : G);

@@ -25,7 +25,7 @@ enum CtrlWord : int {
   kCtrlMoveExit = 240,    // workgroups of the fused kernel that have finished (reset by the last)
   kCtrlMarkDone = 256,    // groups of mark workgroups of the one-launch form that are done (reset by the last)
   kCtrlMarkReady = 288,   // 8 copies, one line apart (one per XCD): move-pair epoch + 1 once every mark is in
-  kCtrlGatherExit = 544,  // tiles of the one-pass gather that have finished (reset by the last)
+  kCtrlGatherExit = 544,  // groups of 64 tiles of the one-pass gather that have finished (reset by the last)
   kCtrlMarkGroup = 576,   // 8 copies, one line apart: mark workgroups of the one-launch form done, per
                           // group of ids equal mod 8 (reset by the last of the group)
   kCtrlSpinCap = 832,     // test hook: polls before a bounded wait gives up (0 = the wait's own limit)
@@ -89,8 +89,8 @@ struct rz_ctx {
   rz::DeviceBuffer counts;     // per-slice orphan counts (uint64: dest | src << 32)
   rz::DeviceBuffer orphans;    // dest orphans when RZ_PRESERVE_REMOVALS is set
   rz::DeviceBuffer status;     // look-back status words of the partition
-  rz::DeviceBuffer ploaded;    // partition: per tile, the epoch once its items are loaded
-  rz::DeviceBuffer pgcnt;      // partition: per 64 tiles, the number of them loaded (zero between calls)
+  rz::DeviceBuffer ploaded;    // partition and gather: per tile, the epoch once its items are loaded
+  rz::DeviceBuffer pgcnt;      // per 64 tiles, the number of them loaded (partition) or done (gather); zero between calls
   rz::DeviceBuffer pgdone;     // partition: per 64 tiles, the epoch once all of them are loaded
   rz::DeviceBuffer pent;       // partition's bucketed marks: per 2^19-position bin, its removals
   rz::DeviceBuffer pcur;       // partition's bucketed marks: per bin its count, then per bin a done counter (zero between calls)

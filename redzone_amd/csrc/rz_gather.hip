@@ -2,21 +2,19 @@
 //
 // Preserve-list gather (paper p.14, eq. 3): A'[i] = A[P[i]] for i < p, P
 // strictly ascending.  Two forms:
-//  - one pass, in place (p >= kGatherOnePassMin): tiles of outputs in
-//    blockIdx order; a tile writes once every earlier tile has read its
-//    sources (loaded flags, summarised per group of 64 tiles), the same guard
-//    as the partition's in-place compaction.  Streams P, A[P] and the output
-//    once: 4.25 TB/s at p = 0.99 n on MI355X.
-//  - two passes (small p): gather into context scratch with no ordering
+//  - one pass, in place, no scratch for the items: tiles of outputs in
+//    blockIdx order; a tile writes once every earlier tile whose sources lie
+//    in its output range has read them.  At most two tiles do: the sources in
+//    T positions are at most T consecutive entries of P.  A tile finds them
+//    with a search over the tiles' first entries.
+//  - two passes (gather_sparse below): gather into context scratch with no ordering
 //    between workgroups, then a device copy back to the front of the list.
-//    Below a few million items the one-pass form's flag traffic and serial
-//    wait cost more than the copy.
 #include "rz_ctx.hpp"
 #include "rz_device.hpp"
 
 namespace rz {
 
-constexpr uint32_t kGatherOnePassMin = 1u << 22;
+constexpr uint32_t kFlagStride = 16;  // words between the tiles' flags: polls do not meet the neighbours' stores
 
 template <typename T, int WG, int IPT>
 __global__ __launch_bounds__(WG) void rz_gather_kernel(const T* __restrict__ A, uint32_t n,
@@ -36,20 +34,26 @@ __global__ __launch_bounds__(WG) void rz_gather_kernel(const T* __restrict__ A, 
   }
 }
 
-// One pass, in place: tile t gathers outputs [t*TILE, (t+1)*TILE) into
-// registers, sets its loaded flag (and its group word once all 64 tiles of
-// its group have loaded), waits until every earlier tile has loaded, and
-// writes its outputs.  The sources of a tile lie at or after its first output
-// (P ascends, P[i] >= i), so only earlier tiles' sources can sit in its output
-// range, and later tiles never write below it.  Flags carry the call's tag,
-// the epoch word plus one; the last tile to leave (every tile has read the
-// epoch by then) stores the tag as the new epoch, so no flag is ever cleared
-// and no separate launch advances the epoch.
+// One pass, in place: tile t gathers outputs [t T, (t + 1) T) into registers,
+// sets its loaded flag, waits for the two earlier tiles that may still have to
+// read from its output range, and writes.  P ascends, so P[i] >= i: a tile's sources lie at or after
+// its own outputs, and only earlier tiles' sources can sit in its output range.
+// With `lo` the last tile whose first source lies before t T, the sources in
+// [t T, (t + 1) T) start in tile lo and, being at most T, end in tile lo + 1.
+// Tiles are dispatched in id order and wait on earlier ones only.  Flags carry
+// the call's tag, the epoch word plus one; the last tile to leave (every tile
+// has read the epoch by then) stores the tag as the new epoch, so no flag is
+// ever cleared and no separate launch advances the epoch.
+//
+// Bound: P, the sources' lines and the outputs, streamed; for small p the
+// chain load P, load sources, flag, poll, write.  Waiting for every earlier
+// tile (a counter per 64 tiles, whole groups polled) took 98 us for 2^24.5 of
+// 2.5 p 4-byte items where this takes 89, and 23.3 against 19.4 for 2^22 at 95%.
 template <typename T, int WG, int IPT>
 __global__ __launch_bounds__(WG) void rz_gather_inplace(T* __restrict__ A, uint32_t n,
                                                         const int32_t* __restrict__ P, uint32_t p,
                                                         uint32_t* __restrict__ loaded, uint32_t* __restrict__ gcnt,
-                                                        uint32_t* __restrict__ gdone, uint32_t ntiles,
+                                                        uint32_t ntiles, uint32_t follow,
                                                         uint32_t* __restrict__ ctrl) {
   constexpr uint32_t TILE = WG * IPT;
   const uint32_t t = blockIdx.x, i0 = t * TILE;
@@ -68,40 +72,46 @@ __global__ __launch_bounds__(WG) void rz_gather_inplace(T* __restrict__ A, uint3
     v[j] = T();
     if (i < p) v[j] = A[src[j] < n ? src[j] : i];  // an index out of range (invalid list) reads in bounds
   }
-  wait_all_memory();
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    st_relaxed(&loaded[t], epoch);
-    const uint32_t g = t >> 6, members = min(64u, ntiles - (g << 6));
-    if (add_relaxed(&gcnt[g], 1u) == members - 1u) {
-      st_relaxed(&gcnt[g], 0u);
-      st_relaxed(&gdone[g], epoch);
+  uint32_t lo = 0;  // P[u TILE] < i0 for tiles u in [0, lo], or for none and lo is 0
+  if (threadIdx.x < kWave && t > 0) {
+    // First the 64 tiles around where a list as dense as up to here would have
+    // it (one round of loads, behind the items'), then 64-way over the side it lies on.
+    const float first = (float)(uint32_t)__builtin_amdgcn_readfirstlane((int)src[0]);  // P[i0]
+    const float guess = first > 0.f ? (float)i0 * ((float)i0 / first) * (1.f / TILE) : 0.f;
+    const uint32_t g = guess < (float)t ? (uint32_t)guess : t, w0 = g > 32u ? g - 32u : 0u, w = w0 + lane_id();
+    uint64_t below = ballot(w < t && (uint32_t)P[min(w, t) * TILE] < i0);
+    uint32_t len = 0;  // lo is in [lo, lo + len)
+    if (below) {
+      const uint32_t last = 63u - (uint32_t)__builtin_clzll(below);
+      lo = w0 + last;
+      if (last == 63u) len = t - lo;
+    } else {
+      len = w0;
+    }
+    while (len > 1) {
+      const uint32_t step = (len + kWave - 1) / kWave;
+      const uint32_t u = lo + lane_id() * step;
+      below = ballot(lane_id() * step < len && (uint32_t)P[min(u, t) * TILE] < i0);
+      const uint32_t last = below ? 63u - (uint32_t)__builtin_clzll(below) : 0u;
+      lo += last * step;
+      len = min(step, len - last * step);
     }
   }
+  wait_all_memory();
+  __syncthreads();
+  if (threadIdx.x == 0) st_relaxed(&loaded[t * kFlagStride], epoch);
   if (threadIdx.x < kWave && t != 0) {
-    // every earlier tile has loaded: whole groups by their word, this tile's
-    // own group tile by tile; up to 8 words per lane per round trip
-    const int lane = lane_id();
-    const uint32_t g1 = t >> 6, tb = g1 << 6;
-    const uint32_t total = g1 + (t - tb);
+    // lanes 0 and 1: the tiles that may read here; lanes 2 on: the `follow` tiles just before this one
+    const uint32_t l = lane_id(), u = l < 2 ? lo + l : t - min(t, l - 1u);
+    const bool wait = l < 2 + follow && u < t;
     uint32_t spins = 0, pause = 1;
-    for (uint32_t c0 = 0; c0 < total;) {
-      bool ok = true;
-#pragma unroll
-      for (int r = 0; r < 8; ++r) {
-        const uint32_t c = c0 + (uint32_t)(r * kWave + lane);
-        if (c < total) ok &= (c < g1 ? ld_relaxed(&gdone[c]) : ld_relaxed(&loaded[tb + (c - g1)])) == epoch;
+    while (ballot(wait && ld_relaxed(&loaded[u * kFlagStride]) != epoch)) {
+      if (++spins > spin_cap(ctrl, 1u << 22)) {
+        if (lane_id() == 0) or_relaxed(&ctrl[kCtrlError], kErrLookbackTimeout);
+        break;
       }
-      if (ballot(!ok)) {
-        if (++spins > spin_cap(ctrl, 1u << 22)) {
-          if (lane == 0) or_relaxed(&ctrl[kCtrlError], kErrLookbackTimeout);
-          break;
-        }
-        for (uint32_t i = 0; i < pause; ++i) __builtin_amdgcn_s_sleep(1);
-        if (pause < 16u) pause <<= 1;
-        continue;
-      }
-      c0 += 8 * kWave;
+      for (uint32_t i = 0; i < pause; ++i) __builtin_amdgcn_s_sleep(1);
+      if (pause < 16u) pause <<= 1;
     }
   }
   __syncthreads();
@@ -110,24 +120,35 @@ __global__ __launch_bounds__(WG) void rz_gather_inplace(T* __restrict__ A, uint3
     const uint32_t i = i0 + j * WG + threadIdx.x;
     if (i < p) A[i] = v[j];
   }
-  if (threadIdx.x == 0 && add_relaxed(&ctrl[kCtrlGatherExit], 1u) == ntiles - 1u) {
-    st_relaxed(&ctrl[kCtrlGatherExit], 0u);
-    st_relaxed(&ctrl[kCtrlEpoch], e0 + 1u);
+  if (threadIdx.x == 0) {
+    // exits counted per 64 tiles, then the groups: same-address atomics take about 11 ns each
+    const uint32_t g = t >> 6, members = min(64u, ntiles - (g << 6));
+    if (add_relaxed(&gcnt[g], 1u) == members - 1u) {
+      st_relaxed(&gcnt[g], 0u);
+      if (add_relaxed(&ctrl[kCtrlGatherExit], 1u) == ((ntiles + 63u) >> 6) - 1u) {
+        st_relaxed(&ctrl[kCtrlGatherExit], 0u);
+        st_relaxed(&ctrl[kCtrlEpoch], e0 + 1u);
+      }
+    }
   }
 }
 
-template <typename T, int IPT>
+template <typename T, int WG, int IPT>
 static rz_status gather_inplace_launch(rz_ctx* ctx, T* A, uint32_t n, const int32_t* P, uint32_t p, hipStream_t s) {
-  constexpr int WG = 1024;
   const uint32_t tiles = (p + WG * IPT - 1) / (WG * IPT);
   const uint32_t groups = (tiles + 63) / 64;
   rz_status st;
-  if ((st = ensure(ctx, ctx->ploaded, (size_t)tiles * 4, s)) != RZ_OK) return st;
+  if ((st = ensure(ctx, ctx->ploaded, (size_t)tiles * kFlagStride * 4, s)) != RZ_OK) return st;
   if ((st = ensure(ctx, ctx->pgcnt, (size_t)groups * 4, s)) != RZ_OK) return st;
-  if ((st = ensure(ctx, ctx->pgdone, (size_t)groups * 4, s)) != RZ_OK) return st;
   uint32_t* ctrl = (uint32_t*)ctx->ctrl.ptr;
+  // Fewer than half of many 8- or 16-byte items kept: sources and outputs are
+  // far apart, and tiles that follow each other read and write them in longer
+  // stretches (2^24.5 of 2.5 p 16-byte items 258 us, 270 each on its own; 8-byte
+  // 146 and 149).  Dense and 4-byte lists lose by it (8-byte, 95% kept 104
+  // against 97).
+  const uint32_t follow = sizeof(T) >= 8 && p >= 1u << 22 && (uint64_t)p * 2 < n ? 32u : 0u;
   hipLaunchKernelGGL((rz_gather_inplace<T, WG, IPT>), dim3(tiles), dim3(WG), 0, s, A, n, P, p,
-                     (uint32_t*)ctx->ploaded.ptr, (uint32_t*)ctx->pgcnt.ptr, (uint32_t*)ctx->pgdone.ptr, tiles, ctrl);
+                     (uint32_t*)ctx->ploaded.ptr, (uint32_t*)ctx->pgcnt.ptr, tiles, follow, ctrl);
   RZ_HIP(hipGetLastError());
   return RZ_OK;
 }
@@ -145,10 +166,24 @@ static rz_status gather_launch(rz_ctx* ctx, T* A, uint32_t n, const int32_t* P, 
   return RZ_OK;
 }
 
+// Fewer than an eighth of the items kept, and fewer than 2^22: every item
+// comes from a page of its own, and many small workgroups with nothing to
+// wait for hide that better (p = 2^19 of 50 p 4-byte items: 11.2 us two passes,
+// 12.8-14 one; 500 p: 14.3 and 21).  From an eighth up one launch in place is
+// the faster one: 2^17 of 2.5 p 9.4 -> 7.0 us, 2^22 of 8-byte items
+// 25.5 -> 22.7 at 95% kept.
+static bool gather_sparse(int64_t n, int64_t p) { return p * 8 < n && p < ((int64_t)1 << 22); }
+
 template <typename T, int IPT>
 static rz_status gather_form(rz_ctx* ctx, void* A, int64_t n, const int32_t* P, int64_t p, hipStream_t s) {
-  if ((uint32_t)p >= kGatherOnePassMin) return gather_inplace_launch<T, IPT>(ctx, (T*)A, (uint32_t)n, P, (uint32_t)p, s);
-  return gather_launch<T, IPT>(ctx, (T*)A, (uint32_t)n, P, (uint32_t)p, s);
+  if (gather_sparse(n, p)) return gather_launch<T, IPT>(ctx, (T*)A, (uint32_t)n, P, (uint32_t)p, s);
+  // Big tiles: every workgroup pays for its dispatch, flags and exit (2^21 of
+  // 5 M 8-byte items: 245 tiles of 1,024 x 8 14.6 us, 489 of 512 x 8 18.6).
+  // With a quarter of the CUs or fewer at work, half tiles win (2^19 of 2.5 p
+  // items: 8.4 against 9.2 us, 4-byte 7.8 against 8.4).
+  if (p <= (int64_t)1024 * IPT * (ctx->cu_count / 4))
+    return gather_inplace_launch<T, 1024, IPT / 2>(ctx, (T*)A, (uint32_t)n, P, (uint32_t)p, s);
+  return gather_inplace_launch<T, 1024, IPT>(ctx, (T*)A, (uint32_t)n, P, (uint32_t)p, s);
 }
 
 }  // namespace rz

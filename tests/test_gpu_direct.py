@@ -118,3 +118,29 @@ def test_add_remove_sources(oracle, esz, k, variant):
             assert first_mismatch(cap[: m - k].cpu().numpy(), want2[: m - k]) < 0
     assert ctx.check_errors() == 0
     ctx.close()
+
+
+@pytest.mark.parametrize("esz", [4, 8, 16])
+@pytest.mark.parametrize("p", [1, 1000, 8192, 8193, 64 * 8192, 64 * 8192 + 1, 65 * 4096 + 3, (1 << 22) + 17])
+def test_gather_tiles(ctx, esz, p):
+    """The one-pass gather's tiles and its search for the tiles that read from
+    a tile's outputs: kept items in one run at the end, behind a gap, in runs,
+    spread out, and dense at first then sparse (so that the guessed position is
+    wrong), in one context with calls of both tile sizes."""
+    keep = {"run at the end": torch.arange(p) + p // 2,
+            "gap": torch.cat([torch.arange(p // 2), torch.arange(p // 2, p) + p // 3 + 5]),
+            "spread": torch.arange(p) * 3 + 1,
+            "sparse then dense": torch.cat([torch.arange(p // 8) * 30, p // 8 * 30 + torch.arange(p - p // 8)]),
+            "dense then sparse": torch.cat([torch.arange(p - p // 8), p - p // 8 + torch.arange(p // 8) * 30]),
+            "all": torch.arange(p)}
+    for name, P in keep.items():
+        n = int(P[-1]) + 1
+        if p * 8 < n or n * esz > 1 << 28:
+            continue
+        announce("gather tiles", esz, p, name)
+        A = torch.empty((n,) if esz == 4 else (n, esz // 4), dtype=torch.int32, device="cuda")
+        ctx.gen_payload(A, p)
+        want = A[P.cuda()].clone()
+        assert ctx.gather_preserve(A, P.to(torch.int32).cuda(), n=n) == p
+        assert torch.equal(A[:p], want)
+    assert ctx.check_errors() == 0

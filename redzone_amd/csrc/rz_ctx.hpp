@@ -67,6 +67,7 @@ enum StampIndex : int {
 // internal flag: the tail bitmap was set by the caller (rz_remove_premarked)
 constexpr uint32_t kFlagPremarked = 0x80000000u;
 
+constexpr uint32_t kFlagStride = 16;  // words between tiles' loaded flags: polls do not meet the neighbours' stores
 constexpr int kMaxSlices = 4096;  // cap on move-kernel workgroups (LDS prefix in the pairing kernel)
 
 struct DeviceBuffer {
@@ -90,8 +91,8 @@ struct rz_ctx {
   rz::DeviceBuffer orphans;    // dest orphans when RZ_PRESERVE_REMOVALS is set
   rz::DeviceBuffer status;     // look-back status words of the partition
   rz::DeviceBuffer ploaded;    // partition and gather: per tile, the epoch once its items are loaded
-  rz::DeviceBuffer pgcnt;      // per 64 tiles, the number of them loaded (partition) or done (gather); zero between calls
-  rz::DeviceBuffer pgdone;     // partition: per 64 tiles, the epoch once all of them are loaded
+  rz::DeviceBuffer pgcnt;      // gather: per 64 tiles, the number of them done (zero between calls)
+  rz::DeviceBuffer ptrem;      // partition: removals per bin, then per tile (written by the bucketed marks)
   rz::DeviceBuffer pent;       // partition's bucketed marks: per 2^19-position bin, its removals
   rz::DeviceBuffer pcur;       // partition's bucketed marks: per bin its count, then per bin a done counter (zero between calls)
   rz::DeviceBuffer ctrl;       // control block (rz::CtrlWord)
@@ -187,9 +188,16 @@ bool dense_bucket_marks(const rz_tile_config& cfg, int64_t k, uint32_t flags);
 // r - base of the m-bit bitmap `bits` (zero on entry); epoch_ctrl (may be
 // null) gets the compaction's epoch started, stat (may be null) the number of
 // removals in the window.  m up to 2^29 (bucket_marks_fit).
+// With tc, the removals per tile of 2^tlog positions and per bin of 2^tpb
+// tiles are counted where a bin has one workgroup (tc->made).
+struct TileCounts {
+  uint32_t tlog = 0, tpb = 0;
+  uint32_t *trem = nullptr, *brem = nullptr;
+  bool made = false;
+};
 bool bucket_marks_fit(int64_t m);
 rz_status bucket_marks(rz_ctx* ctx, const int32_t* R, int64_t k, uint32_t base, int64_t m, uint32_t* bits,
-                       uint32_t* epoch_ctrl, uint64_t* stat, hipStream_t s);
+                       uint32_t* epoch_ctrl, uint64_t* stat, hipStream_t s, TileCounts* tc = nullptr);
 // dense form: whether (cfg, n, k) can be launched (checked before any kernel of a call runs)
 bool dense_shape_ok(const rz_ctx* ctx, const rz_tile_config& cfg, uint32_t esz, int64_t n, int64_t k, uint32_t flags);
 // After a failed device check: zero the scratch the kernels keep zero between

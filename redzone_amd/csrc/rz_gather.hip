@@ -14,8 +14,6 @@
 
 namespace rz {
 
-constexpr uint32_t kFlagStride = 16;  // words between the tiles' flags: polls do not meet the neighbours' stores
-
 template <typename T, int WG, int IPT>
 __global__ __launch_bounds__(WG) void rz_gather_kernel(const T* __restrict__ A, uint32_t n,
                                                        const int32_t* __restrict__ P, uint32_t p,

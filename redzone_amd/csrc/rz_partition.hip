@@ -6,10 +6,10 @@
 // (StreamCompact_OneBlock, redzone.hxx:526-603) or with thrust::remove
 // (Thrust_remove.hxx:15-17).  Here:
 //   rz_mark_all   sets one bit per removal in an n-bit bitmap (payload
-//                 agnostic) and bumps the look-back epoch; lists of 2^23
-//                 items and more with 2^20 removals and more group the
-//                 marks by bitmap region first (bucket_marks, rz_dense.hip)
-//                 and write every bitmap word whole;
+//                 agnostic) and bumps the look-back epoch; larger lists
+//                 (kPartBucketMinN, kPartBucketMinK) group the marks by
+//                 bitmap region first (bucket_marks), write every bitmap
+//                 word whole and count the removals of every tile;
 //   rz_compact    one pass over all n items in tiles of WG*IPT, tile id =
 //                 workgroup id (workgroups are dispatched in id order).  Each
 //                 tile ranks its kept items with wave ballots and one LDS scan,
@@ -23,12 +23,13 @@
 //                 The 16-byte aligned form (rz_compact_vec) publishes a
 //                 tile's kept count as soon as it has the tile's bitmap words
 //                 (the count needs no item), so the look-back never waits for
-//                 loads; the in-place guard is separate: a tile sets its
-//                 loaded flag (and its group of 64 tiles a group word) once
-//                 its items are in registers, and a tile writes only after
-//                 every tile overlapping its output range has loaded.  It
-//                 stages the kept items in LDS and writes them as whole
-//                 vectors.
+//                 loads; where the marks counted the removals per tile, it
+//                 adds them up instead and there is no look-back.  The
+//                 in-place guard is separate: a tile sets its loaded flag
+//                 once its items are in registers, and a tile writes only
+//                 after the (at most two) tiles overlapping its output range
+//                 have loaded.  It stages the kept items in LDS and writes
+//                 them as whole vectors.
 #include <atomic>
 
 #include "rz_compact_dev.hpp"
@@ -124,11 +125,18 @@ struct CompactShared {
   uint32_t excl;
 };
 
-template <typename T, int WG, int VPT>
+// COUNTED: the mark kernel counted the removals of every tile (trem) and of
+// every bin of 2^tpb tiles (brem); a tile adds up what lies before it instead
+// of publishing its count and looking back.
+// Bound: the items in and out.  n = 2^28 4-byte items, a quarter removed: 398 us
+// (4.7 TB/s), 439 with the look-back; n = 16 M 27 us and 31, 33 when a tile also
+// waited for every earlier tile from its output range on.
+template <typename T, int WG, int VPT, bool COUNTED>
 __global__ __launch_bounds__(WG) void rz_compact_vec(T* __restrict__ A, uint32_t n, uint32_t* __restrict__ bits,
-                                                      uint64_t* __restrict__ status, uint32_t* __restrict__ loaded,
-                                                      uint32_t* __restrict__ gcnt, uint32_t* __restrict__ gdone,
-                                                      uint32_t ntiles, uint32_t* __restrict__ ctrl) {
+                                                      uint64_t* __restrict__ status,
+                                                      const uint32_t* __restrict__ trem,
+                                                      const uint32_t* __restrict__ brem, uint32_t tpb,
+                                                      uint32_t* __restrict__ loaded, uint32_t* __restrict__ ctrl) {
   constexpr int V = 16 / sizeof(T);
   constexpr int NW = WG / kWave;
   constexpr int E = VPT * NW;
@@ -168,7 +176,14 @@ __global__ __launch_bounds__(WG) void rz_compact_vec(T* __restrict__ A, uint32_t
   };
   // wave 0 loads its items after it has published the tile's count, so that
   // its status store does not wait behind them (loads and stores retire in order)
-  if (wave != 0) load_items();
+  uint32_t removed = 0;  // before this tile (wave 0, COUNTED)
+  if (COUNTED && wave == 0) {
+    const uint32_t b = t >> tpb, inb = t & ((1u << tpb) - 1u), first = b << tpb;
+    for (uint32_t i = lane; i < b; i += kWave) removed += brem[i];
+    for (uint32_t i = lane; i < inb; i += kWave) removed += trem[first + i];
+    removed = wave_sum(removed);
+  }
+  if (COUNTED || wave != 0) load_items();
   __syncthreads();
   // the tile's kept count depends on the bitmap alone
   uint32_t keep[VPT], pre[VPT];
@@ -202,38 +217,31 @@ __global__ __launch_bounds__(WG) void rz_compact_vec(T* __restrict__ A, uint32_t
       ex += loc[q];
     }
     if (lane == kWave - 1) sh.off[E] = xs;
-    const uint32_t agg = __shfl(xs, kWave - 1, kWave);
-    // the count goes out before any item is read: the offsets of later
-    // tiles never wait for loads
-    if (lane == 0) st_relaxed(&status[t], pack_status(t == 0 ? kFlagIncl : kFlagAgg, epoch, agg));
-    load_items();
+    if constexpr (!COUNTED) {
+      const uint32_t agg = __shfl(xs, kWave - 1, kWave);
+      // the count goes out before any item is read: the offsets of later
+      // tiles never wait for loads
+      if (lane == 0) st_relaxed(&status[t], pack_status(t == 0 ? kFlagIncl : kFlagAgg, epoch, agg));
+      load_items();
+    }
   }
   wait_all_memory();  // every item load of this tile has returned
   __syncthreads();
   if (tid == 0) {
-    // this tile's input may now be overwritten: its flag, and its group's
-    // word once all 64 tiles of the group (fewer in the last) have loaded.
-    // The counters and the words live in separate arrays: words polled next
-    // to counters being incremented slowed the pass by half.
-    st_relaxed(&loaded[t], epoch);
-    const uint32_t g = t >> 6, members = min(64u, ntiles - (g << 6));
-    if (add_relaxed(&gcnt[g], 1u) == members - 1u) {
-      st_relaxed(&gcnt[g], 0u);
-      st_relaxed(&gdone[g], epoch);
-    }
+    st_relaxed(&loaded[t * kFlagStride], epoch);  // this tile's input may now be overwritten
   }
   // kept items in tile order into LDS (wave 0 stages its items, then looks back)
 #pragma unroll
   for (int j = 0; j < VPT; ++j) stage_kept<T, V>(sh.stage, x[j], keep[j], sh.off[j * NW + wave] + pre[j]);
   if (wave == 0) {
     const uint32_t agg = sh.off[E];
-    uint32_t excl = 0;
-    if (t != 0) {
+    uint32_t excl = COUNTED ? base - removed : 0u;
+    uint32_t pause = 1, spins = 0;
+    if (!COUNTED && t != 0) {
       // The nearest predecessor's word alone first (one load per poll, pause
       // doubling to 16 x 64 cycles), then windows of 64 back to an inclusive
       // prefix: polling whole windows from every waiting tile costs more
       // fabric bandwidth than the moves.
-      uint32_t pause = 1, spins = 0;
       while (true) {
         const uint64_t st = ld_relaxed(&status[t - 1]);
         if ((((uint32_t)(st >> 32) & 0x3fffffffu) == epoch && (st >> 62) != 0u) || ++spins > spin_cap(ctrl, 1u << 22)) break;
@@ -266,36 +274,22 @@ __global__ __launch_bounds__(WG) void rz_compact_vec(T* __restrict__ A, uint32_t
         jb -= kWave;
       }
       if (lane == 0) st_relaxed(&status[t], pack_status(kFlagIncl, epoch, excl + agg));
-      // The pass is in place: every tile whose input overlaps [excl, base)
-      // must have loaded before this tile writes.  Those are tiles [u, t):
-      // whole groups of 64 by their word, the two ends tile by tile.
-      const uint32_t u = excl / TILE;
-      const uint32_t g0 = (u + 63u) >> 6, g1 = t >> 6;
-      const bool groups = g0 < g1;
-      const uint32_t a_end = groups ? (g0 << 6) : t, b_beg = groups ? (g1 << 6) : t;
-      const uint32_t na = a_end - u, ng = groups ? g1 - g0 : 0u, nb = t - b_beg;
-      const uint32_t total = na + ng + nb;
+    }
+    if (t != 0) {
+      // The pass is in place: the tiles whose input overlaps this tile's output
+      // range [excl, excl + agg) must have loaded before it writes.  The range
+      // is no longer than a tile, so those are at most two.
+      const uint32_t u = excl / TILE + lane;
+      const bool wait = lane < 2 && u < t && u * TILE < excl + agg;
       spins = 0;
       pause = 1;
-      for (uint32_t c0 = 0; c0 < total;) {
-        const uint32_t c = c0 + lane;
-        bool ok = true;
-        if (c < na)
-          ok = ld_relaxed(&loaded[u + c]) == epoch;
-        else if (c < na + ng)
-          ok = ld_relaxed(&gdone[g0 + (c - na)]) == epoch;
-        else if (c < total)
-          ok = ld_relaxed(&loaded[b_beg + (c - na - ng)]) == epoch;
-        if (ballot(!ok)) {
-          if (++spins > spin_cap(ctrl, 1u << 22)) {
-            if (lane == 0) or_relaxed(&ctrl[kCtrlError], kErrLookbackTimeout);
-            break;
-          }
-          for (uint32_t i = 0; i < pause; ++i) __builtin_amdgcn_s_sleep(1);
-          if (pause < 16u) pause <<= 1;
-          continue;
+      while (ballot(wait && ld_relaxed(&loaded[u * kFlagStride]) != epoch)) {
+        if (++spins > spin_cap(ctrl, 1u << 22)) {
+          if (lane == 0) or_relaxed(&ctrl[kCtrlError], kErrLookbackTimeout);
+          break;
         }
-        c0 += kWave;
+        for (uint32_t i = 0; i < pause; ++i) __builtin_amdgcn_s_sleep(1);
+        if (pause < 16u) pause <<= 1;
       }
     }
     if (lane == 0) sh.excl = excl;
@@ -387,6 +381,7 @@ constexpr int kPartWG = 256, kPartIPT = 16;
 // ---------------------------------------------------------------------------
 constexpr uint32_t kPartMinBinLog = 15, kPartMaxBinLog = 20;  // 4 to 128 KiB LDS bitmaps
 constexpr uint32_t kPartMaxBins = 1024;
+constexpr uint32_t kMaxTilesPerBin = 256;  // 2^20 positions in tiles of 2^12
 constexpr int64_t kPartMaxWindow = (int64_t)1 << 29;  // entry lists of 2 GiB
 constexpr uint32_t kAppWG = 1024;
 // Removals per thread of a tile (dynamic LDS, 4 bytes a removal).  A bigger
@@ -515,12 +510,19 @@ __global__ __launch_bounds__(1024) void rz_part_append(const int32_t* __restrict
 __global__ __launch_bounds__(1024) void rz_part_bits(const uint32_t* __restrict__ ent, uint32_t* __restrict__ cur,
                                                       uint32_t* __restrict__ bdone, uint32_t m, uint32_t blog,
                                                       uint32_t G, uint32_t* __restrict__ bits,
-                                                      uint32_t* __restrict__ ctrl, uint64_t* __restrict__ stat) {
+                                                      uint32_t* __restrict__ ctrl, uint64_t* __restrict__ stat,
+                                                      uint32_t* __restrict__ trem, uint32_t* __restrict__ brem,
+                                                      uint32_t tlog) {
+  __shared__ uint32_t s_trem[kMaxTilesPerBin], s_brem;
   const uint32_t W = 1u << (blog - 5), cap = 1u << blog;
   extern __shared__ __align__(16) unsigned char dyn[];
   uint32_t* lb = (uint32_t*)dyn;
   const uint32_t bin = blockIdx.x / G, g = blockIdx.x % G, tid = threadIdx.x;
   for (uint32_t w = tid; w < W; w += 1024u) lb[w] = 0u;
+  if (trem) {
+    if (tid < kMaxTilesPerBin) s_trem[tid] = 0u;
+    if (tid == 0) s_brem = 0u;
+  }
   const uint32_t c = min(cur[bin], cap);
   __syncthreads();
   const uint32_t share = ((c + G - 1) / G + 3u) & ~3u;  // a multiple of 4: 16-byte vector loads
@@ -555,12 +557,35 @@ __global__ __launch_bounds__(1024) void rz_part_bits(const uint32_t* __restrict_
   }
   __syncthreads();
   const uint32_t nw = (uint32_t)(((uint64_t)m + 31u) >> 5);
-  for (uint32_t w = tid; w < W; w += 1024u) {
-    const uint32_t gw = (z0 >> 5) + w;
-    if (gw < nw && lb[w]) {
-      if (G == 1) bits[gw] = lb[w];
-      else or_relaxed(&bits[gw], lb[w]);
+  // each wave a contiguous 1/16 of the words, so that a tile's removals add up
+  // in registers (a reduction per 64 words took 10 us of 84 at 2^26 removals)
+  const uint32_t share_w = W / (1024u / kWave), w0 = (tid / kWave) * share_w;
+  uint32_t cnt = 0;
+  for (uint32_t i = 0; i < share_w; i += kWave) {
+    const uint32_t w = w0 + i + lane_id(), gw = (z0 >> 5) + w, v = lb[w];
+    if (gw < nw && v) {
+      if (G == 1) bits[gw] = v;
+      else or_relaxed(&bits[gw], v);
     }
+    if (trem) {
+      cnt += (uint32_t)__popc(v);
+      const uint32_t end = w0 + i + kWave;
+      if (i + kWave == share_w || (end & ((1u << (tlog - 5)) - 1u)) == 0u) {  // the end of a tile, or of the share
+        cnt = wave_sum(cnt);
+        if (lane_id() == 0 && cnt) atomicAdd(&s_trem[(end - 1u) >> (tlog - 5)], cnt);
+        cnt = 0;
+      }
+    }
+  }
+  if (trem) {
+    __syncthreads();
+    const uint32_t tiles = 1u << (blog - tlog);
+    if (tid < tiles) {
+      trem[bin * tiles + tid] = s_trem[tid];
+      if (s_trem[tid]) atomicAdd(&s_brem, s_trem[tid]);
+    }
+    __syncthreads();
+    if (tid == 0) brem[bin] = s_brem;
   }
   if (tid == 0) {
     // every workgroup of the bin has read its count: the last puts it back to zero
@@ -595,7 +620,7 @@ static rz_status append_launch(rz_ctx* ctx, const int32_t* R, int64_t k, uint32_
 }
 
 rz_status bucket_marks(rz_ctx* ctx, const int32_t* R, int64_t k, uint32_t base, int64_t m, uint32_t* bits,
-                       uint32_t* epoch_ctrl, uint64_t* stat, hipStream_t s) {
+                       uint32_t* epoch_ctrl, uint64_t* stat, hipStream_t s, TileCounts* tc) {
   if (!bucket_marks_fit(m) || k < 1 || k > INT32_MAX) return RZ_EINVAL;
   // the device gives a workgroup the big tile (and its bins' bitmaps) or the small one only
   const bool big = (size_t)4 * kAppWG * kAppIPTBig + 16384 <= (size_t)ctx->lds_max && k >= kAppBigK;
@@ -614,6 +639,18 @@ rz_status bucket_marks(rz_ctx* ctx, const int32_t* R, int64_t k, uint32_t base, 
     RZ_HIP(hipFuncSetAttribute((const void*)rz_part_bits, hipFuncAttributeMaxDynamicSharedMemorySize, (int)most));
     if (dev >= 0 && dev < 64) attr_mask.fetch_or(1ull << dev, std::memory_order_relaxed);
   }
+  uint32_t G = ((uint32_t)ctx->cu_count + nbins - 1) / nbins;  // about one workgroup per CU
+  G = G < 1 ? 1 : (G > 16 ? 16 : G);
+  uint32_t *trem = nullptr, *brem = nullptr;
+  if (tc) {
+    tc->made = G == 1 && blog >= tc->tlog;
+    if (tc->made) {  // a bin's one workgroup has its whole bitmap: the removals per tile are counted on the way
+      tc->tpb = blog - tc->tlog;
+      if ((st = ensure(ctx, ctx->ptrem, ((size_t)(nbins + 1) << tc->tpb) * 4 + kPartMaxBins * 4, s)) != RZ_OK) return st;
+      brem = tc->brem = (uint32_t*)ctx->ptrem.ptr;
+      trem = tc->trem = brem + kPartMaxBins;
+    }
+  }
   uint32_t* cur = (uint32_t*)ctx->pcur.ptr;
   uint32_t* ent = (uint32_t*)ctx->pent.ptr;
   const bool all = epoch_ctrl != nullptr;  // the partition: base 0, m = n
@@ -624,10 +661,8 @@ rz_status bucket_marks(rz_ctx* ctx, const int32_t* R, int64_t k, uint32_t base, 
   st = big ? RZ_APPEND(kAppIPTBig) : mid ? RZ_APPEND(kAppIPT) : RZ_APPEND(kAppIPTSmall);
 #undef RZ_APPEND
   if (st != RZ_OK) return st;
-  uint32_t G = ((uint32_t)ctx->cu_count + nbins - 1) / nbins;  // about one workgroup per CU
-  G = G < 1 ? 1 : (G > 16 ? 16 : G);
   hipLaunchKernelGGL(rz_part_bits, dim3(nbins * G), dim3(1024), lds_bits, s, (const uint32_t*)ent, cur, cur + nbins,
-                     (uint32_t)m, blog, G, bits, epoch_ctrl, stat);
+                     (uint32_t)m, blog, G, bits, epoch_ctrl, stat, trem, brem, tc ? tc->tlog : 0u);
   RZ_HIP(hipGetLastError());
   return RZ_OK;
 }
@@ -659,30 +694,31 @@ static rz_status partition_impl(rz_ctx* ctx, T* A, int64_t n, const int32_t* R, 
   rz_status st;
   if ((st = ensure(ctx, ctx->list_bits, (size_t)((n + 63) / 64) * 8, s)) != RZ_OK) return st;
   if ((st = ensure(ctx, ctx->status, (size_t)tiles * 8, s)) != RZ_OK) return st;
-  const int64_t groups = (tiles + 63) / 64;
-  if (vec) {
-    if ((st = ensure(ctx, ctx->ploaded, (size_t)tiles * 4, s)) != RZ_OK) return st;
-    if ((st = ensure(ctx, ctx->pgcnt, (size_t)groups * 4, s)) != RZ_OK) return st;
-    if ((st = ensure(ctx, ctx->pgdone, (size_t)groups * 4, s)) != RZ_OK) return st;
-  }
+  if (vec && (st = ensure(ctx, ctx->ploaded, (size_t)tiles * kFlagStride * 4, s)) != RZ_OK) return st;
   uint32_t* bits = (uint32_t*)ctx->list_bits.ptr;
   uint32_t* ctrl = (uint32_t*)ctx->ctrl.ptr;
   const int64_t gw = (k + 255) / 256;
   const dim3 g1((uint32_t)(gw < (int64_t)ctx->cu_count * 8 ? (gw > 0 ? gw : 1) : ctx->cu_count * 8));
   if ((st = prof_mark(ctx, flags, 0, s)) != RZ_OK) return st;
   const bool bucketed = k >= kPartBucketMinK && n >= kPartBucketMinN && bucket_marks_fit(n);
+  TileCounts tc;
+  tc.tlog = (uint32_t)log2_floor(TILE);
   if (bucketed) {
     // the bitmap is zero here: every call leaves the words it used clear
-    if ((st = bucket_marks(ctx, R, k, 0u, n, bits, ctrl, nullptr, s)) != RZ_OK) return st;
+    if ((st = bucket_marks(ctx, R, k, 0u, n, bits, ctrl, nullptr, s, vec ? &tc : nullptr)) != RZ_OK) return st;
   } else {
     hipLaunchKernelGGL(rz_mark_all, g1, dim3(256), 0, s, R, (uint32_t)k, (uint32_t)n, bits, ctrl);
   }
   RZ_HIP(hipGetLastError());
   if ((st = prof_mark(ctx, flags, 1, s)) != RZ_OK) return st;
-  if (vec)
-    hipLaunchKernelGGL((rz_compact_vec<T, kVecWG, VecShape<T>::VPT>), dim3((uint32_t)tiles), dim3(kVecWG), 0, s, A,
-                       (uint32_t)n, bits, (uint64_t*)ctx->status.ptr, (uint32_t*)ctx->ploaded.ptr,
-                       (uint32_t*)ctx->pgcnt.ptr, (uint32_t*)ctx->pgdone.ptr, (uint32_t)tiles, ctrl);
+  if (vec && tc.made)
+    hipLaunchKernelGGL((rz_compact_vec<T, kVecWG, VecShape<T>::VPT, true>), dim3((uint32_t)tiles), dim3(kVecWG), 0, s,
+                       A, (uint32_t)n, bits, (uint64_t*)nullptr, tc.trem, tc.brem, tc.tpb,
+                       (uint32_t*)ctx->ploaded.ptr, ctrl);
+  else if (vec)
+    hipLaunchKernelGGL((rz_compact_vec<T, kVecWG, VecShape<T>::VPT, false>), dim3((uint32_t)tiles), dim3(kVecWG), 0, s,
+                       A, (uint32_t)n, bits, (uint64_t*)ctx->status.ptr, (const uint32_t*)nullptr,
+                       (const uint32_t*)nullptr, 0u, (uint32_t*)ctx->ploaded.ptr, ctrl);
   else
     hipLaunchKernelGGL((rz_compact<T, kPartWG, kPartIPT>), dim3((uint32_t)tiles), dim3(kPartWG), 0, s, A,
                        (uint32_t)n, bits, (uint64_t*)ctx->status.ptr, ctrl);

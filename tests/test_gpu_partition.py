@@ -57,6 +57,26 @@ def test_partition_mark_tiles(ctx, oracle, n, k, pattern):
     _run(ctx, oracle, W.index_payload(n), W.removals(pattern, n, k, seed=k))
 
 
+@pytest.mark.parametrize("esz", [4, 8, 16])
+@pytest.mark.parametrize("n", [255 << 15, (255 << 15) + 1, (1 << 23) + 5, (1 << 24) - 1])
+def test_partition_counted_tiles(ctx, oracle, esz, n):
+    """List sizes on both sides of the point from which a mark bin has one
+    workgroup, which then counts the removals per tile (no look-back)."""
+    announce("counted tiles", esz, n)
+    A = torch.empty((n,) if esz == 4 else (n, esz // 4), dtype=torch.int32, device="cuda")
+    ctx.gen_payload(A, n)
+    for frac, pattern in ((3, "uniform"), (9, "clustered")):
+        k = n // frac
+        R = W.removals(pattern, n, k, seed=5, device="cuda")
+        keep = torch.ones(n, dtype=torch.bool, device="cuda")
+        keep[R.long()] = False
+        want = A[keep]
+        got = A.clone()
+        assert ctx.partition(got, R) == n - k
+        assert torch.equal(got[: n - k], want)
+    assert ctx.check_errors() == 0
+
+
 def test_partition_unaligned_list(ctx, oracle):
     """A list that starts one item into a buffer is not 16-byte aligned: the
     scalar tile kernel handles it."""

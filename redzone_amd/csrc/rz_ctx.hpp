@@ -105,9 +105,10 @@ struct rz_ctx {
   rz::DeviceBuffer dense_fine;   // dense form: fine-bin head writes (fixed capacity per bin)
   rz::DeviceBuffer dense_src;    // dense form: source orphan values by rank
   rz::DeviceBuffer gstatus;    // preserve-list gather: the gathered items before they are copied back
-  rz::DeviceBuffer dispatch;   // network parameters, one list descriptor, its features and the choice
+  rz::DeviceBuffer dispatch;   // network parameters
   bool dispatch_ready = false; // parameters installed (else the k < n/2 rule)
-  uint8_t* auto_host = nullptr;  // pinned staging of the descriptor and the choice
+  uint8_t* auto_host = nullptr;  // pinned staging of rz_remove_auto's choice
+  uint8_t* auto_host_dev = nullptr;  // its device address
   rz::DeviceBuffer choose;       // rz_dispatch_choose: descriptors, features, choices
   uint8_t* choose_host = nullptr;  // its pinned staging: descriptors, then choices
   uint8_t* choose_host_dev = nullptr;  // the same staging's device address

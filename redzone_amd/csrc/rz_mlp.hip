@@ -26,58 +26,83 @@ static_assert(NP == RZ_MLP_PARAMS, "parameter count");
 // features: one wave per list, a 256-entry strided sample of the removal list
 // ---------------------------------------------------------------------------
 // The features of list d, by one 64-lane workgroup (s_x: 256 floats of LDS);
-// lane 0 writes them to o[0..F).
+// lanes 0 to F - 1 write them to o[0..F).  All loads of the sample are in
+// flight together: one after another, with a 64-bit division each, they were
+// most of the 5.6 us a list took.
 __device__ __forceinline__ void list_features(const rz_list_desc& d, float* s_x, float* o) {
   const int lane = threadIdx.x;
   const double n = (double)(d.n > 0 ? d.n : 1);
   const int64_t k = d.k;
   const int64_t sz = d.n - d.k;
   const int m = k < 256 ? (int)k : 256;  // sample size
-  float sum = 0.f, sum2 = 0.f, tail = 0.f;
-  for (int j = lane; j < m; j += 64) {
-    const int64_t i = (int64_t)j * k / m;
-    const int64_t r = d.removals[i];
-    const float x = (float)((double)r / n);
-    s_x[j] = x;
-    sum += x;
-    sum2 += x * x;
-    tail += (r >= sz) ? 1.f : 0.f;
-  }
   // adjacent pairs (R[i], R[i+1]) at 128 strided positions: runs of the removal list
-  float consec = 0.f, near = 0.f;
   const int mp = k < 2 ? 0 : (k - 1 < 128 ? (int)(k - 1) : 128);
-  for (int j = lane; j < mp; j += 64) {
-    const int64_t i = (int64_t)j * (k - 1) / mp;
-    const int64_t a = d.removals[i], b = d.removals[i + 1];
-    consec += (b == a + 1) ? 1.f : 0.f;
-    near += (b - a < 64 && a - b < 64) ? 1.f : 0.f;
+  int32_t r[4], pa[2], pb[2];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const int j = lane + 64 * q;  // sample j is at j k / m: m is k or 256
+    r[q] = j < m ? d.removals[m < 256 ? (int64_t)j : ((int64_t)j * k) >> 8] : 0;
+  }
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    const int j = lane + 64 * q;  // pair j is at j (k - 1) / mp
+    const int64_t i = mp < 128 ? (int64_t)j : ((int64_t)j * (k - 1)) >> 7;
+    pa[q] = j < mp ? d.removals[i] : 0;
+    pb[q] = j < mp ? d.removals[i + 1] : 0;
+  }
+  float sum = 0.f, sum2 = 0.f, tail = 0.f;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    if (lane + 64 * q < m) {
+      const float x = (float)((double)r[q] / n);
+      s_x[lane + 64 * q] = x;
+      sum += x;
+      sum2 += x * x;
+      tail += (r[q] >= sz) ? 1.f : 0.f;
+    }
+  }
+  float consec = 0.f, near = 0.f;
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    if (lane + 64 * q < mp) {
+      const int64_t a = pa[q], b = pb[q];
+      consec += (b == a + 1) ? 1.f : 0.f;
+      near += (b - a < 64 && a - b < 64) ? 1.f : 0.f;
+    }
   }
   __syncthreads();
   float up = 0.f;
-  for (int j = lane; j + 1 < m; j += 64) up += s_x[j + 1] > s_x[j] ? 1.f : 0.f;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const int j = lane + 64 * q;
+    if (j + 1 < m) up += s_x[j + 1] > s_x[j] ? 1.f : 0.f;
+  }
   sum = wave_sum(sum);
   sum2 = wave_sum(sum2);
   tail = wave_sum(tail);
   consec = wave_sum(consec);
   near = wave_sum(near);
   up = wave_sum(up);
-  if (lane == 0) {
+  if (lane < F) {
     const float fm = m > 0 ? (float)m : 1.f;
     const float mean = sum / fm;
     const float var = fmaxf(sum2 / fm - mean * mean, 0.f);
     const double frac = (double)k / n;
-    o[0] = (float)(log2(n) / 32.0);
-    o[1] = k > 0 ? (float)(log2((double)k) / 32.0) : 0.f;
-    o[2] = (float)frac;
-    o[3] = k > 0 ? (float)fmax(log2(frac) / 20.0, -1.0) : -1.f;
-    o[4] = (float)d.elem_bytes / 16.f;
-    o[5] = m > 0 ? tail / fm : 0.f;
-    o[6] = mean;
-    o[7] = sqrtf(var);
-    o[8] = mp > 0 ? consec / (float)mp : 0.f;
-    o[9] = mp > 0 ? near / (float)mp : 0.f;
-    o[10] = m > 1 ? up / (float)(m - 1) : 0.f;
-    o[11] = 1.f;
+    // one logarithm, of another argument per lane
+    const double lg = log2(lane == 0 ? n : k <= 0 ? 1.0 : lane == 1 ? (double)k : frac);
+    float f = 1.f;
+    if (lane == 0) f = (float)(lg / 32.0);
+    if (lane == 1) f = k > 0 ? (float)(lg / 32.0) : 0.f;
+    if (lane == 2) f = (float)frac;
+    if (lane == 3) f = k > 0 ? (float)fmax(lg / 20.0, -1.0) : -1.f;
+    if (lane == 4) f = (float)d.elem_bytes / 16.f;
+    if (lane == 5) f = m > 0 ? tail / fm : 0.f;
+    if (lane == 6) f = mean;
+    if (lane == 7) f = sqrtf(var);
+    if (lane == 8) f = mp > 0 ? consec / (float)mp : 0.f;
+    if (lane == 9) f = mp > 0 ? near / (float)mp : 0.f;
+    if (lane == 10) f = m > 1 ? up / (float)(m - 1) : 0.f;
+    o[lane] = f;
   }
 }
 
@@ -92,29 +117,56 @@ __global__ __launch_bounds__(64) void rz_features_kernel(const rz_list_desc* __r
 // ---------------------------------------------------------------------------
 // MLP
 // ---------------------------------------------------------------------------
+// The parameters in LDS, each row of W in a stride of its own odd length (32
+// lanes reading a column hit 32 banks).
+constexpr int S1 = F + 1, S2 = H + 1;
+struct NetShared {
+  float w1[H * S1], w2[H * S2], w3[H * S2], w4[C * S2], b[3 * H + C];
+};
+constexpr int kNetLoads = (NP + 63) / 64;
+// Parameter i of the library's layout has its place in the shared copy.
+__device__ __forceinline__ void net_store(NetShared& s, int i, float v) {
+  if (i < OB1) s.w1[i / F * S1 + i % F] = v;
+  else if (i < OW2) s.b[i - OB1] = v;
+  else if (i < OB2) s.w2[(i - OW2) / H * S2 + (i - OW2) % H] = v;
+  else if (i < OW3) s.b[H + i - OB2] = v;
+  else if (i < OB3) s.w3[(i - OW3) / H * S2 + (i - OW3) % H] = v;
+  else if (i < OW4) s.b[2 * H + i - OB3] = v;
+  else if (i < OB4) s.w4[(i - OW4) / H * S2 + (i - OW4) % H] = v;
+  else s.b[3 * H + i - OB4] = v;
+}
+
 // One layer by one wave: lane o's pre-activation b[o] + sum_i W[o][i] in_i,
 // in_i broadcast from lane i, summed in ascending i.
-__device__ __forceinline__ float layer_wave(const float* __restrict__ W, const float* __restrict__ b, float in,
-                                            int nin, int o) {
-  float acc = b[o];
-  for (int i = 0; i < nin; ++i) acc = fmaf(W[o * nin + i], __shfl(in, i), acc);
+template <int NIN>
+__device__ __forceinline__ float layer_wave(const float* w, float bias, float in) {
+  float acc = bias;
+#pragma unroll
+  for (int i = 0; i < NIN; ++i)
+    acc = fmaf(w[i], __int_as_float(__builtin_amdgcn_readlane(__float_as_int(in), i)), acc);
   return acc;
 }
 
 static_assert((H & (H - 1)) == 0 && (C & (C - 1)) == 0 && H <= 64 && F <= 64, "one unit per lane");
 
-// The network on one row by one 64-lane wave: lane f < F holds feature f on
-// entry; y_out (may be null) gets the C outputs.  Returns the argmin (every
-// lane), ties to the lower index as in rz_mlp_forward_kernel's contract.
-__device__ __forceinline__ int forward_wave(const float* __restrict__ P, float x, float* __restrict__ y_out) {
+// The network on one row by one 64-lane workgroup: lane f < F holds feature f
+// on entry, p the parameters as loaded (parameter q * 64 + lane in p[q]);
+// y_out (may be null) gets the C outputs.  Returns the argmin (every lane),
+// ties to the lower index.
+__device__ __forceinline__ int forward_wave(const float (&p)[kNetLoads], NetShared& s, float x,
+                                            float* __restrict__ y_out) {
   const int lane = threadIdx.x & 63, o = lane & (H - 1), c = lane & (C - 1);
-  float a = layer_wave(P + OW1, P + OB1, x, F, o);
+#pragma unroll
+  for (int q = 0; q < kNetLoads; ++q)
+    if (q * 64 + lane < NP) net_store(s, q * 64 + lane, p[q]);
+  __syncthreads();
+  float a = layer_wave<F>(&s.w1[o * S1], s.b[o], x);
   float h = a > 0.f ? a : 0.f;
-  a = layer_wave(P + OW2, P + OB2, h, H, o);
+  a = layer_wave<H>(&s.w2[o * S2], s.b[H + o], h);
   h = a > 0.f ? a : 0.f;
-  a = layer_wave(P + OW3, P + OB3, h, H, o);
+  a = layer_wave<H>(&s.w3[o * S2], s.b[2 * H + o], h);
   h = a > 0.f ? a : 0.f;
-  const float y = layer_wave(P + OW4, P + OB4, h, H, c);
+  const float y = layer_wave<H>(&s.w4[c * S2], s.b[3 * H + c], h);
   if (y_out && lane < C) y_out[lane] = y;
   int best = 0;
   float yb = __shfl(y, 0);
@@ -127,39 +179,60 @@ __device__ __forceinline__ int forward_wave(const float* __restrict__ P, float x
   }
   return best;
 }
+__device__ __forceinline__ void net_load(const float* __restrict__ params, float (&p)[kNetLoads]) {
+#pragma unroll
+  for (int q = 0; q < kNetLoads; ++q) p[q] = params[min(q * 64 + (int)(threadIdx.x & 63), NP - 1)];
+}
 
 // One 64-lane workgroup per row.
 __global__ __launch_bounds__(64) void rz_mlp_forward_kernel(const float* __restrict__ params,
                                                              const float* __restrict__ X, int32_t B,
                                                              float* __restrict__ Y, int32_t* __restrict__ choice) {
+  __shared__ NetShared sh;
   const int b = blockIdx.x;
   if (b >= B) return;
   const int lane = threadIdx.x;
+  float p[kNetLoads];
+  net_load(params, p);
   const float x = lane < F ? X[(size_t)b * F + lane] : 0.f;
-  const int best = forward_wave(params, x, Y ? Y + (size_t)b * C : nullptr);
+  const int best = forward_wave(p, sh, x, Y ? Y + (size_t)b * C : nullptr);
   if (choice && lane == 0) choice[b] = best;
 }
 
-// rz_dispatch_choose for up to kChooseArgMax lists: the descriptors come as a
-// kernel argument (no upload), one 64-lane workgroup per list computes its
-// features and the forward pass, and lane 0 stores the choice straight into
-// the caller-visible pinned staging with a system-scope store.
+// rz_dispatch_choose for up to kChooseArgMax lists, and rz_remove_auto: the
+// descriptors come as a kernel argument (no upload), one 64-lane workgroup per
+// list computes its features and the forward pass, the parameters' loads
+// going out first, and lane 0 stores the choice straight into the
+// caller-visible pinned staging with a system-scope store.
 constexpr int kChooseArgMax = 48;
 struct ChooseArgs {
   rz_list_desc d[kChooseArgMax];
 };
 
+__device__ __forceinline__ void choose_one(const rz_list_desc& d, const float* __restrict__ params,
+                                           int32_t* __restrict__ h_choice) {
+  __shared__ float s_x[256];
+  __shared__ float s_f[F];
+  __shared__ NetShared sh;
+  float p[kNetLoads];
+  net_load(params, p);
+  list_features(d, s_x, s_f);
+  __syncthreads();
+  const float x = threadIdx.x < F ? s_f[threadIdx.x] : 0.f;
+  const int best = forward_wave(p, sh, x, nullptr);
+  if (threadIdx.x == 0) __hip_atomic_store(h_choice, best, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 __global__ __launch_bounds__(64) void rz_choose_kernel(ChooseArgs a, int32_t nlists, const float* __restrict__ params,
                                                         int32_t* __restrict__ h_choice) {
   const int li = blockIdx.x;
   if (li >= nlists) return;
-  __shared__ float s_x[256];
-  __shared__ float s_f[F];
-  list_features(a.d[li], s_x, s_f);
-  __syncthreads();
-  const float x = threadIdx.x < F ? s_f[threadIdx.x] : 0.f;
-  const int best = forward_wave(params, x, nullptr);
-  if (threadIdx.x == 0) __hip_atomic_store(&h_choice[li], best, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  choose_one(a.d[li], params, h_choice + li);
+}
+
+__global__ __launch_bounds__(64) void rz_choose_one_kernel(rz_list_desc d, const float* __restrict__ params,
+                                                            int32_t* __restrict__ h_choice) {
+  choose_one(d, params, h_choice);
 }
 
 // ---------------------------------------------------------------------------
@@ -427,13 +500,6 @@ rz_status rz_dispatch_method_config(int32_t method, uint32_t elem_bytes, rz_tile
   return RZ_EINVAL;
 }
 
-// dispatch buffer: [params NP floats | pad to 256 B | descriptor | features | choice]
-static constexpr size_t kDispParams = ((size_t)NP * 4 + 255) & ~(size_t)255;
-static constexpr size_t kDispDesc = kDispParams;
-static constexpr size_t kDispFeat = kDispDesc + 256;
-static constexpr size_t kDispChoice = kDispFeat + 256;
-static constexpr size_t kDispBytes = kDispChoice + 256;
-
 rz_status rz_dispatch_set_params(rz_ctx* ctx, const float* h_params) {
   if (!ctx) return RZ_EINVAL;
   std::lock_guard<std::mutex> lock(ctx->mu);
@@ -443,7 +509,7 @@ rz_status rz_dispatch_set_params(rz_ctx* ctx, const float* h_params) {
   rz_status st = RZ_OK;
   if (!h_params) {
     ctx->dispatch_ready = false;
-  } else if ((st = ensure(ctx, ctx->dispatch, kDispBytes, nullptr)) == RZ_OK) {
+  } else if ((st = ensure(ctx, ctx->dispatch, (size_t)NP * 4, nullptr)) == RZ_OK) {
     if (hipMemcpy(ctx->dispatch.ptr, h_params, (size_t)NP * 4, hipMemcpyHostToDevice) != hipSuccess) st = RZ_EHIP;
     ctx->dispatch_ready = st == RZ_OK;
   }
@@ -463,25 +529,24 @@ static rz_status auto_choose(rz_ctx* ctx, void* d_data, int64_t n, uint32_t esz,
   (void)hipGetDevice(&prev);
   if (prev != ctx->device) (void)hipSetDevice(ctx->device);
   rz_status st = RZ_OK;
-  if (!ctx->auto_host && hipHostMalloc((void**)&ctx->auto_host, 256, hipHostMallocDefault) != hipSuccess) {
+  // mapped and coherent: the choice kernel stores into it directly
+  if (!ctx->auto_host &&
+      (hipHostMalloc((void**)&ctx->auto_host, 256, hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess ||
+       hipHostGetDevicePointer((void**)&ctx->auto_host_dev, ctx->auto_host, 0) != hipSuccess)) {
+    if (ctx->auto_host) (void)hipHostFree(ctx->auto_host);
     ctx->auto_host = nullptr;
     st = RZ_ENOMEM;
   }
   if (st == RZ_OK) {
-    char* base = (char*)ctx->dispatch.ptr;
-    rz_list_desc* hd = (rz_list_desc*)ctx->auto_host;
-    *hd = rz_list_desc{d_data, d_removals, n, k, esz, 0u};
-    int32_t* hc = (int32_t*)(ctx->auto_host + 128);
+    // One launch (5.8 us): a descriptor upload, the two kernels and a copy back
+    // took a call of 42 us 7 us more.
+    volatile int32_t* hc = (volatile int32_t*)ctx->auto_host;
     *hc = -1;
-    if (hipMemcpyAsync(base + kDispDesc, hd, sizeof(rz_list_desc), hipMemcpyHostToDevice, s) != hipSuccess) st = RZ_EHIP;
-    if (st == RZ_OK)
-      st = rz_features(ctx, (const rz_list_desc*)(base + kDispDesc), 1, (float*)(base + kDispFeat), s);
-    if (st == RZ_OK)
-      st = rz_mlp_forward(ctx, (const float*)base, (const float*)(base + kDispFeat), 1, nullptr,
-                          (int32_t*)(base + kDispChoice), s);
-    if (st == RZ_OK && hipMemcpyAsync(hc, base + kDispChoice, 4, hipMemcpyDeviceToHost, s) != hipSuccess) st = RZ_EHIP;
-    if (st == RZ_OK && hipStreamSynchronize(s) != hipSuccess) st = RZ_EHIP;
-    if (st == RZ_OK) *method = (*hc >= 0 && *hc < RZ_MLP_OUTPUTS) ? *hc : (2 * k < n ? 0 : 3);
+    hipLaunchKernelGGL(rz_choose_one_kernel, dim3(1), dim3(64), 0, s, rz_list_desc{d_data, d_removals, n, k, esz, 0u},
+                       (const float*)ctx->dispatch.ptr, (int32_t*)ctx->auto_host_dev);
+    if (hipGetLastError() != hipSuccess || hipStreamSynchronize(s) != hipSuccess) st = RZ_EHIP;
+    const int32_t c = *hc;
+    if (st == RZ_OK) *method = (c >= 0 && c < RZ_MLP_OUTPUTS) ? c : (2 * k < n ? 0 : 3);
   }
   if (prev >= 0 && prev != ctx->device) (void)hipSetDevice(prev);
   return st;

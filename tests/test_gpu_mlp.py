@@ -58,6 +58,22 @@ def test_forward_and_grad_match_oracle(ctx):
     assert np.array_equal(g, g2.cpu().numpy())
 
 
+def test_features_at_sample_edges(ctx):
+    """Removal counts around the sample sizes (256 entries, 128 pairs), where
+    the strided positions change from every entry to every k-th."""
+    lists, host = [], []
+    for k in (1, 2, 64, 127, 128, 129, 130, 255, 256, 257, 300, 1000, 65537):
+        n = 3 * k + 5
+        R = W.clustered_removals(n, k, seed=k)
+        lists.append((W.payload(4, n, seed=k).cuda(), R.cuda()))
+        host.append((R.numpy(), n, 4))
+    announce("feature edges")
+    F = D.Dispatcher(ctx).features(lists).cpu().numpy()
+    for i, (R, n, esz) in enumerate(host):
+        want = MR.features(R, n, esz)
+        assert np.allclose(F[i], want, atol=2e-6, rtol=1e-5), (len(R), F[i], want)
+
+
 @pytest.mark.parametrize("batch", [1, 31, 32, 33, 300, 32 * 256 - 1, 32 * 256 + 1, 32 * 512 + 45])
 def test_grad_at_tile_edges(ctx, batch):
     """Batches around the gradient kernel's 32-sample tiles and around the

@@ -28,6 +28,8 @@ __all__ = ["Context", "Batch", "ListDescs", "remove", "partition", "TileConfig",
 
 def elem_bytes_of(data):
     """Bytes per item of a tensor of shape (n,) or (n, w): the whole row is one item."""
+    if data.dim() == 1:
+        return data.element_size()
     per_row = 1
     for d in data.shape[1:]:
         per_row *= d
@@ -35,20 +37,43 @@ def elem_bytes_of(data):
 
 
 def _stream_handle(stream, device):
+    """Address of the stream; without one, of the calling thread's current stream."""
+    return _current_stream(device) if stream is None else stream.cuda_stream
+
+
+# A call that changes nothing (k = 0) used to cost 3.6 us of host time, half of
+# what a small removal takes; without Stream, device and c_void_p objects it costs
+# 1.7 us.  torch is imported by the first call that needs it, and only then bound.
+def _current_stream(device):
     import torch
 
-    if stream is None:
-        stream = torch.cuda.current_stream(device)
-    return ctypes.c_void_p(stream.cuda_stream)
+    global _current_stream
+    address = torch.cuda.current_stream(device).cuda_stream  # initialises torch's device state
+    _current_stream = getattr(torch._C, "_cuda_getCurrentRawStream",
+                              lambda d: torch.cuda.current_stream(d).cuda_stream)
+    return address
+
+
+_int32 = None
+
+
+def _check_int32(t, name):
+    import torch
+
+    global _int32
+    _int32 = torch.int32
+    if t.dtype != _int32:
+        raise ValueError(f"{name} must be int32")
 
 
 def _check_tensor(t, name, device):
+    if t.is_cuda and t.get_device() == device and t.is_contiguous():
+        return
     if not t.is_cuda:
         raise ValueError(f"{name} must be a device tensor")
     if t.device.index != device:
         raise ValueError(f"{name} is on {t.device}, the context is on cuda:{device}")
-    if not t.is_contiguous():
-        raise ValueError(f"{name} must be contiguous")
+    raise ValueError(f"{name} must be contiguous")
 
 
 class Context:
@@ -106,13 +131,12 @@ class Context:
     def _args(self, data, removals, n, k):
         _check_tensor(data, "data", self.device)
         _check_tensor(removals, "removals", self.device)
-        import torch
-
-        if removals.dtype != torch.int32:
-            raise ValueError("removals must be int32")
-        n = data.shape[0] if n is None else int(n)
-        k = removals.shape[0] if k is None else int(k)
-        if n > data.shape[0] or k > removals.shape[0]:
+        if removals.dtype is not _int32:
+            _check_int32(removals, "removals")
+        n_max, k_max = data.shape[0], removals.shape[0]
+        n = n_max if n is None else int(n)
+        k = k_max if k is None else int(k)
+        if n > n_max or k > k_max:
             raise ValueError("n / k exceed the tensors")
         return n, k, elem_bytes_of(data)
 
@@ -124,11 +148,11 @@ class Context:
         n, k, esz = self._args(data, removals, n, k)
         s = _stream_handle(stream, self.device)
         if config is None:
-            self._call("rz_remove", self._h, ctypes.c_void_p(data.data_ptr()), n, esz,
-                       ctypes.c_void_p(removals.data_ptr()), k, flags, s)
+            self._call("rz_remove", self._h, data.data_ptr(), n, esz,
+                       removals.data_ptr(), k, flags, s)
         else:
-            self._call("rz_remove_config", self._h, ctypes.c_void_p(data.data_ptr()), n, esz,
-                       ctypes.c_void_p(removals.data_ptr()), k, flags, ctypes.byref(config), s)
+            self._call("rz_remove_config", self._h, data.data_ptr(), n, esz,
+                       removals.data_ptr(), k, flags, ctypes.byref(config), s)
         return n - k
 
     def remove_sized(self, data, removals, d_n, d_k, n_cap=None, k_cap=None, flags=0, stream=None):
@@ -145,9 +169,9 @@ class Context:
             _check_tensor(t, name, self.device)
             if t.dtype != torch.int32 or t.numel() < 1:
                 raise ValueError(f"{name} must be an int32 tensor of at least one element")
-        self._call("rz_remove_sized", self._h, ctypes.c_void_p(data.data_ptr()), n_cap, esz,
-                   ctypes.c_void_p(removals.data_ptr()), k_cap, ctypes.c_void_p(d_n.data_ptr()),
-                   ctypes.c_void_p(d_k.data_ptr()), flags, _stream_handle(stream, self.device))
+        self._call("rz_remove_sized", self._h, data.data_ptr(), n_cap, esz,
+                   removals.data_ptr(), k_cap, d_n.data_ptr(),
+                   d_k.data_ptr(), flags, _stream_handle(stream, self.device))
 
     def add_remove(self, data, n, additions, removals, k=None, flags=0, stream=None):
         """Appends `additions` after data[:n] (data must hold n + g items), then
@@ -156,17 +180,15 @@ class Context:
         _check_tensor(data, "data", self.device)
         _check_tensor(additions, "additions", self.device)
         _check_tensor(removals, "removals", self.device)
-        import torch
-
-        if removals.dtype != torch.int32:
-            raise ValueError("removals must be int32")
+        if removals.dtype is not _int32:
+            _check_int32(removals, "removals")
         esz = elem_bytes_of(data)
         if elem_bytes_of(additions) != esz:
             raise ValueError("additions must have the list's item size")
         g = additions.shape[0]
         k = removals.shape[0] if k is None else int(k)
-        self._call("rz_add_remove", self._h, ctypes.c_void_p(data.data_ptr()), int(n), data.shape[0], esz,
-                   ctypes.c_void_p(additions.data_ptr()), g, ctypes.c_void_p(removals.data_ptr()), k, flags,
+        self._call("rz_add_remove", self._h, data.data_ptr(), int(n), data.shape[0], esz,
+                   additions.data_ptr(), g, removals.data_ptr(), k, flags,
                    _stream_handle(stream, self.device))
         return int(n) + g - k
 
@@ -174,8 +196,8 @@ class Context:
         """In place: data[i] = data[keep[i]] for i < p (keep strictly ascending,
         int32).  Returns p."""
         n, p, esz = self._args(data, keep, n, p)
-        self._call("rz_gather_preserve", self._h, ctypes.c_void_p(data.data_ptr()), n, esz,
-                   ctypes.c_void_p(keep.data_ptr()), p, flags, _stream_handle(stream, self.device))
+        self._call("rz_gather_preserve", self._h, data.data_ptr(), n, esz,
+                   keep.data_ptr(), p, flags, _stream_handle(stream, self.device))
         return p
 
     def mark_removals(self, removals, n, tail_bits, k=None, stream=None):
@@ -186,8 +208,8 @@ class Context:
         k = removals.shape[0] if k is None else int(k)
         if tail_bits.numel() * tail_bits.element_size() < 4 * ((k + 31) // 32):
             raise ValueError("tail_bits holds fewer than ceil(k/32) words")
-        self._call("rz_mark_removals", self._h, ctypes.c_void_p(removals.data_ptr()), int(n), k,
-                   ctypes.c_void_p(tail_bits.data_ptr()), _stream_handle(stream, self.device))
+        self._call("rz_mark_removals", self._h, removals.data_ptr(), int(n), k,
+                   tail_bits.data_ptr(), _stream_handle(stream, self.device))
 
     def remove_premarked(self, data, removals, tail_bits, n=None, k=None, flags=0, config=None, stream=None):
         """remove() with the tail marks already in tail_bits (see mark_removals and
@@ -197,8 +219,8 @@ class Context:
         if tail_bits.numel() * tail_bits.element_size() < 4 * ((k + 31) // 32):
             raise ValueError("tail_bits holds fewer than ceil(k/32) words")
         cfg = ctypes.byref(config) if config is not None else None
-        self._call("rz_remove_premarked", self._h, ctypes.c_void_p(data.data_ptr()), n, esz,
-                   ctypes.c_void_p(removals.data_ptr()), k, ctypes.c_void_p(tail_bits.data_ptr()), flags, cfg,
+        self._call("rz_remove_premarked", self._h, data.data_ptr(), n, esz,
+                   removals.data_ptr(), k, tail_bits.data_ptr(), flags, cfg,
                    _stream_handle(stream, self.device))
         return n - k
 
@@ -221,16 +243,16 @@ class Context:
         back, so it synchronises the stream."""
         n, k, esz = self._args(data, removals, n, k)
         m = ctypes.c_int32(-1)
-        self._call("rz_remove_auto", self._h, ctypes.c_void_p(data.data_ptr()), n, esz,
-                   ctypes.c_void_p(removals.data_ptr()), k, flags, ctypes.byref(m), _stream_handle(stream, self.device))
+        self._call("rz_remove_auto", self._h, data.data_ptr(), n, esz,
+                   removals.data_ptr(), k, flags, ctypes.byref(m), _stream_handle(stream, self.device))
         return n - k, m.value
 
     def partition(self, data, removals, n=None, k=None, flags=0, stream=None):
         """O(n) stable in-place partition; survivors keep their order.  Returns n - k."""
         n, k, esz = self._args(data, removals, n, k)
         s = _stream_handle(stream, self.device)
-        self._call("rz_partition_on", self._h, ctypes.c_void_p(data.data_ptr()), n, esz,
-                   ctypes.c_void_p(removals.data_ptr()), k, flags, s)
+        self._call("rz_partition_on", self._h, data.data_ptr(), n, esz,
+                   removals.data_ptr(), k, flags, s)
         return n - k
 
     def last_profile(self):
@@ -275,12 +297,12 @@ class Context:
     def gen_uniform_removals(self, removals, n, seed, stream=None):
         """Fills the int32 device tensor `removals` (k entries) with k distinct indices of [0, n)."""
         _check_tensor(removals, "removals", self.device)
-        self._call("rz_gen_uniform_removals", self._h, ctypes.c_void_p(removals.data_ptr()), int(n),
+        self._call("rz_gen_uniform_removals", self._h, removals.data_ptr(), int(n),
                    removals.shape[0], int(seed), _stream_handle(stream, self.device))
 
     def gen_payload(self, data, seed, stream=None):
         _check_tensor(data, "data", self.device)
-        self._call("rz_gen_payload", self._h, ctypes.c_void_p(data.data_ptr()), data.shape[0], elem_bytes_of(data),
+        self._call("rz_gen_payload", self._h, data.data_ptr(), data.shape[0], elem_bytes_of(data),
                    int(seed), _stream_handle(stream, self.device))
 
     # ---- autotuner ---------------------------------------------------------

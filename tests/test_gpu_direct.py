@@ -144,3 +144,41 @@ def test_gather_tiles(ctx, esz, p):
         assert ctx.gather_preserve(A, P.to(torch.int32).cuda(), n=n) == p
         assert torch.equal(A[:p], want)
     assert ctx.check_errors() == 0
+
+
+@pytest.mark.parametrize("given", [False, True])
+def test_calls_run_on_the_stream_they_name(ctx, given):
+    """The caller's current stream, or the stream it passes, on every call (not
+    only the first): the list is filled on that stream right before."""
+    n, k = 60000, 700
+    s = torch.cuda.Stream()
+    R = torch.arange(5, 5 + k, dtype=torch.int32, device="cuda")
+    new = torch.arange(n, dtype=torch.int32, device="cuda")
+    torch.cuda.synchronize()
+    for _ in range(3):
+        data = torch.empty_like(new)
+        torch.cuda.synchronize()
+        with torch.cuda.stream(s):
+            data.copy_(new)
+            if not given:
+                assert ctx.remove(data, R, flags=rz.RZ_PRESERVE_REMOVALS) == n - k
+        if given:
+            assert ctx.remove(data, R, flags=rz.RZ_PRESERVE_REMOVALS, stream=s) == n - k
+        s.synchronize()
+        got = data[: n - k].cpu()
+        assert torch.equal(got.sort().values, torch.cat([new[:5], new[5 + k:]]).cpu())
+
+
+def test_tensors_that_are_refused(ctx):
+    data = torch.zeros(64, dtype=torch.int32, device="cuda")
+    R = torch.zeros(4, dtype=torch.int32, device="cuda")
+    for bad in ((data.cpu(), R), (data, R.cpu()), (data[::2], R), (data, R.long()), (data, R[::2]), (data, R.float())):
+        with pytest.raises(ValueError):
+            ctx.remove(*bad)
+    with pytest.raises(ValueError):
+        ctx.remove(data, R, k=5)
+    with pytest.raises(ValueError):
+        ctx.remove(data, R, n=65)
+    with pytest.raises(ValueError):
+        ctx.add_remove(data, 60, R, R.long())
+    torch.cuda.synchronize()

@@ -81,7 +81,8 @@ typedef struct rz_tile_config {
                           items: a list of several slices of at most 8,192 pairs each pairs its orphans
                           inside the move items, through look-back and exchange words, or 5 = as 2, with
                           the tail marks of lists of 2^19 to 2^22 removals grouped in buckets of 2^15
-                          tail positions and each bucket's bitmap words written whole),
+                          tail positions and each bucket's bitmap words written whole; shorter lists of
+                          several slices mark their tails through an LDS bitmap in 2 and 5),
                           4 = two kernels (mark, then move with in-kernel orphan pairing; slices longer than
                               the workgroup LDS allows run as variant 0),
                           5 = dense form: head writes grouped by destination bin, then one scatter per bin

@@ -16,6 +16,9 @@
 //                 rz_fused_dev.hpp).  The list's MARK j also zeroes the
 //                 slice's look-back word and its share of the list's exchange
 //                 words, so no list state survives from an earlier launch.
+// A list of several slices whose tail bitmap fits LDS (fewer than 2^19 removals
+// at 512 threads) has fewer MARK items, of 8,192 removals each: they gather their
+// marks in LDS and merge whole words (lds_marks).
 // With batch variant 5, a list of 2^19 to 2^22 removals marks its tail in
 // buckets instead of one atomic per tail removal:
 //   MARK j        groups the tail removals of removals [jL, (j+1)L) by bucket
@@ -45,8 +48,10 @@
 // Within a queue the lists follow each other (MARK items of a list, then its
 // MOVE items, then its PAIR items, with the next list's MARK items pulled
 // ahead of the MOVE items and the PAIR items behind the next list's MOVE
-// items; one-slice lists last), so each XCD writes into few lists at a time.  Items of a queue are dequeued in index order with
-// an atomic ticket, and every wait is on items of the same list, which sit
+// items; one-slice lists last), so each XCD writes into few lists at a time.
+// (PAIR items right behind their list's MOVE items: 1,263 us instead of 1,187 for
+// 4,096 lists of 2^8 to 2^20 items; streaming loads of R and the tail past the
+// caches: 1,232.)  Items of a queue are dequeued in index order with an atomic ticket, and every wait is on items of the same list, which sit
 // earlier in the same queue, so the queues drain whatever the number of
 // resident workgroups: no cooperative launch is needed.
 // The last workgroup to leave resets the tickets and the per-list counters, so
@@ -74,6 +79,12 @@ constexpr uint32_t kMaxBuckets = 128;                             // lists of fe
 constexpr uint32_t kBucketMinK = 1u << 19;                        // ... and at least this many
 constexpr uint32_t kBucketMaxL = 8192;                            // slice length the LDS staging holds
 constexpr uint16_t kPlanBucketed = 5;                             // ListPlan::method of such a list
+// Tail marks gathered in an LDS bitmap of the whole tail: lists of up to 1,024
+// removals per thread (2^18 for 256, 64 KB of bitmap at 512 threads, which
+// still lets two workgroups share a CU).
+constexpr uint32_t kLdsMarkPerThread = 1024;
+constexpr uint32_t kLdsMarkL = 8192;  // removals per MARK item
+constexpr uint16_t kPlanLdsMark = 6;  // ListPlan::method of such a list
 // longest slice of a list with fused items (its orphans take 4 bytes per pair of LDS)
 constexpr uint32_t kFusedItemMaxL = 8192;
 
@@ -93,6 +104,11 @@ struct ListPlan {
 };
 static_assert(sizeof(ListPlan) == 80, "ListPlan is one 80-byte record");
 
+// MARK items of a list of several slices
+__host__ __device__ inline uint32_t mark_items(const ListPlan& P) {
+  return P.method == kPlanLdsMark ? (P.k + kLdsMarkL - 1) / kLdsMarkL : P.m;
+}
+
 // queue control words (uint32 index into the queue control block): the ticket
 // of queue x at kQTicket + 32 x (a line each), then the exit count
 constexpr int kQueues = 8;
@@ -107,8 +123,8 @@ struct QueueSplit {
 // appended to their buckets' entry lists in whole runs.
 template <int WG>
 __device__ __forceinline__ void bucket_marks(const int32_t* __restrict__ R, uint32_t a, uint32_t b, uint32_t k,
-                                             uint32_t sZ, uint32_t* __restrict__ ent, uint32_t* __restrict__ cur) {
-  __shared__ uint32_t s_stage[kBucketMaxL];
+                                             uint32_t sZ, uint32_t* __restrict__ ent, uint32_t* __restrict__ cur,
+                                             uint32_t* __restrict__ s_stage) {
   __shared__ uint32_t s_cnt[kMaxBuckets], s_lbase[kMaxBuckets], s_gbase[kMaxBuckets];
   __shared__ uint32_t s_total;
   const uint32_t tid = threadIdx.x;
@@ -169,6 +185,40 @@ __device__ __forceinline__ void bucket_marks(const int32_t* __restrict__ R, uint
   }
 }
 
+// MARK item of a list whose k-bit tail bitmap fits LDS: marks of removals
+// [a, b) gathered there, then its words that are not zero merged into the
+// list's bitmap, or written to it if this is the list's only MARK item.  The
+// words merged are consecutive, so a line of the bitmap is one memory request
+// (a mark by itself is one each).  Items of 8,192 removals: of 16,384 or 32,768
+// the merges are fewer still, but MOVE items wait longer for the last of them
+// (1,187, 1,200 and 1,238 us for 4,096 lists of 2^8 to 2^20 items).
+template <int WG>
+__device__ __forceinline__ void lds_marks(const int32_t* __restrict__ R, uint32_t a, uint32_t b, uint32_t k,
+                                          uint32_t sZ, uint32_t* __restrict__ lds, uint32_t* __restrict__ bits) {
+  const uint32_t tid = threadIdx.x, words = (k + 31) >> 5;
+  for (uint32_t w = tid; w < words; w += WG) lds[w] = 0u;
+  __syncthreads();
+  constexpr int U = 8;  // loads in flight per thread, then their uses
+  for (uint32_t i0 = a + tid; i0 < b; i0 += WG * U) {
+    uint32_t r[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) r[u] = i0 + u * WG < b ? (uint32_t)R[i0 + u * WG] : sZ - 1u;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const uint32_t z = r[u] - sZ;  // wraps to >= 2^31 > k below the tail
+      if (z < k) atomicOr(&lds[z >> 5], 1u << (z & 31));
+    }
+  }
+  __syncthreads();
+  const bool only = a == 0 && b == k;
+  for (uint32_t w = tid; w < words; w += WG) {
+    const uint32_t v = lds[w];
+    if (!v) continue;
+    if (only) st_relaxed(&bits[w], v);
+    else or_relaxed(&bits[w], v);
+  }
+}
+
 // BUCKET item b: bucket b's bits into LDS, then its bitmap words written whole
 // (the bitmap is zero outside the marks); the bucket's count back to zero.
 template <int WG>
@@ -218,6 +268,7 @@ __device__ __forceinline__ void run_item(const ListPlan& P, uint32_t li, uint32_
   uint32_t* lb = bits + P.bits_off;
   uint64_t* lc = counts + P.counts_off;
   const uint32_t tid = threadIdx.x;
+  extern __shared__ uint32_t s_dyn[];  // MARK items: the staging of bucketed marks, or the tail's bitmap
   if (kind == kSingle) {
     mark_body<false>(R, P.k, P.k, P.sZ, lb, nullptr, tid, WG);
     wait_all_memory();
@@ -229,7 +280,9 @@ __device__ __forceinline__ void run_item(const ListPlan& P, uint32_t li, uint32_
   } else if (kind == kMark) {
     const uint32_t a = j * P.L, b = min(a + P.L, P.k);
     if (BUCK && P.method == kPlanBucketed) {
-      if constexpr (BUCK) bucket_marks<WG>(R, a, b, P.k, P.sZ, (uint32_t*)P.ent, (uint32_t*)P.cur);
+      if constexpr (BUCK) bucket_marks<WG>(R, a, b, P.k, P.sZ, (uint32_t*)P.ent, (uint32_t*)P.cur, s_dyn);
+    } else if (P.method == kPlanLdsMark) {
+      lds_marks<WG>(R, j * kLdsMarkL, min((j + 1) * kLdsMarkL, P.k), P.k, P.sZ, s_dyn, lb);
     } else {
       mark_body<false>(R + a, b - a, P.k, P.sZ, lb, nullptr, tid, WG);
     }
@@ -276,7 +329,7 @@ __device__ __forceinline__ void run_item(const ListPlan& P, uint32_t li, uint32_
     if (BUCK && P.method == kPlanBucketed)
       wait_count(&done[3 * li + 2], (P.k + kBucketW - 1) >> kBucketLog, ctrl);  // the BUCKET items
     else
-      wait_count(&done[3 * li], P.m, ctrl);
+      wait_count(&done[3 * li], mark_items(P), ctrl);
     move_slice<T, WG, IPT, true>(A, R, Rd, P.k, P.sZ, P.L, j, lb, lc, msh, &done[3 * li + 1]);
   } else {
     wait_count(&done[3 * li + 1], P.m, ctrl);
@@ -480,7 +533,7 @@ struct rz_batch {
   rz::QueueSplit split;
   rz::DeviceBuffer plans, qctl, bits, counts, orphans, slots, ents, curs;  // plans holds the items too
   const uint2* d_items = nullptr;  // the items, in `plans` after the list plans
-  size_t lds = 0;  // dynamic LDS of the launch: the longest fused-item slice's orphan list
+  size_t lds = 0;  // dynamic LDS of the launch: the most that one of its items needs
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
   rz_batch_info info;
@@ -520,7 +573,7 @@ static rz_status batch_plan(rz_batch* b, const rz_list_desc* lists, int32_t nlis
   items.clear();
   keys.clear();
   uint64_t bits_words = 0, count_words = 0, orphan_words = 0, slot_words = 0, ent_words = 0, cur_words = 0;
-  uint32_t fused_L = 0;
+  uint32_t fused_L = 0, tail_k = 0;
   bool any_part = false;
   for (int32_t i = 0; i < nlists; ++i) {
     const rz_list_desc& d = lists[i];
@@ -560,6 +613,15 @@ static rz_status batch_plan(rz_batch* b, const rz_list_desc* lists, int32_t nlis
         plans[i].cur = cur_words;
         ent_words += (uint64_t)nb * kBucketW;
         cur_words += nb;
+      } else if (plans[i].m > 1 && d.k <= (int64_t)cfg.wg_size * kLdsMarkPerThread) {
+        // One atomic per tail removal went to memory each: 16.2 of the 83 M memory
+        // requests of 4,096 lists of 2^8 to 2^20 items (17 M tail removals), and 26 G/s
+        // is the most that such atomics reach.  With the bitmap 1.7 M are left and the
+        // batch takes 1,190 us instead of 1,385; 512 lists of 428 K removals 2,820 us,
+        // with buckets 3,175, with atomics 3,750; sparse lists (1,024 of 32 K removals
+        // in 2^20 items) 1,210 either way.
+        plans[i].method = kPlanLdsMark;
+        tail_k = std::max(tail_k, plans[i].k);
       }
       bits_words += (uint64_t)((d.k + 63) / 64) * 2;
       count_words += plans[i].m;
@@ -615,7 +677,8 @@ static rz_status batch_plan(rz_batch* b, const rz_list_desc* lists, int32_t nlis
     };
     // the three phases of a list: marks, then moves (or partition tiles), then PAIR items
     auto marks = [&](uint32_t li) {
-      push_all(li, plans[li].method == RZ_METHOD_PARTITION ? kPMark : kMark, plans[li].m);
+      if (plans[li].method == RZ_METHOD_PARTITION) push_all(li, kPMark, plans[li].m);
+      else push_all(li, kMark, mark_items(plans[li]));
     };
     auto moves = [&](uint32_t li) {
       const ListPlan& P = plans[li];
@@ -682,7 +745,8 @@ static rz_status batch_plan(rz_batch* b, const rz_list_desc* lists, int32_t nlis
     if (plan_bytes) RZ_HIP(hipMemcpy(b->plans.ptr, plans.data(), plan_bytes, hipMemcpyHostToDevice));
     if (item_bytes) RZ_HIP(hipMemcpy((char*)b->plans.ptr + item_off, items.data(), item_bytes, hipMemcpyHostToDevice));
   }
-  const size_t lds = (size_t)fused_L * 4;
+  const size_t lds = 4 * std::max<size_t>({(size_t)fused_L, (size_t)(tail_k + 31) / 32,
+                                           (size_t)(ent_words ? kBucketMaxL : 0u)});
   // some list runs fused items, or partition items
   const int mode = (fused_L ? kModeFused : 0) | (any_part ? kModePart : 0) | (ent_words ? kModeBuck : 0);
   if (mode) kern = queue_kernel(cfg.wg_size, cfg.items, mode);

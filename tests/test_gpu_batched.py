@@ -261,3 +261,26 @@ def test_batch_bucketed_marks(ctx, oracle):
     finally:
         ctx.set_batch_config(old)
     assert ctx.check_errors() == 0
+
+
+@pytest.mark.parametrize("esz,wg", [(4, 512), (8, 256), (16, 512)])
+def test_tail_marks_in_lds(ctx, oracle, esz, wg):
+    """Lists around the edges of the marks gathered in LDS: the first list of two
+    slices, one and two MARK items, a bitmap's last word and bit, and the longest
+    tail that fits (and one removal more); replayed, since every launch has to
+    leave the bitmaps zero."""
+    step, top = wg * 8, wg * 1024
+    specs = [(3 * k, k, esz, p) for k in (step, step + 1, 8191, 8192, 8193, 16384 + 33, 5 * 8192 + 31)
+             for p in ("uniform", "tail_heavy")]
+    specs += [(top + 5000, top - 1, esz, "uniform"), (2 * top, top, esz, "tail_heavy"),
+              (2 * top + 1, top + 1, esz, "uniform"), (8192 + 1, 8192, esz, "uniform")]
+    L = Lists(specs, seed=esz)
+    for variant in (0, 5):
+        announce("tail marks in lds", esz, wg, variant)
+        b = ctx.batch(L.pairs(), config=rz.TileConfig(wg, 8, 0, variant, 1, 1))
+        for rep in range(2):
+            L.restore()
+            b.launch()
+            L.check(oracle, f"variant {variant} launch {rep}")
+        b.close()
+    assert ctx.check_errors() == 0

@@ -18,7 +18,8 @@
 //                 words, so no list state survives from an earlier launch.
 // A list of several slices whose tail bitmap fits LDS (fewer than 2^19 removals
 // at 512 threads) has fewer MARK items, of 8,192 removals each: they gather their
-// marks in LDS and merge whole words (lds_marks).
+// marks in LDS and merge whole words (mark_range), or store them if the item is the
+// list's only one.
 // With batch variant 5, a list of 2^19 to 2^22 removals marks its tail in
 // buckets instead of one atomic per tail removal:
 //   MARK j        groups the tail removals of removals [jL, (j+1)L) by bucket
@@ -83,7 +84,10 @@ constexpr uint16_t kPlanBucketed = 5;                             // ListPlan::m
 // removals per thread (2^18 for 256, 64 KB of bitmap at 512 threads, which
 // still lets two workgroups share a CU).
 constexpr uint32_t kLdsMarkPerThread = 1024;
-constexpr uint32_t kLdsMarkL = 8192;  // removals per MARK item
+// Removals per MARK item: of 16,384 or 32,768 the merges are fewer still, but
+// MOVE items wait longer for the last of them (1,187, 1,200 and 1,238 us for 4,096
+// lists of 2^8 to 2^20 items).
+constexpr uint32_t kLdsMarkL = 8192;
 constexpr uint16_t kPlanLdsMark = 6;  // ListPlan::method of such a list
 // longest slice of a list with fused items (its orphans take 4 bytes per pair of LDS)
 constexpr uint32_t kFusedItemMaxL = 8192;
@@ -185,40 +189,6 @@ __device__ __forceinline__ void bucket_marks(const int32_t* __restrict__ R, uint
   }
 }
 
-// MARK item of a list whose k-bit tail bitmap fits LDS: marks of removals
-// [a, b) gathered there, then its words that are not zero merged into the
-// list's bitmap, or written to it if this is the list's only MARK item.  The
-// words merged are consecutive, so a line of the bitmap is one memory request
-// (a mark by itself is one each).  Items of 8,192 removals: of 16,384 or 32,768
-// the merges are fewer still, but MOVE items wait longer for the last of them
-// (1,187, 1,200 and 1,238 us for 4,096 lists of 2^8 to 2^20 items).
-template <int WG>
-__device__ __forceinline__ void lds_marks(const int32_t* __restrict__ R, uint32_t a, uint32_t b, uint32_t k,
-                                          uint32_t sZ, uint32_t* __restrict__ lds, uint32_t* __restrict__ bits) {
-  const uint32_t tid = threadIdx.x, words = (k + 31) >> 5;
-  for (uint32_t w = tid; w < words; w += WG) lds[w] = 0u;
-  __syncthreads();
-  constexpr int U = 8;  // loads in flight per thread, then their uses
-  for (uint32_t i0 = a + tid; i0 < b; i0 += WG * U) {
-    uint32_t r[U];
-#pragma unroll
-    for (int u = 0; u < U; ++u) r[u] = i0 + u * WG < b ? (uint32_t)R[i0 + u * WG] : sZ - 1u;
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const uint32_t z = r[u] - sZ;  // wraps to >= 2^31 > k below the tail
-      if (z < k) atomicOr(&lds[z >> 5], 1u << (z & 31));
-    }
-  }
-  __syncthreads();
-  const bool only = a == 0 && b == k;
-  for (uint32_t w = tid; w < words; w += WG) {
-    const uint32_t v = lds[w];
-    if (!v) continue;
-    if (only) st_relaxed(&bits[w], v);
-    else or_relaxed(&bits[w], v);
-  }
-}
-
 // BUCKET item b: bucket b's bits into LDS, then its bitmap words written whole
 // (the bitmap is zero outside the marks); the bucket's count back to zero.
 template <int WG>
@@ -282,7 +252,8 @@ __device__ __forceinline__ void run_item(const ListPlan& P, uint32_t li, uint32_
     if (BUCK && P.method == kPlanBucketed) {
       if constexpr (BUCK) bucket_marks<WG>(R, a, b, P.k, P.sZ, (uint32_t*)P.ent, (uint32_t*)P.cur, s_dyn);
     } else if (P.method == kPlanLdsMark) {
-      lds_marks<WG>(R, j * kLdsMarkL, min((j + 1) * kLdsMarkL, P.k), P.k, P.sZ, s_dyn, lb);
+      const uint32_t a6 = j * kLdsMarkL, b6 = min(a6 + kLdsMarkL, P.k);
+      mark_range<WG>(R, a6, b6, P.sZ, 0u, P.k, b6 - a6 == P.k, s_dyn, lb);
     } else {
       mark_body<false>(R + a, b - a, P.k, P.sZ, lb, nullptr, tid, WG);
     }

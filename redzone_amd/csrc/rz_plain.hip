@@ -78,6 +78,16 @@ __global__ __launch_bounds__(256) void rz_mark_tail_sorted(const int32_t* __rest
   mark_body<false>(R + lo, hi - lo, k, sZ, bits, nullptr, threadIdx.x, 256u);
 }
 
+// Workgroup (range, chunk): the marks of one range of the tail among one chunk
+// of the removals, ranges of a chunk side by side.
+__global__ __launch_bounds__(1024) void rz_mark_ranges(const int32_t* __restrict__ R, uint32_t k, uint32_t sZ,
+                                                       uint32_t* __restrict__ bits, uint32_t ranges, uint32_t span,
+                                                       uint32_t chunk) {
+  extern __shared__ uint32_t s_orph[];
+  const uint32_t lo = blockIdx.x % ranges * span, a = blockIdx.x / ranges * chunk;
+  mark_range<1024, false, 16>(R, a, min(a + chunk, k), sZ, lo, min(span, k - lo), false, s_orph, bits);
+}
+
 template <typename T, int WG, int IPT>
 __global__ __launch_bounds__(WG) void rz_move(T* __restrict__ A, const int32_t* __restrict__ R,
                                                int32_t* __restrict__ Rd, uint32_t k, uint32_t sZ, uint32_t L,
@@ -170,11 +180,21 @@ template <int WG>
 __device__ __forceinline__ void mark_group_body(const int32_t* __restrict__ R, uint32_t k, uint32_t sZ,
                                                 uint32_t* __restrict__ bits, uint32_t* __restrict__ ctrl, int stats,
                                                 uint32_t nm, uint32_t tile, int sorted,
-                                                uint64_t* __restrict__ stamps) {
+                                                uint64_t* __restrict__ stamps, uint32_t ranges = 0,
+                                                uint32_t span = 0) {
   uint64_t* const my_stamps = stamps ? stamps + (size_t)blockIdx.x * kStampsPerGroup : nullptr;
   if (my_stamps && threadIdx.x == 0) my_stamps[kStampStart] = wall_clock64();
   const uint32_t lo = blockIdx.x * tile, hi = min(lo + tile, k);
-  if (!sorted || (uint32_t)R[hi - 1] >= sZ) {  // a sorted chunk below the red zone has no marks
+  if (ranges) {
+    // this workgroup's range of the tail and chunk (of `tile` removals), as in rz_mark_ranges
+    extern __shared__ uint32_t s_orph[];  // span / 32 words or more
+    const uint32_t z0 = blockIdx.x % ranges * span, a = blockIdx.x / ranges * tile;
+    const uint32_t b = min(a + tile, k), len = min(span, k - z0);
+    if (stats)
+      mark_range<WG, true, 16>(R, a, b, sZ, z0, len, false, s_orph, bits, (uint64_t*)&ctrl[kCtrlStatTail]);
+    else
+      mark_range<WG, false, 16>(R, a, b, sZ, z0, len, false, s_orph, bits);
+  } else if (!sorted || (uint32_t)R[hi - 1] >= sZ) {  // a sorted chunk below the red zone has no marks
     // a whole tile's loads in flight at once (16 per thread for 4,096 removals and 256 threads)
     if (stats)
       mark_body<true, 16>(R + lo, hi - lo, k, sZ, bits, (uint64_t*)&ctrl[kCtrlStatTail], threadIdx.x, WG);
@@ -215,9 +235,9 @@ __global__ __launch_bounds__(WG) void rz_mark_move_pair(T* __restrict__ A, const
                                                          uint32_t tile, uint32_t backoff, int sorted, int early,
                                                          uint32_t* __restrict__ err_out,
                                                          uint64_t* __restrict__ stamps, const T* __restrict__ add,
-                                                         uint32_t split) {
+                                                         uint32_t split, uint32_t ranges) {
   if (blockIdx.x < nm) {
-    mark_group_body<WG>(R, k, sZ, bits, ctrl, stats, nm, tile, sorted, stamps);
+    mark_group_body<WG>(R, k, sZ, bits, ctrl, stats, nm, tile, sorted, stamps, ranges, 32u * L);
     return;
   }
   move_pair_body<T, WG, IPT, true>(A, R, k, sZ, L, ns, bits, mstatus, slots, slot_cap, ctrl, stats, early,
@@ -594,10 +614,66 @@ constexpr rz_tile_config kSmallFused = {256, 4, 512, 6, 12, 1};
 static int clamp_tile_log(int tile_log) {
   return tile_log == 0 ? kFusedMarkTileLog : (tile_log < 8 ? 8 : (tile_log > 16 ? 16 : tile_log));
 }
-// mark workgroups of the one-launch form for k removals
-static uint32_t mark_groups(int64_t k, int tile_log) {
-  const uint32_t tile = 1u << clamp_tile_log(tile_log);
-  return (uint32_t)((k + tile - 1) / tile);
+
+// Whether the tail marks of an unsorted list are gathered by ranges in LDS: a
+// mark by itself is a memory request, of which 26 G/s is the most, and a call
+// makes k * k / n of them; by ranges every removal is read once per range, from
+// the caches.  Whole calls on MI355X, 4-byte items, marks one by one -> by ranges,
+// us, at n = 1.3 k / 2.2 k / 4 k / 5 k / 8 k:
+//   k = 2^15.6     15.0 -> 10.4 / 13.7 -> 11.1 / 11.6 -> 10.5 / 11.0 -> 10.5 / 10.5 -> 10.6
+//   k = 2^17.5     17.3 -> 12.1 / 15.5 -> 13.1 / 13.8 -> 13.0 / 13.5 -> 13.2 / 12.2 -> 12.4
+//   k = 2^19.0     34.0 -> 17.3 / 26.9 -> 19.1 / 21.8 -> 19.6 / 20.3 -> 19.8 / 18.0 -> 19.3
+//   k = 2^20.95    80.8 -> 36.5 / 64.0 -> 42.1 / 52.4 -> 45.8 / 49.2 -> 45.8 / 44.1 -> 46.8
+//   k = 2^22.6    232.9 -> 98.9 / 199 -> 145 / 171 -> 166 / 177 -> 184 / 186 -> 212
+//   k = 2^23.3    388 -> 214 / 324 -> 283 / 276 -> 315 / 273 -> 332 / 302 -> 393
+// and much the same for 8- and 16-byte items.  The two meet at n = 4.3 k for
+// 2^19.5 and 2^20.5 and later for the others; the direct form has k below 2^15.
+static bool range_marks(int64_t n, int64_t k) { return k >= 1 << 15 && k < 1 << 23 && 4 * n <= 17 * k; }
+
+// The mark workgroups of a call: tiles of removals, or (ranges > 0) ranges of
+// `span` tail positions times chunks of `tile` removals.
+struct MarkPlan {
+  uint32_t nm, tile, ranges;
+};
+static MarkPlan range_plan(int64_t k, uint32_t span) {
+  MarkPlan p;
+  // A chunk's words are merged once per workgroup, so small calls take fewer:
+  // 128 / 256 / 512 workgroups, n = 2.2 k, us: k = 2^17.5 13.1 / 13.8 / -,
+  // 2^18.5 17.0 / 17.1 / -, 2^20 - / 27.9 / 28.5, 2^20.95 - / 48.7 / 42.1.
+  const uint32_t groups = (uint32_t)std::min<int64_t>(512, std::max<int64_t>(128, k / 4096));
+  p.ranges = (uint32_t)((k + span - 1) / span);
+  const uint32_t chunks = groups > p.ranges ? groups / p.ranges : 1u;
+  p.tile = (uint32_t)((k + chunks - 1) / chunks);
+  p.nm = p.ranges * (uint32_t)((k + p.tile - 1) / p.tile);
+  return p;
+}
+// One-launch form: the mark workgroups' LDS is the slices', so a range is 32 L
+// positions, and shapes of short slices (more than 16 ranges) keep the tiles.
+static MarkPlan mark_plan(int64_t n, int64_t k, uint32_t L, int tile_log, bool sorted) {
+  if (!sorted && range_marks(n, k) && k <= 16ll * 32 * L) return range_plan(k, 32u * L);
+  MarkPlan p;
+  p.tile = 1u << clamp_tile_log(tile_log);
+  p.nm = (uint32_t)((k + p.tile - 1) / p.tile);
+  p.ranges = 0;
+  return p;
+}
+
+// The marks as a kernel of their own; `grid` for one mark at a time.
+static void launch_marks(const int32_t* R, int64_t n, int64_t k, uint32_t* bits, bool sorted, dim3 grid,
+                         hipStream_t s) {
+  const uint32_t sZ = (uint32_t)(n - k);
+  if (sorted) {
+    hipLaunchKernelGGL(rz_mark_tail_sorted, dim3((uint32_t)((k + kSortedChunk - 1) / kSortedChunk)), dim3(256), 0, s,
+                       R, (uint32_t)k, sZ, bits);
+  } else if (range_marks(n, k)) {
+    // ranges of 8, 16 and 32 KB: about 16 of them
+    const uint32_t span = k <= 1 << 20 ? 1u << 16 : k <= 1 << 21 ? 1u << 17 : 1u << 18;
+    const MarkPlan p = range_plan(k, span);
+    hipLaunchKernelGGL(rz_mark_ranges, dim3(p.nm), dim3(1024), span / 8, s, R, (uint32_t)k, sZ, bits, p.ranges, span,
+                       p.tile);
+  } else {
+    hipLaunchKernelGGL(rz_mark_tail<false>, grid, dim3(256), 0, s, R, (uint32_t)k, sZ, bits, (uint64_t*)nullptr);
+  }
 }
 
 // Variant 6: nm mark workgroups, then the ns move-and-pair slices, one grid.
@@ -609,14 +685,12 @@ static bool dispatch_mark_move_pair(int wg, int ipt, hipStream_t s, T* A, const 
                                     const T* add = nullptr, uint32_t split = 0xffffffffu) {
   const uint32_t bo = kMarkWaitBackoff;
   const size_t lds = (size_t)L * 4;
-  tile_log = clamp_tile_log(tile_log);
-  const uint32_t tile = 1u << tile_log;
-  const uint32_t nm = (k + tile - 1) / tile;
+  const MarkPlan mp = mark_plan((int64_t)sZ + k, k, L, tile_log, sorted != 0);
 #define RZ_MMP_CASE(W, I)                                                                                      \
   if (wg == W && ipt == I) {                                                                                   \
-    hipLaunchKernelGGL((rz_mark_move_pair<T, W, I>), dim3(nm + ns), dim3(W), lds, s, A, R, k, sZ, L, ns, bits, \
-                       mstatus, slots, slot_cap, ctrl, stats, nm, tile, bo, sorted, early, err_out, stamps,    \
-                       add, split);                                                                            \
+    hipLaunchKernelGGL((rz_mark_move_pair<T, W, I>), dim3(mp.nm + ns), dim3(W), lds, s, A, R, k, sZ, L, ns,    \
+                       bits, mstatus, slots, slot_cap, ctrl, stats, mp.nm, mp.tile, bo, sorted, early, err_out, \
+                       stamps, add, split, mp.ranges);                                                         \
     return true;                                                                                               \
   }
   RZ_MMP_CASE(256, 2) RZ_MMP_CASE(256, 4) RZ_MMP_CASE(256, 8) RZ_MMP_CASE(256, 16)
@@ -733,11 +807,8 @@ static rz_status plain_impl(rz_ctx* ctx, T* A, int64_t n, int32_t* R, int64_t k,
   } else if (stats)
     hipLaunchKernelGGL(rz_mark_tail<true>, g1, dim3(256), 0, s, R, (uint32_t)k, sZ, bits,
                        (uint64_t*)(ctrl + kCtrlStatTail));
-  else if (flags & RZ_SORTED)
-    hipLaunchKernelGGL(rz_mark_tail_sorted, dim3((uint32_t)((k + kSortedChunk - 1) / kSortedChunk)), dim3(256), 0,
-                       s, R, (uint32_t)k, sZ, bits);
   else
-    hipLaunchKernelGGL(rz_mark_tail<false>, g1, dim3(256), 0, s, R, (uint32_t)k, sZ, bits, (uint64_t*)nullptr);
+    launch_marks(R, n, k, bits, (flags & RZ_SORTED) != 0, g1, s);
   RZ_HIP(hipGetLastError());
   if ((st = prof_mark(ctx, flags, 1, s)) != RZ_OK) return st;
   if (cfg.variant == 5) {
@@ -751,12 +822,14 @@ static rz_status plain_impl(rz_ctx* ctx, T* A, int64_t n, int32_t* R, int64_t k,
   }
   uint64_t* stamps = nullptr;
   if (fused && (flags & RZ_PROFILE)) {
-    const uint32_t groups = ns + (one_launch ? mark_groups(k, cfg.slice_steps) : 0u);
+    const uint32_t marks =
+        one_launch ? mark_plan(n, k, L, cfg.slice_steps, (flags & RZ_SORTED) != 0).nm : 0u;
+    const uint32_t groups = ns + marks;
     if ((st = ensure(ctx, ctx->stamps, (size_t)groups * kStampsPerGroup * 8, s)) != RZ_OK) return st;
     stamps = (uint64_t*)ctx->stamps.ptr;
     if ((st = fill_u32((uint32_t*)stamps, 0u, (size_t)groups * kStampsPerGroup * 2, s)) != RZ_OK) return st;
     ctx->stamp_groups = groups;
-    ctx->stamp_marks = one_launch ? mark_groups(k, cfg.slice_steps) : 0u;
+    ctx->stamp_marks = marks;
   }
   if (one_launch) {
     if (!dispatch_mark_move_pair<T>(cfg.wg_size, cfg.items, s, A, R, (uint32_t)k, sZ, L, ns, bits,
@@ -825,14 +898,8 @@ static rz_status fused_static_impl(T* A, int64_t n, const int32_t* R, int64_t k,
                                     early, fs.err_out))
       return RZ_EINVAL;
   } else {
-    if (flags & RZ_SORTED)
-      hipLaunchKernelGGL(rz_mark_tail_sorted, dim3((uint32_t)((k + kSortedChunk - 1) / kSortedChunk)), dim3(256), 0,
-                         s, R, (uint32_t)k, sZ, fs.bits);
-    else {
-      const int64_t g1w = (k + 256 * 4 - 1) / (256 * 4);
-      hipLaunchKernelGGL(rz_mark_tail<false>, dim3((uint32_t)(g1w < 2048 ? g1w : 2048)), dim3(256), 0, s, R,
-                         (uint32_t)k, sZ, fs.bits, (uint64_t*)nullptr);
-    }
+    const int64_t g1w = (k + 256 * 4 - 1) / (256 * 4);
+    launch_marks(R, n, k, fs.bits, (flags & RZ_SORTED) != 0, dim3((uint32_t)(g1w < 2048 ? g1w : 2048)), s);
     RZ_HIP(hipGetLastError());
     if (!dispatch_move_pair<T>(cfg.wg_size, cfg.items, s, A, R, (uint32_t)k, sZ, L, ns, fs.bits, fs.mstatus,
                                fs.slots, slot_cap, fs.ctrl, 0, early, fs.err_out))

@@ -73,6 +73,46 @@ __device__ __forceinline__ void mark_body(const int32_t* __restrict__ R, uint32_
   }
 }
 
+// The marks of tail positions [lo, lo + span) among removals [a, b), gathered
+// in LDS ((span + 31) / 32 words) and merged by words into the bitmap, or
+// stored when no other workgroup marks these positions (`only`).  lo is a
+// multiple of 32.  The words merged are consecutive, so a line of the bitmap
+// is one memory request, where a mark by itself is one each.
+template <int WG, bool STATS = false, int U = 8>
+__device__ __forceinline__ void mark_range(const int32_t* __restrict__ R, uint32_t a, uint32_t b, uint32_t sZ,
+                                           uint32_t lo, uint32_t span, bool only, uint32_t* __restrict__ lds,
+                                           uint32_t* __restrict__ bits, uint64_t* __restrict__ stat_tail = nullptr) {
+  const uint32_t tid = threadIdx.x, words = (span + 31) >> 5;
+  uint32_t hits = 0;
+  for (uint32_t w = tid; w < words; w += WG) lds[w] = 0u;
+  __syncthreads();
+  // U loads per thread in flight, then their uses
+  for (uint32_t i0 = a + tid; i0 < b; i0 += WG * U) {
+    uint32_t r[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) r[u] = i0 + u * WG < b ? (uint32_t)R[i0 + u * WG] : sZ - 1u;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const uint32_t z = r[u] - sZ - lo;  // wraps to >= 2^31 > span below the range
+      if (z < span) {
+        atomicOr(&lds[z >> 5], 1u << (z & 31));
+        if (STATS) ++hits;
+      }
+    }
+  }
+  if (STATS) {
+    hits = wave_sum(hits);
+    if (lane_id() == 0 && hits) add_relaxed(stat_tail, (uint64_t)hits);
+  }
+  __syncthreads();
+  for (uint32_t w = tid; w < words; w += WG) {
+    const uint32_t v = lds[w];
+    if (!v) continue;
+    if (only) st_relaxed(&bits[(lo >> 5) + w], v);
+    else or_relaxed(&bits[(lo >> 5) + w], v);
+  }
+}
+
 // ---------------------------------------------------------------------------
 // 2. move and collect orphans
 // ---------------------------------------------------------------------------

@@ -1,0 +1,41 @@
+"""Tail marks gathered by ranges in LDS (lists that lose a quarter of their items
+or more), in every form that marks by itself, against the CPU oracle: the edges of
+the rule, of ranges, chunks and words."""
+import pytest
+import torch
+
+import redzone_amd as rz
+from redzone_amd import workloads as W
+from tests.parity import announce, expected_canonical, gpu_remove_parity
+
+pytestmark = pytest.mark.gpu
+
+# one launch with slices of 2^10 and 2^12 pairs, fused, three kernels, dense with marks of its own kernel
+SHAPES = [(256, 4, 512, 6, 12, 1), (512, 8, 512, 6, 12, 1), (512, 4, 512, 4, 0, 1), (256, 4, 512, 0, 0, 1),
+          (512, 8, 1024, 5, 10, 1)]
+
+
+@pytest.mark.parametrize("esz,pattern", [(4, "uniform"), (8, "tail_heavy"), (16, "uniform"), (4, "clustered")])
+@pytest.mark.parametrize("k", [(1 << 15) - 1, 1 << 15, (1 << 16) + 33, 3 * 131072 + 1, (1 << 20) - 31, (1 << 20) + 1])
+def test_range_marks(ctx, oracle, esz, pattern, k):
+    top = 17 * k // 4  # the rule's last n, and the first beyond it
+    for n in (k + 1, 2 * k + 5, top, top + 1):
+        if n > 3 * k and (k > 1 << 18 or pattern == "clustered"):
+            continue
+        A = W.payload(esz, n, seed=k % 97)
+        R = W.removals(pattern, n, k, seed=k % 89)
+        want = expected_canonical(oracle, A.numpy(), R.numpy())
+        for s in SHAPES:
+            announce("range marks", esz, pattern, k, n, s)
+            gpu_remove_parity(ctx, oracle, A, R, config=rz.TileConfig(*s), want=want)
+    assert ctx.check_errors() == 0
+
+
+def test_range_marks_counted(ctx):
+    """The tail removals counted by the one-launch form are those of the list."""
+    k, n = 70001, 150000
+    R = W.removals("uniform", n, k, seed=3)
+    d = W.payload(4, n, seed=4).cuda()
+    ctx.remove(d, R.cuda(), flags=rz.RZ_STATS, config=rz.TileConfig(512, 4, 512, 6, 12, 1))
+    torch.cuda.synchronize()
+    assert ctx.last_stats().tail_removals == int((R >= n - k).sum())

@@ -6,8 +6,9 @@
 // (StreamCompact_OneBlock, redzone.hxx:526-603) or with thrust::remove
 // (Thrust_remove.hxx:15-17).  Here:
 //   rz_mark_all   sets one bit per removal in an n-bit bitmap (payload
-//                 agnostic) and bumps the look-back epoch; larger lists
-//                 (kPartBucketMinN, kPartBucketMinK) group the marks by
+//                 agnostic) and bumps the look-back epoch; denser lists mark
+//                 by ranges of the list in LDS (rz_part_ranges), and larger
+//                 ones (kPartBucketMinN, kPartBucketMinK) group the marks by
 //                 bitmap region first (bucket_marks), write every bitmap
 //                 word whole and count the removals of every tile;
 //   rz_compact    one pass over all n items in tiles of WG*IPT, tile id =
@@ -33,6 +34,7 @@
 #include <atomic>
 
 #include "rz_compact_dev.hpp"
+#include "rz_redzone_dev.hpp"
 #include "rz_ctx.hpp"
 #include "rz_device.hpp"
 
@@ -675,6 +677,42 @@ rz_status bucket_marks(rz_ctx* ctx, const int32_t* R, int64_t k, uint32_t base, 
 // k=n/4 40 -> 36 us.  At n=2^20, k=2^18 the atomics still win (30 vs 41 us).
 constexpr int64_t kPartBucketMinK = 1 << 19, kPartBucketMinN = 1 << 20;
 
+// Below that, and where the two kernels of the bucketed marks are mostly their
+// launches, workgroup (range, chunk) marks one range of the list among one chunk
+// of the removals in LDS and merges the words (mark_range).  Whole calls on 4-byte
+// items, us, random atomics or bucketed (b) -> by ranges, k/n = 0.1 / 0.4 / 0.8:
+//   n = 74,000       8.9 ->  9.8 / 11.0 ->  9.7 / 13.7   ->  9.3
+//   n = 296,000     10.2 -> 10.4 / 15.4 -> 10.1 / 22.5   -> 10.3
+//   n = 592,000     11.6 -> 10.8 / 19.5 -> 11.3 / 30.6   -> 12.2
+//   n = 1,185,000   14.7 -> 12.9 / 28.6 -> 15.0 / 20.3 b -> 16.3
+//   n = 2,370,000   22.3 -> 18.4 / 23.4 b -> 21.6 / 26.1 b -> 23.3
+//   n = 4,740,000   36.1 -> 27.7 / 31.0 b -> 34.5 / 33.4 b -> 40
+//   n = 9,480,000 and k/n = 0.02: 35.5 -> 35.1
+// and the same differences for 16-byte items.
+constexpr int64_t kPartRangeMaxN = 3 << 20;  // where the bucketed marks are the other choice
+static bool part_ranges(int64_t n, int64_t k, bool bucketed) {
+  if (bucketed && n > kPartRangeMaxN) return false;
+  return k >= 1 << 15 ? n <= 12 * k : k >= 1 << 14 && n <= 4 * k;
+}
+__global__ __launch_bounds__(1024) void rz_part_ranges(const int32_t* __restrict__ R, uint32_t k, uint32_t n,
+                                                       uint32_t* __restrict__ bits, uint32_t ranges, uint32_t span,
+                                                       uint32_t chunk, uint32_t* __restrict__ ctrl) {
+  extern __shared__ __align__(16) unsigned char dyn[];  // span / 32 words
+  const uint32_t lo = blockIdx.x % ranges * span, a = blockIdx.x / ranges * chunk, b = min(a + chunk, k);
+  mark_range<1024, false, 16>(R, a, b, 0u, lo, min(span, n - lo), a == 0 && b == k, (uint32_t*)dyn, bits);
+  if (blockIdx.x == 0 && threadIdx.x == 0) add_relaxed(&ctrl[kCtrlEpoch], 1u);
+}
+static void launch_part_ranges(const int32_t* R, int64_t n, int64_t k, uint32_t* bits, uint32_t* ctrl, hipStream_t s) {
+  // 3 to 5 ranges and 24 chunks while a range fits 32 KB; more chunks merge more
+  // words, fewer leave each workgroup more of the removals to read
+  uint32_t span = 1u << 15;
+  while (span < 1u << 18 && 5ll * span < n) span <<= 1;
+  const uint32_t ranges = (uint32_t)((n + span - 1) / span);
+  const uint32_t chunks = std::min(24u, std::max(1u, 256u / ranges)), chunk = ((uint32_t)k + chunks - 1) / chunks;
+  hipLaunchKernelGGL(rz_part_ranges, dim3(ranges * (((uint32_t)k + chunk - 1) / chunk)), dim3(1024), span / 8, s, R,
+                     (uint32_t)k, (uint32_t)n, bits, ranges, span, chunk, ctrl);
+}
+
 // 1024 threads x 4 vectors: 64 KiB tiles (staged in LDS); bigger tiles take
 // fewer look-back hops per byte (a 1 GiB probe: 16 KiB tiles 0.70 ms,
 // 64 KiB 0.54 ms, 128 KiB 0.56 ms; 1024 x 4 2% ahead of 512 x 8).
@@ -700,12 +738,16 @@ static rz_status partition_impl(rz_ctx* ctx, T* A, int64_t n, const int32_t* R, 
   const int64_t gw = (k + 255) / 256;
   const dim3 g1((uint32_t)(gw < (int64_t)ctx->cu_count * 8 ? (gw > 0 ? gw : 1) : ctx->cu_count * 8));
   if ((st = prof_mark(ctx, flags, 0, s)) != RZ_OK) return st;
-  const bool bucketed = k >= kPartBucketMinK && n >= kPartBucketMinN && bucket_marks_fit(n);
+  bool bucketed = k >= kPartBucketMinK && n >= kPartBucketMinN && bucket_marks_fit(n);
+  const bool ranges = part_ranges(n, k, bucketed);
+  bucketed = bucketed && !ranges;
   TileCounts tc;
   tc.tlog = (uint32_t)log2_floor(TILE);
   if (bucketed) {
     // the bitmap is zero here: every call leaves the words it used clear
     if ((st = bucket_marks(ctx, R, k, 0u, n, bits, ctrl, nullptr, s, vec ? &tc : nullptr)) != RZ_OK) return st;
+  } else if (ranges) {
+    launch_part_ranges(R, n, k, bits, ctrl, s);
   } else {
     hipLaunchKernelGGL(rz_mark_all, g1, dim3(256), 0, s, R, (uint32_t)k, (uint32_t)n, bits, ctrl);
   }

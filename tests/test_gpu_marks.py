@@ -39,3 +39,27 @@ def test_range_marks_counted(ctx):
     ctx.remove(d, R.cuda(), flags=rz.RZ_STATS, config=rz.TileConfig(512, 4, 512, 6, 12, 1))
     torch.cuda.synchronize()
     assert ctx.last_stats().tail_removals == int((R >= n - k).sum())
+
+
+@pytest.mark.parametrize("order", ["rising", "falling", "pairs", "sorted"])
+def test_range_marks_of_runs(ctx, oracle, order):
+    """Removals whose neighbours share bitmap words, in every order of a row."""
+    k = 40000 + 77
+    n = 2 * k + 3
+    R = torch.arange(n - k - k // 3, n - k // 3, dtype=torch.int32)
+    if order == "falling":
+        R = R.flip(0).contiguous()
+    elif order == "pairs":  # two runs that alternate lane by lane
+        R = torch.stack([R[: k // 2], R[k - k // 2:]], 1).reshape(-1)[: k - 1].contiguous()
+    elif order == "sorted":
+        R = W.uniform_removals(n, k, seed=9).sort().values.contiguous()
+    A = W.payload(4, n, seed=8)
+    want = expected_canonical(oracle, A.numpy(), R.numpy())
+    for s in SHAPES:
+        announce("range marks runs", order, s)
+        gpu_remove_parity(ctx, oracle, A, R, config=rz.TileConfig(*s), want=want)
+    d = A.cuda()
+    assert ctx.partition(d, R.cuda()) == n - len(R)
+    keep = torch.ones(n, dtype=torch.bool)
+    keep[R.long()] = False
+    assert torch.equal(d[: n - len(R)].cpu(), A[keep])

@@ -146,3 +146,17 @@ def test_partition_tile_counts_change_between_calls(ctx, oracle, esz):
         for frac in (0.01, 0.5):
             announce("partition tiles", esz, tiles, n, frac)
             _run(ctx, oracle, W.payload(esz, n, seed=61 + i), W.uniform_removals(n, int(n * frac), seed=62 + i))
+
+
+@pytest.mark.parametrize("esz", [4, 8, 16])
+@pytest.mark.parametrize("pattern", ["uniform", "clustered"])
+def test_partition_range_marks(ctx, oracle, esz, pattern):
+    """Marks by ranges in LDS: the first and last k and n of their rule and the
+    next beyond, lists that end on a range's and a word's edge or one item past
+    it, and k = n - 1."""
+    for n, k in [(40000, 1 << 14), (4 << 14, 1 << 14), ((4 << 14) + 1, 1 << 14), (30000, (1 << 14) - 1),
+                 (5 << 15, 1 << 15), ((5 << 15) + 1, 1 << 15), (12 << 15, 1 << 15), ((12 << 15) + 1, 1 << 15),
+                 (3 << 16, (3 << 16) - 1), ((3 << 17) + 33, 300007), (655361, 131101), (3 << 20, 1 << 19),
+                 ((3 << 20) + 1, 1 << 19), (1310721, (1 << 19) - 1), (5_000_003, (1 << 19) - 1)]:
+        announce("partition ranges", esz, pattern, n, k)
+        _run(ctx, oracle, W.payload(esz, n, seed=50), W.removals(pattern, n, k, seed=51))

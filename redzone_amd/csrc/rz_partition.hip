@@ -45,7 +45,7 @@ __global__ __launch_bounds__(256) void rz_mark_all(const int32_t* __restrict__ R
   const uint32_t stride = gridDim.x * 256u;
   for (uint32_t i = blockIdx.x * 256u + threadIdx.x; i < k; i += stride) {
     const uint32_t r = (uint32_t)R[i];
-    if (r < n) or_relaxed(&bits[r >> 5], 1u << (r & 31));
+    set_runs<false>(bits, r, r < n);
   }
   if (blockIdx.x == 0 && threadIdx.x == 0) add_relaxed(&ctrl[kCtrlEpoch], 1u);
 }

@@ -42,6 +42,40 @@ template <bool COH, typename T> __device__ __forceinline__ T ld_x(const T* p) {
 }
 
 // ---------------------------------------------------------------------------
+// bits of neighbouring removals
+// ---------------------------------------------------------------------------
+// Removals of neighbouring positions in neighbouring lanes (sorted or clustered
+// lists) serialise their atomics on one or two words, 64 cycles a wave in LDS.
+// next_word: the word of the lane above in the row of 16 (kNoWord for the last).
+constexpr uint32_t kNoWord = 0xfffffffeu;
+__device__ __forceinline__ uint32_t next_word(uint32_t w) {
+  return (uint32_t)__builtin_amdgcn_update_dpp((int)kNoWord, (int)w, 0x101, 0xf, 0xf, false);  // row_shl:1
+}
+// Sets bit z of a bitmap (in LDS or in memory) for the lanes with `hit`: each row ORs
+// its runs of one word together, and one lane of a run makes the atomic.  (Equal words that are
+// not neighbours may be merged as well, which changes nothing.)  2^20 removals in a
+// row of 2.2 times as many items: partition 48.6 -> 26.3 us, removal 47.0 -> 30.7.
+// On every removal it costs random lists 1 us of 12, so a round asks first.
+template <bool LDS>
+__device__ __forceinline__ void set_runs(uint32_t* __restrict__ bits, uint32_t z, bool hit) {
+  const uint32_t w = hit ? z >> 5 : 0xffffffffu;
+  uint32_t v = hit ? 1u << (z & 31) : 0u;
+#define RZ_OR_STEP(D)                                                                                          \
+  {                                                                                                            \
+    const uint32_t pw = (uint32_t)__builtin_amdgcn_update_dpp((int)kNoWord, (int)w, 0x110 + D, 0xf, 0xf, false); \
+    const uint32_t pv = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x110 + D, 0xf, 0xf, false);          \
+    if (pw == w) v |= pv;                                                                                      \
+  }
+  RZ_OR_STEP(1) RZ_OR_STEP(2) RZ_OR_STEP(4) RZ_OR_STEP(8)  // row_shr
+#undef RZ_OR_STEP
+  const uint32_t above = next_word(w);
+  if (hit && above != w) {
+    if (LDS) atomicOr(&bits[w], v);
+    else or_relaxed(&bits[w], v);
+  }
+}
+
+// ---------------------------------------------------------------------------
 // 1. mark: R[0, count) (a window of the removal list of a list with k
 // removals and red zone start sZ); thread gtid of `stride` threads.
 // ---------------------------------------------------------------------------
@@ -61,42 +95,16 @@ __device__ __forceinline__ void mark_body(const int32_t* __restrict__ R, uint32_
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const uint32_t z = r[u] - sZ;  // wraps to >= 2^31 > k below the tail
-      if (z < k) {
-        or_relaxed(&bits[z >> 5], 1u << (z & 31));
-        if (STATS) ++hits;
-      }
+      const uint64_t in = ballot(z < k);
+      if (__popcll(in) >= 8) set_runs<false>(bits, z, z < k);
+      else if (z < k) or_relaxed(&bits[z >> 5], 1u << (z & 31));
+      if (STATS) hits += z < k ? 1u : 0u;
     }
   }
   if (STATS) {
     hits = wave_sum(hits);
     if (lane_id() == 0 && hits) add_relaxed(stat_tail, (uint64_t)hits);
   }
-}
-
-// Removals of neighbouring positions in neighbouring lanes (sorted or clustered
-// lists) serialise their LDS atomics on one or two words, 64 cycles a wave.
-// next_word: the word of the lane above in the row of 16 (kNoWord for the last).
-constexpr uint32_t kNoWord = 0xfffffffeu;
-__device__ __forceinline__ uint32_t next_word(uint32_t w) {
-  return (uint32_t)__builtin_amdgcn_update_dpp((int)kNoWord, (int)w, 0x101, 0xf, 0xf, false);  // row_shl:1
-}
-// Sets bit z of an LDS bitmap for the lanes with `hit`: each row ORs its runs of
-// one word together, and one lane of a run goes to LDS.  (Equal words that are
-// not neighbours may be merged as well, which changes nothing.)  2^20 removals in a
-// row of 2.2 times as many items: partition 48.6 -> 26.3 us, removal 47.0 -> 30.7.
-// On every removal it costs random lists 1 us of 12, so a round asks first.
-__device__ __forceinline__ void set_runs_lds(uint32_t* __restrict__ lds, uint32_t z, bool hit) {
-  const uint32_t w = hit ? z >> 5 : 0xffffffffu;
-  uint32_t v = hit ? 1u << (z & 31) : 0u;
-#define RZ_OR_STEP(D)                                                                                          \
-  {                                                                                                            \
-    const uint32_t pw = (uint32_t)__builtin_amdgcn_update_dpp((int)kNoWord, (int)w, 0x110 + D, 0xf, 0xf, false); \
-    const uint32_t pv = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x110 + D, 0xf, 0xf, false);          \
-    if (pw == w) v |= pv;                                                                                      \
-  }
-  RZ_OR_STEP(1) RZ_OR_STEP(2) RZ_OR_STEP(4) RZ_OR_STEP(8)  // row_shr
-#undef RZ_OR_STEP
-  if (hit && next_word(w) != w) atomicOr(&lds[w], v);
 }
 
 // The marks of tail positions [lo, lo + span) among removals [a, b), gathered
@@ -123,7 +131,7 @@ __device__ __forceinline__ void mark_range(const int32_t* __restrict__ R, uint32
     const uint32_t w1 = next_word(w0);
     if (__popcll(ballot(z0 < span && w1 == w0)) >= 8) {
 #pragma unroll
-      for (int u = 0; u < U; ++u) set_runs_lds(lds, r[u] - sZ - lo, r[u] - sZ - lo < span);
+      for (int u = 0; u < U; ++u) set_runs<true>(lds, r[u] - sZ - lo, r[u] - sZ - lo < span);
     } else {
 #pragma unroll
       for (int u = 0; u < U; ++u) {

@@ -92,13 +92,22 @@ __device__ __forceinline__ void mark_body(const int32_t* __restrict__ R, uint32_
       const uint32_t i = i0 + u * stride;
       r[u] = i < count ? (uint32_t)R[i] : sZ - 1u;  // sZ-1 is never inside the tail (k > 0 => sZ < n)
     }
+    // z = r - sZ wraps to >= 2^31 > k below the tail
+    uint32_t most = 0;
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const uint32_t z = r[u] - sZ;  // wraps to >= 2^31 > k below the tail
-      const uint64_t in = ballot(z < k);
-      if (__popcll(in) >= 8) set_runs<false>(bits, z, z < k);
-      else if (z < k) or_relaxed(&bits[z >> 5], 1u << (z & 31));
-      if (STATS) hits += z < k ? 1u : 0u;
+      most = max(most, (uint32_t)__popcll(ballot(r[u] - sZ < k)));
+      if (STATS) hits += r[u] - sZ < k ? 1u : 0u;
+    }
+    // Random lists stay below 32 of 64 (they mark one by one up to k / n = 0.24).  One
+    // question a round: a branch per removal cost 0.4 us of 133.
+    if (__builtin_expect(most >= 32u, 0)) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) set_runs<false>(bits, r[u] - sZ, r[u] - sZ < k);
+    } else {
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (r[u] - sZ < k) or_relaxed(&bits[(r[u] - sZ) >> 5], 1u << ((r[u] - sZ) & 31));
     }
   }
   if (STATS) {

@@ -214,8 +214,8 @@ rz_status rz_remove_config(rz_ctx* ctx, void* d_data, int64_t n, uint32_t elem_b
  * device k needs leave at once.  The result is rz_remove's for (n, k).  Device
  * values outside 0 <= k <= n <= n_cap, k <= k_cap move nothing and set
  * RZ_ERR_SIZES (read by rz_check_errors).  Runs the one-launch fused form
- * (variant 6) with the tuned shape for k_cap when that is a fused form, else
- * 256 x 8; RZ_EINVAL if no fused shape fits k_cap (more than about 58.7 M
+ * (variant 6) with the tuned shape for k_cap when that is a fused form, with
+ * 256 x 4 where the tuned shape is the direct form (variant 7), else 256 x 8; RZ_EINVAL if no fused shape fits k_cap (more than about 58.7 M
  * removals: use rz_remove).  Flags: RZ_PRESERVE_REMOVALS, RZ_SORTED,
  * RZ_ANY_PAIRING, RZ_STATS, RZ_PROFILE; RZ_VALIDATE (which needs k on the
  * host) and RZ_COOPERATIVE are RZ_EINVAL.  A graph capture needs an eager call

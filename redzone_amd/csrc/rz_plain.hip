@@ -167,7 +167,8 @@ __global__ __launch_bounds__(WG) void rz_move_pair(T* __restrict__ A, const int3
 }
 
 // Variant 6: the mark step in the same launch.  Workgroups [0, nm) each mark
-// a tile of `tile` removals and count themselves done, and the last of them
+// a tile of `tile` removals (of dense lists a range of the tail among a chunk of
+// them, see range_marks) and count themselves done, and the last of them
 // raises a ready word per XCD; the move-and-pair slices come after them in
 // dispatch order (so every mark workgroup is running or done when a slice
 // waits), prefetch their first step and wait for their XCD's ready word.

@@ -8,9 +8,9 @@
 //   rz_mark_all   sets one bit per removal in an n-bit bitmap (payload
 //                 agnostic) and bumps the look-back epoch; denser lists mark
 //                 by ranges of the list in LDS (rz_part_ranges), and larger
-//                 ones (kPartBucketMinN, kPartBucketMinK) group the marks by
-//                 bitmap region first (bucket_marks), write every bitmap
-//                 word whole and count the removals of every tile;
+//                 ones (part_marks) group the marks by bitmap region first
+//                 (bucket_marks), write every bitmap word whole and count the
+//                 removals of every tile;
 //   rz_compact    one pass over all n items in tiles of WG*IPT, tile id =
 //                 workgroup id (workgroups are dispatched in id order).  Each
 //                 tile ranks its kept items with wave ballots and one LDS scan,
@@ -37,6 +37,7 @@
 #include "rz_redzone_dev.hpp"
 #include "rz_ctx.hpp"
 #include "rz_device.hpp"
+#include "rz_rules.hpp"
 
 namespace rz {
 
@@ -384,7 +385,6 @@ constexpr int kPartWG = 256, kPartIPT = 16;
 constexpr uint32_t kPartMinBinLog = 15, kPartMaxBinLog = 20;  // 4 to 128 KiB LDS bitmaps
 constexpr uint32_t kPartMaxBins = 1024;
 constexpr uint32_t kMaxTilesPerBin = 256;  // 2^20 positions in tiles of 2^12
-constexpr int64_t kPartMaxWindow = (int64_t)1 << 29;  // entry lists of 2 GiB
 constexpr uint32_t kAppWG = 1024;
 // Removals per thread of a tile (dynamic LDS, 4 bytes a removal).  A bigger
 // tile writes longer runs of consecutive words per bin: a run's two ends share
@@ -669,31 +669,10 @@ rz_status bucket_marks(rz_ctx* ctx, const int32_t* R, int64_t k, uint32_t base, 
   return RZ_OK;
 }
 
-// Marks of lists of at least kPartBucketMinN items and kPartBucketMinK removals
-// are grouped by bitmap region first: one random device atomic per removal
-// runs at about 40 G/s, where the two bucketing kernels stream.  Whole calls
-// on 4-byte items, random atomics -> bucketed: n=2^22, k=n/2 105 -> 43 us
-// (clustered 160 -> 47 us); n=6,000,000, k=0.8n 202 -> 55 us; n=2^21,
-// k=n/4 40 -> 36 us.  At n=2^20, k=2^18 the atomics still win (30 vs 41 us).
-constexpr int64_t kPartBucketMinK = 1 << 19, kPartBucketMinN = 1 << 20;
-
-// Below that, and where the two kernels of the bucketed marks are mostly their
-// launches, workgroup (range, chunk) marks one range of the list among one chunk
-// of the removals in LDS and merges the words (mark_range).  Whole calls on 4-byte
-// items, us, random atomics or bucketed (b) -> by ranges, k/n = 0.1 / 0.4 / 0.8:
-//   n = 74,000       8.9 ->  9.8 / 11.0 ->  9.7 / 13.7   ->  9.3
-//   n = 296,000     10.2 -> 10.4 / 15.4 -> 10.1 / 22.5   -> 10.3
-//   n = 592,000     11.6 -> 10.8 / 19.5 -> 11.3 / 30.6   -> 12.2
-//   n = 1,185,000   14.7 -> 12.9 / 28.6 -> 15.0 / 20.3 b -> 16.3
-//   n = 2,370,000   22.3 -> 18.4 / 23.4 b -> 21.6 / 26.1 b -> 23.3
-//   n = 4,740,000   36.1 -> 27.7 / 31.0 b -> 34.5 / 33.4 b -> 40
-//   n = 9,480,000 and k/n = 0.02: 35.5 -> 35.1
-// and the same differences for 16-byte items.
-constexpr int64_t kPartRangeMaxN = 3 << 20;  // where the bucketed marks are the other choice
-static bool part_ranges(int64_t n, int64_t k, bool bucketed) {
-  if (bucketed && n > kPartRangeMaxN) return false;
-  return k >= 1 << 15 ? n <= 12 * k : k >= 1 << 14 && n <= 4 * k;
-}
+// ---------------------------------------------------------------------------
+// Marks by ranges (part_marks): workgroup (range, chunk) marks one range of the
+// list among one chunk of the removals in LDS and merges the words.
+// ---------------------------------------------------------------------------
 __global__ __launch_bounds__(1024) void rz_part_ranges(const int32_t* __restrict__ R, uint32_t k, uint32_t n,
                                                        uint32_t* __restrict__ bits, uint32_t ranges, uint32_t span,
                                                        uint32_t chunk, uint32_t* __restrict__ ctrl) {
@@ -703,10 +682,9 @@ __global__ __launch_bounds__(1024) void rz_part_ranges(const int32_t* __restrict
   if (blockIdx.x == 0 && threadIdx.x == 0) add_relaxed(&ctrl[kCtrlEpoch], 1u);
 }
 static void launch_part_ranges(const int32_t* R, int64_t n, int64_t k, uint32_t* bits, uint32_t* ctrl, hipStream_t s) {
-  // 3 to 5 ranges and 24 chunks while a range fits 32 KB; more chunks merge more
-  // words, fewer leave each workgroup more of the removals to read
-  uint32_t span = 1u << 15;
-  while (span < 1u << 18 && 5ll * span < n) span <<= 1;
+  // 24 chunks: more merge more words, fewer leave each workgroup more of the
+  // removals to read
+  const uint32_t span = part_range_span(n);
   const uint32_t ranges = (uint32_t)((n + span - 1) / span);
   const uint32_t chunks = std::min(24u, std::max(1u, 256u / ranges)), chunk = ((uint32_t)k + chunks - 1) / chunks;
   hipLaunchKernelGGL(rz_part_ranges, dim3(ranges * (((uint32_t)k + chunk - 1) / chunk)), dim3(1024), span / 8, s, R,
@@ -738,15 +716,13 @@ static rz_status partition_impl(rz_ctx* ctx, T* A, int64_t n, const int32_t* R, 
   const int64_t gw = (k + 255) / 256;
   const dim3 g1((uint32_t)(gw < (int64_t)ctx->cu_count * 8 ? (gw > 0 ? gw : 1) : ctx->cu_count * 8));
   if ((st = prof_mark(ctx, flags, 0, s)) != RZ_OK) return st;
-  bool bucketed = k >= kPartBucketMinK && n >= kPartBucketMinN && bucket_marks_fit(n);
-  const bool ranges = part_ranges(n, k, bucketed);
-  bucketed = bucketed && !ranges;
+  const PartMarks marks = part_marks(n, k);
   TileCounts tc;
   tc.tlog = (uint32_t)log2_floor(TILE);
-  if (bucketed) {
+  if (marks == PartMarks::kBuckets) {
     // the bitmap is zero here: every call leaves the words it used clear
     if ((st = bucket_marks(ctx, R, k, 0u, n, bits, ctrl, nullptr, s, vec ? &tc : nullptr)) != RZ_OK) return st;
-  } else if (ranges) {
+  } else if (marks == PartMarks::kRanges) {
     launch_part_ranges(R, n, k, bits, ctrl, s);
   } else {
     hipLaunchKernelGGL(rz_mark_all, g1, dim3(256), 0, s, R, (uint32_t)k, (uint32_t)n, bits, ctrl);

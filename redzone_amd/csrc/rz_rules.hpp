@@ -1,0 +1,57 @@
+// rz_rules.hpp -- which form a call takes, as plain functions of its sizes (no
+// HIP: a host program can include this file alone).
+#pragma once
+
+#include <cstdint>
+
+namespace rz {
+
+// ---------------------------------------------------------------------------
+// the partition's marks
+// ---------------------------------------------------------------------------
+constexpr int64_t kPartMaxWindow = (int64_t)1 << 29;  // bucketed marks: entry lists of 2 GiB
+
+enum class PartMarks { kAtomic, kRanges, kBuckets };
+
+// Marks of lists of at least kPartBucketMinN items and kPartBucketMinK removals
+// are grouped by bitmap region first: one random device atomic per removal
+// runs at about 40 G/s, where the two bucketing kernels stream.  Whole calls
+// on 4-byte items, random atomics -> bucketed: n=2^22, k=n/2 105 -> 43 us
+// (clustered 160 -> 47 us); n=6,000,000, k=0.8n 202 -> 55 us; n=2^21,
+// k=n/4 40 -> 36 us.  At n=2^20, k=2^18 the atomics still win (30 vs 41 us).
+constexpr int64_t kPartBucketMinK = 1 << 19, kPartBucketMinN = 1 << 20;
+
+// Below that, and where the two kernels of the bucketed marks are mostly their
+// launches, workgroup (range, chunk) marks one range of the list among one chunk
+// of the removals in LDS and merges the words (mark_range).  Whole calls on 4-byte
+// items, us, random atomics or bucketed (b) -> by ranges, k/n = 0.1 / 0.4 / 0.8:
+//   n = 74,000       8.9 ->  9.8 / 11.0 ->  9.7 / 13.7   ->  9.3
+//   n = 296,000     10.2 -> 10.4 / 15.4 -> 10.1 / 22.5   -> 10.3
+//   n = 592,000     11.6 -> 10.8 / 19.5 -> 11.3 / 30.6   -> 12.2
+//   n = 1,185,000   14.7 -> 12.9 / 28.6 -> 15.0 / 20.3 b -> 16.3
+//   n = 2,370,000   22.3 -> 18.4 / 23.4 b -> 21.6 / 26.1 b -> 23.3
+//   n = 4,740,000   36.1 -> 27.7 / 31.0 b -> 34.5 / 33.4 b -> 40
+//   n = 9,480,000 and k/n = 0.02: 35.5 -> 35.1
+// and the same differences for 16-byte items.
+constexpr int64_t kPartRangeMaxN = 3 << 20;  // where the bucketed marks are the other choice
+
+// Every range reads all of the removals once, so ranges are for lists of few of
+// them: with fewer than kPartBucketMinK removals n <= 12 k keeps them to 24 of 2^18
+// positions, and above the bucketed marks' window (where a list would have
+// thousands) the atomics mark whatever k is.
+inline PartMarks part_marks(int64_t n, int64_t k) {
+  if (n > kPartMaxWindow) return PartMarks::kAtomic;
+  const bool bucketed = k >= kPartBucketMinK && n >= kPartBucketMinN;
+  if (bucketed && n > kPartRangeMaxN) return PartMarks::kBuckets;
+  if (k >= 1 << 15 ? n <= 12 * k : k >= 1 << 14 && n <= 4 * k) return PartMarks::kRanges;
+  return bucketed ? PartMarks::kBuckets : PartMarks::kAtomic;
+}
+
+// Positions per range: 3 to 5 ranges while a range fits 32 KB of LDS bitmap.
+inline uint32_t part_range_span(int64_t n) {
+  uint32_t span = 1u << 15;
+  while (span < 1u << 18 && 5ll * span < n) span <<= 1;
+  return span;
+}
+
+}  // namespace rz

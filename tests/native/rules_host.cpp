@@ -1,0 +1,27 @@
+// The rules of rz_rules.hpp at the sizes on stdin, one question a line:
+//   part <n> <k>   ->  atomic | buckets | ranges <number of ranges>
+#include <cstdio>
+#include <cstring>
+
+#include "../../redzone_amd/csrc/rz_rules.hpp"
+
+int main() {
+  char what[32];
+  while (scanf("%31s", what) == 1) {
+    if (!strcmp(what, "part")) {
+      long long n, k;
+      if (scanf("%lld %lld", &n, &k) != 2) return 1;
+      switch (rz::part_marks(n, k)) {
+        case rz::PartMarks::kAtomic: printf("atomic\n"); break;
+        case rz::PartMarks::kBuckets: printf("buckets\n"); break;
+        case rz::PartMarks::kRanges: {
+          const long long span = rz::part_range_span(n);
+          printf("ranges %lld\n", (n + span - 1) / span);
+        }
+      }
+    } else {
+      return 1;
+    }
+  }
+  return 0;
+}

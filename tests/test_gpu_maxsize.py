@@ -101,3 +101,29 @@ def test_max_size_rec16(ctx, oracle, big):
     del host
     m = first_mismatch(got[: N_MAX - k], want[: N_MAX - k])
     assert m < 0, f"first mismatch at {m}"
+
+
+@pytest.mark.parametrize("n", [(1 << 29) + 12345, N_MAX])
+def test_partition_above_the_bucketed_window(ctx, big, n):
+    """A quarter removed from lists above 2^29 items, whose marks are one atomic
+    per removal, compared on the device."""
+    A0, _ = big
+    k = n // 4
+    announce("partition above 2^29", n, k)
+    R = torch.empty(k, dtype=torch.int32, device="cuda")
+    ctx.gen_uniform_removals(R, n, 170)
+    A = A0[:n].clone()
+    assert ctx.partition(A, R) == n - k
+    keep = torch.ones(n, dtype=torch.bool, device="cuda")
+    keep[R.long()] = False
+    at = 0
+    for lo in range(0, n, 1 << 27):
+        hi = min(lo + (1 << 27), n)
+        want = A0[lo:hi][keep[lo:hi]]
+        assert torch.equal(A[at:at + want.shape[0]], want), (n, lo)
+        at += want.shape[0]
+    assert at == n - k
+    ctx.partition(A, R, flags=rz.RZ_PROFILE)
+    marks = ctx.last_profile()[0]
+    print("marks", n, k, round(marks, 2), "ms")
+    assert ctx.check_errors() == 0

@@ -1,0 +1,45 @@
+"""Which form a call takes (redzone_amd/csrc/rz_rules.hpp), through a small host
+program: over whole ranges of sizes, without a GPU."""
+import os
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+
+@pytest.fixture(scope="module")
+def ask(tmp_path_factory):
+    exe = str(tmp_path_factory.mktemp("rules") / "rules_host")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-o", exe, os.path.join(ROOT, "tests", "native", "rules_host.cpp")],
+                   check=True)
+
+    def run(questions):
+        text = "\n".join(" ".join(str(x) for x in q) for q in questions)
+        out = subprocess.run([exe], input=text, capture_output=True, text=True, check=True, timeout=60).stdout.split("\n")
+        assert len(out) == len(questions) + 1
+        return out[:-1]
+
+    return run
+
+
+def test_partition_marks_read_the_removals_a_bounded_number_of_times(ask):
+    """Marks by ranges read all removals once per range: never more than 24 of
+    them, up to the largest list."""
+    sizes = [1 << b for b in range(10, 31)] + [(1 << 29) + 1, 3 << 28, (1 << 31) - 1]
+    qs = [("part", n, max(1, int(n / f))) for n in sizes for f in (1.01, 1.5, 2, 3.9, 4, 4.1, 11.9, 12, 12.1, 100)]
+    kinds = set()
+    for q, a in zip(qs, ask(qs)):
+        kinds.add(a.split()[0])
+        assert not a.startswith("ranges") or int(a.split()[1]) <= 24, (q, a)
+        if q[1] > 1 << 29:
+            assert a == "atomic", (q, a)
+    assert kinds == {"atomic", "ranges", "buckets"}
+
+
+def test_partition_marks_at_the_edges(ask):
+    assert ask([("part", 1 << 29, 1 << 27), ("part", (1 << 29) + 1, 1 << 27), ("part", 3 << 20, 1 << 19),
+                ("part", (3 << 20) + 1, 1 << 19), ("part", 12 << 15, 1 << 15), ("part", (12 << 15) + 1, 1 << 15),
+                ("part", 12 * ((1 << 19) - 1), (1 << 19) - 1), ("part", 1 << 28, (1 << 19) - 1),
+                ("part", 1 << 28, 1 << 19)]) == \
+        ["buckets", "atomic", "ranges 12", "buckets", "ranges 3", "atomic", "ranges 24", "atomic", "buckets"]

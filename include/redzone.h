@@ -85,7 +85,7 @@ typedef struct rz_tile_config {
                           several slices mark their tails through an LDS bitmap in 2 and 5),
                           4 = two kernels (mark, then move with in-kernel orphan pairing; slices longer than
                               the workgroup LDS allows run as variant 0),
-                          5 = dense form: head writes grouped by destination bin, then one scatter per bin
+                          5 = dense form: head writes grouped by destination bin, then written bin by bin
                               (for k/n of several percent and up),
                           6 = variant 4 in one launch: mark workgroups first, move slices after them wait for
                               the marks (same LDS limit and fallback as variant 4),
@@ -94,7 +94,7 @@ typedef struct rz_tile_config {
                               used; with premarked tails or RZ_COOPERATIVE: 256 x 4 of variant 4 or 1) */
   int32_t slice_steps; /* variant 2 and batches: steps per slice (0 = 4); variant 5: log2 of the target
                           number of destination bins, 3..12 (0 = 10; a bin is at least 512 KiB of the list,
-                          1 MiB for 16-byte items); variant 6: log2 of the removals
+                          1 MiB for 16-byte items and in lists above half a GiB); variant 6: log2 of the removals
                           each mark workgroup takes, 8..16 (0 = 12) */
   int32_t chunk;       /* variant 2 and batches: queue items taken per ticket (0 = 1) */
 } rz_tile_config;

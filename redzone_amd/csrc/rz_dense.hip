@@ -32,7 +32,9 @@
 //               whole lines where one entry per lane is 64 requests.  A bin's
 //               windows run on one XCD (workgroups go to the 8 XCDs round
 //               robin), whose L2 serves the entries to all of them.  Items
-//               that no removal names are neither read nor written.
+//               that no removal names are neither read nor written.  In
+//               lists above half a GiB where windows would read more than they
+//               save (dense_scatter), a bin's entries are stored one by one.
 //
 // Every array is refilled by each call; the look-back words and the cursors
 // are cleared by its first kernel.  The tail bitmap is zero on entry, set by
@@ -49,6 +51,7 @@
 #include <atomic>
 
 #include "rz_fused_dev.hpp"
+#include "rz_rules.hpp"
 
 namespace rz {
 
@@ -475,12 +478,35 @@ __global__ __launch_bounds__(1024) void rz_dense_write(T* __restrict__ A, Entrie
     if (((have[o >> 5] >> (o & 31u)) & 1u) && p0 + o < sZ) A[p0 + o] = win[o];
 }
 
+// Large or sparse lists (dense_scatter): a bin's entries split among G
+// workgroups on one XCD, one store per entry.  Bins in order, so an XCD writes
+// into one or two of them at a time and the stores combine in its L2.
+// Bound: those stores, 25 to 40 G/s.
+template <typename T>
+__global__ __launch_bounds__(1024) void rz_dense_scatter(T* __restrict__ A, Entries<T> fine,
+                                                         const uint32_t* __restrict__ fcur, uint32_t NBf, uint32_t bsf,
+                                                         uint32_t G, uint32_t sZ) {
+  const uint32_t x = blockIdx.x & 7u, rest = blockIdx.x >> 3;
+  const uint32_t g = rest % G, f = (rest / G) * 8u + x;
+  if (f >= NBf) return;
+  const uint32_t cnt = min(fcur[f], 1u << bsf), per = (cnt + G - 1) / G;
+  const uint32_t lo = min(g * per, cnt), hi = min(lo + per, cnt);
+  const size_t s = (size_t)f << bsf;
+  for (uint32_t q = lo + threadIdx.x; q < hi; q += 1024u) {
+    uint32_t p;
+    T v;
+    fine.get(s + q, p, v);
+    if (p < sZ) A[p] = v;
+  }
+}
+
 // ---------------------------------------------------------------------------
 // launch
 // ---------------------------------------------------------------------------
 struct DenseShape {
   uint32_t NBf, bsf;   // destination bins (multiple of 8)
-  uint32_t G, wlog;    // write windows per bin, log2 of a window's positions
+  bool scatter;        // single stores, else windows
+  uint32_t G, wlog;    // write workgroups per bin, log2 of a window's positions
   bool bucket_marks;   // tail marks grouped (else atomic, made by the caller)
 };
 
@@ -562,8 +588,11 @@ static rz_status dense_launch(rz_ctx* ctx, T* A, const int32_t* R, uint32_t k, u
   gb = (gb + kRegions - 1) / kRegions * kRegions;
   hipLaunchKernelGGL((rz_dense_bin<T, WG, D::BIN_IPT>), dim3(gb), dim3(WG), D::LDS, s, moves, region, mcur, dpos, src,
                      npairs, fine, fcur, d.NBf, d.bsf, ctrl);
-  hipLaunchKernelGGL(rz_dense_write<T>, dim3(d.NBf * d.G), dim3(1024), lds_win, s, A, fine, fcur, d.NBf, d.bsf, d.G,
-                     d.wlog, sZ);
+  if (d.scatter)
+    hipLaunchKernelGGL(rz_dense_scatter<T>, dim3(d.NBf * d.G), dim3(1024), 0, s, A, fine, fcur, d.NBf, d.bsf, d.G, sZ);
+  else
+    hipLaunchKernelGGL(rz_dense_write<T>, dim3(d.NBf * d.G), dim3(1024), lds_win, s, A, fine, fcur, d.NBf, d.bsf, d.G,
+                       d.wlog, sZ);
   RZ_HIP(hipGetLastError());
   return RZ_OK;
 }
@@ -591,12 +620,17 @@ static rz_status dense_shape(const rz_ctx* ctx, const rz_tile_config& cfg, uint3
   if (lg > 12) lg = 12;
   if (lg < 3) lg = 3;
   d.wlog = (uint32_t)log2_floor(kWindowBytes / esz);
-  d.bsf = std::max(bin_log(sZ, (int64_t)1 << lg), std::min(bin_log(sZ, 8), d.wlog + min_windows_log(esz)));
+  d.scatter = dense_scatter(esz, n, k);
+  if (d.scatter)
+    d.bsf = std::max(bin_log(sZ, (int64_t)1 << std::min<int>(lg, dense_scatter_bins_log(esz, n, k))),
+                     (uint32_t)log2_floor((1 << 20) / esz));
+  else
+    d.bsf = std::max(bin_log(sZ, (int64_t)1 << lg), std::min(bin_log(sZ, 8), d.wlog + min_windows_log(esz)));
   d.NBf = (uint32_t)((sZ + ((int64_t)1 << d.bsf) - 1) >> d.bsf);
   d.NBf = (d.NBf + 7u) & ~7u;
   d.bucket_marks = bucket_marks;
   if (d.wlog > d.bsf) d.wlog = d.bsf;
-  d.G = 1u << (d.bsf - d.wlog);
+  d.G = d.scatter ? (uint32_t)std::max(1, ctx->cu_count / 8) : 1u << (d.bsf - d.wlog);
   if (d.NBf > (uint32_t)kFineMax) return RZ_EINVAL;
   const size_t lds = (size_t)cfg.wg_size * cfg.items * (esz + 6) + 48 * 1024;  // the largest stage, and static LDS
   if (lds > (size_t)ctx->lds_max) return RZ_EINVAL;

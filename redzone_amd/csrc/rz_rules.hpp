@@ -54,4 +54,33 @@ inline uint32_t part_range_span(int64_t n) {
   return span;
 }
 
+// ---------------------------------------------------------------------------
+// the dense form's last step
+// ---------------------------------------------------------------------------
+// Whether a bin's entries are written one store per entry instead of through
+// LDS windows.  A window is 128 KiB of the list and reads all entries of its bin
+// to keep its own, and there are at most 4,096 bins: in larger lists a bin has
+// more windows, and with few entries per line of the list the windows save no
+// requests either.  Whole calls, windows / single stores, us:
+//   4 B, 2^28 items (1 GiB): k/n = 0.01 222 / 122, 0.125 858 / 833, 0.25 1,128 / 1,123, 0.4 1,396 / 1,412
+//   4 B, 2^31 items: k/n = 0.01 1,807 / 1,245, 0.06 5,787 / 4,952, 0.25 11,810 / 11,426, 0.4 25,736 / 27,050
+//   8 B, 2^27 items (1 GiB): k/n = 0.01 161 / 81, 0.125 704 / 667, 0.25 949 / 909, 0.4 1,130 / 1,061
+//   8 B, 2^29 items: k/n = 0.01 660 / 361, 0.06 1,852 / 1,678, 0.25 4,198 / 4,172, 0.4 5,032 / 4,773
+//   16 B, 2^26 items (1 GiB): k/n = 0.25 733 / 735, 0.4 881 / 889
+//   16 B, 2^27 items: k/n = 0.01 233 / 101, 0.125 998 / 938, 0.25 1,502 / 1,480, 0.4 1,767 / 1,817
+//   16 B, 2^29 items: k/n = 0.01 1,049 / 386, 0.06 2,700 / 2,060, 0.25 6,985 / 5,938, 0.4 8,350 / 7,185
+// Up to half a GiB (1 GiB of 16-byte items) the windows are as fast or faster.
+inline bool dense_scatter(uint32_t esz, int64_t n, int64_t k) {
+  const int64_t head = (n - k) * esz;
+  return head > (esz == 16 ? (int64_t)1 << 30 : (int64_t)1 << 29) &&
+         (esz == 8 || 3 * k < n || (esz == 16 && head > (int64_t)1 << 32));
+}
+// Then a bin is 1 MiB of the list or more, and the most bins (log2) are fewer for
+// larger items, whose shorter chunks leave the bin kernel shorter runs (s / 8 / 9 /
+// 11 for 512 / 2,048 bins: 16 B, 2^28 items, k/n = 0.125 1,944 / 1,983; 8 B, 2^28
+// items, k/n = 0.06 811 / 862, 0.25 2,050 / 1,887).
+inline uint32_t dense_scatter_bins_log(uint32_t esz, int64_t n, int64_t k) {
+  return esz == 4 ? 12 : esz == 8 && 16 * k >= n ? 11 : 9;
+}
+
 }  // namespace rz

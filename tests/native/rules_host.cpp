@@ -1,5 +1,6 @@
 // The rules of rz_rules.hpp at the sizes on stdin, one question a line:
-//   part <n> <k>   ->  atomic | buckets | ranges <number of ranges>
+//   part <n> <k>               ->  atomic | buckets | ranges <number of ranges>
+//   dense <elem_bytes> <n> <k> ->  windows | stores <log2 of the most bins>
 #include <cstdio>
 #include <cstring>
 
@@ -19,6 +20,11 @@ int main() {
           printf("ranges %lld\n", (n + span - 1) / span);
         }
       }
+    } else if (!strcmp(what, "dense")) {
+      long long e, n, k;
+      if (scanf("%lld %lld %lld", &e, &n, &k) != 3) return 1;
+      if (rz::dense_scatter((uint32_t)e, n, k)) printf("stores %u\n", rz::dense_scatter_bins_log((uint32_t)e, n, k));
+      else printf("windows\n");
     } else {
       return 1;
     }

@@ -40,3 +40,31 @@ def test_dense_keeps_unnamed_items(ctx):
     assert first_mismatch(dA.cpu()[keep].numpy(), A[keep].numpy()) < 0
     assert torch.equal(dR.cpu(), R)
     assert torch.equal(dA.cpu()[n - k:], A[n - k:])
+
+
+@pytest.mark.parametrize("esz,n,k", [(4, (1 << 28) + 77, (1 << 25) + 3), (8, (1 << 26) + 70001, 1 << 21),
+                                     (8, (1 << 27) - 3, 50000001), (16, (1 << 26) + (1 << 23) + 1, 1 << 20),
+                                     (16, (1 << 27) + 5, 40000003)])
+@pytest.mark.parametrize("pattern", ["uniform", "block"])
+def test_dense_single_stores(ctx, esz, n, k, pattern):
+    """Lists whose bins are written one store per entry: every item of the list
+    beside the three-kernel form's, removals at random and in one block (bins
+    filled to their last position)."""
+    announce("dense stores", esz, n, k, pattern)
+    A = torch.empty((n,) if esz == 4 else (n, esz // 4), dtype=torch.int32, device="cuda")
+    ctx.gen_payload(A, 11)
+    want = A.clone()
+    if pattern == "uniform":
+        R = torch.empty(k, dtype=torch.int32, device="cuda")
+        ctx.gen_uniform_removals(R, n, 12)
+    else:
+        R = torch.arange(1000, 1000 + k, dtype=torch.int32, device="cuda")
+    ctx.remove(want, R, config=rz.TileConfig(512, 8, 4096, 0, 0, 1), flags=rz.RZ_PRESERVE_REMOVALS)
+    for lg in (12, 11, 3):
+        B = A.clone()
+        cfg = rz.TileConfig(1024, 8 if esz < 16 else 4, 1024, 5, lg, 2)
+        assert ctx.remove(B, R, config=cfg, flags=rz.RZ_PRESERVE_REMOVALS) == n - k
+        assert ctx.check_errors() == 0
+        assert torch.equal(B[: n - k], want[: n - k]), lg
+        assert torch.equal(B[n - k:], A[n - k:]), "the red zone is only read"
+        del B

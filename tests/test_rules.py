@@ -43,3 +43,23 @@ def test_partition_marks_at_the_edges(ask):
                 ("part", 12 * ((1 << 19) - 1), (1 << 19) - 1), ("part", 1 << 28, (1 << 19) - 1),
                 ("part", 1 << 28, 1 << 19)]) == \
         ["buckets", "atomic", "ranges 12", "buckets", "ranges 3", "atomic", "ranges 24", "atomic", "buckets"]
+
+
+def test_dense_lists_that_windows_would_read_too_often(ask):
+    """The dense form writes through windows up to half a GiB of head (1 GiB of
+    16-byte items) and in denser lists above; sparse lists of several GiB never do."""
+    assert ask([("dense", 4, 1 << 27, 1 << 26), ("dense", 4, 1 << 28, 1 << 27), ("dense", 4, 1 << 28, 1 << 26),
+                ("dense", 4, (1 << 31) - 1, 1 << 24), ("dense", 4, (1 << 31) - 1, 9 << 27), ("dense", 8, 1 << 26, 1 << 24),
+                ("dense", 8, 1 << 29, 1 << 24), ("dense", 8, 1 << 29, 1 << 28), ("dense", 16, 1 << 26, 1 << 24),
+                ("dense", 16, 1 << 30, 1 << 24), ("dense", 16, 1 << 30, 3 << 28), ("dense", 16, 1 << 30, (3 << 28) - 1),
+                ("dense", 16, 1 << 28, 3 << 26)]) == \
+        ["windows", "windows", "stores 12", "stores 12", "windows", "windows", "stores 9", "stores 11", "windows",
+         "stores 9", "windows", "stores 9", "windows"]
+    for esz in (4, 8, 16):
+        sizes = [int(2 ** (b / 4)) for b in range(60, 125)]
+        qs = [("dense", esz, n, int(n * f)) for n in sizes for f in (.001, .01, .1, .3, .34, .5, .9)]
+        for (_, e, n, k), a in zip(qs, ask(qs)):
+            if n * e > 1 << 33 and 10 * k <= n:
+                assert a.startswith("stores"), (e, n, k)
+            if (n - k) * e <= 1 << 29:
+                assert a == "windows", (e, n, k)

@@ -398,15 +398,16 @@ __global__ __launch_bounds__(WG) void rz_dense_bin(Entries<T> moves, uint32_t re
     __syncthreads();
     const uint32_t cap = 1u << bsf, t1 = fresh_tid();
     // no branch and S stores whatever the chunk holds, so that the wait for
-    // the next chunk's loads behind them is one for the loads alone
+    // the next chunk's loads behind them is one for the loads alone; past the
+    // chunk's entries the last of them again
+    const uint32_t last = max(tot, 1u) - 1u;
 #pragma unroll
     for (int q = 0; q < IPT; ++q) {
-      const uint32_t e = q * WG + t1;
-      const uint32_t p = sd[e], fe = min(p >> bsf, NBf);
+      const uint32_t e = min(q * WG + t1, last);
+      const uint32_t p = sd[e], fe = min(p >> bsf, NBf - 1u);  // a chunk without entries only after a wait gave up
       const uint32_t r = s_bin[fe] + e;
-      const bool ok = e < tot && r < cap;
-      over |= e < tot && r >= cap;
-      fine.put(ok ? ((size_t)fe << bsf) + r : (size_t)NBf << bsf, p, sv[e]);
+      over |= tot && r >= cap;
+      fine.put(((size_t)fe << bsf) + min(r, cap - 1u), p, sv[e]);
       if (q % 4 == 3) sched_fence();
     }
     if (more) wait_loads();
@@ -547,8 +548,7 @@ static rz_status dense_launch(rz_ctx* ctx, T* A, const int32_t* R, uint32_t k, u
                               uint32_t* bits, uint32_t* ctrl, int stats, uint32_t src_cap, hipStream_t s) {
   using D = DenseTiles<T, WG, IPT>;
   const uint32_t nt = (k + D::S - 1) / D::S, region = region_entries(k, D::S);
-  // the bins, and one place for what has none
-  const size_t fcap = ((size_t)d.NBf << d.bsf) + 1, mcap = (size_t)kRegions * region;
+  const size_t fcap = (size_t)d.NBf << d.bsf, mcap = (size_t)kRegions * region;
   const size_t src_off = ((size_t)src_cap * sizeof(T) + 255) & ~(size_t)255;
   rz_status st;
   if ((st = ensure(ctx, ctx->dense_cnt, (size_t)nt * 8, s)) != RZ_OK) return st;

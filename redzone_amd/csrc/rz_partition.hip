@@ -409,7 +409,7 @@ template <int IPT, bool ALL>
 __global__ __launch_bounds__(1024) void rz_part_append(const int32_t* __restrict__ R, uint32_t k, uint32_t base,
                                                         uint32_t m, uint32_t blog, uint32_t nbins, uint32_t ntiles,
                                                         uint32_t* __restrict__ ent, uint32_t* __restrict__ cur,
-                                                        uint64_t* __restrict__ stat) {
+                                                        uint64_t* __restrict__ stat, uint32_t* __restrict__ none) {
   constexpr uint32_t kAppS = kAppWG * IPT;
   __shared__ uint32_t s_cnt[kPartMaxBins + 1], s_lbase[kPartMaxBins + 1];
   __shared__ uint32_t s_tmp[kAppWG / kWave + 1];
@@ -493,7 +493,7 @@ __global__ __launch_bounds__(1024) void rz_part_append(const int32_t* __restrict
       for (int j = 0; j < IPT; ++j) {
         const uint32_t t = j * kAppWG + t1, v = s_stage[t], bz = min(v >> blog, nbins), g = s_cnt[bz] + t;
         // a place past the bin's list only with duplicate removals, none only with indices out of range
-        ent[t < total && g < (1u << blog) ? ((size_t)bz << blog) + g : (size_t)nbins << blog] = v;
+        *(t < total && g < (1u << blog) ? ent + (((size_t)bz << blog) + g) : none) = v;
         if (j % 4 == 3) sched_fence();
       }
       wait_loads();
@@ -616,7 +616,7 @@ static rz_status append_launch(rz_ctx* ctx, const int32_t* R, int64_t k, uint32_
   // the big tile's LDS leaves one workgroup per CU, which then keeps its next tile's loads in flight
   const uint32_t grid = IPT == kAppIPTBig && tiles > (uint32_t)ctx->cu_count ? (uint32_t)ctx->cu_count : tiles;
   hipLaunchKernelGGL((rz_part_append<IPT, ALL>), dim3(grid), dim3(kAppWG), lds, s, R, (uint32_t)k, base, (uint32_t)m, blog,
-                     nbins, tiles, ent, cur, stat);
+                     nbins, tiles, ent, cur, stat, cur + 2 * kPartMaxBins);
   RZ_HIP(hipGetLastError());
   return RZ_OK;
 }
@@ -631,8 +631,9 @@ rz_status bucket_marks(rz_ctx* ctx, const int32_t* R, int64_t k, uint32_t base, 
   while (blog < max_blog && (m >> blog) > (big ? 256 : 512)) ++blog;
   const uint32_t nbins = (uint32_t)((m + (1ll << blog) - 1) >> blog);
   rz_status st;
-  if ((st = ensure(ctx, ctx->pent, ((size_t)nbins << (blog + 2)) + 4, s)) != RZ_OK) return st;
-  if ((st = ensure(ctx, ctx->pcur, (size_t)nbins * 8, s)) != RZ_OK) return st;  // counts, then done counters
+  if ((st = ensure(ctx, ctx->pent, (size_t)nbins << (blog + 2), s)) != RZ_OK) return st;
+  // counts, then done counters, and behind the most of them a place for removals that have none
+  if ((st = ensure(ctx, ctx->pcur, (size_t)(2 * kPartMaxBins + 1) * 4, s)) != RZ_OK) return st;
   const size_t lds_bits = (size_t)4 << (blog - 5);
   static std::atomic<uint64_t> attr_mask{0};
   const int dev = ctx->device;

@@ -125,8 +125,9 @@ rz_status rz_add_remove(rz_ctx* ctx, void* d_data, int64_t n, int64_t capacity, 
  * i < p, with P strictly ascending and P[p-1] < n (checked with RZ_VALIDATE).
  * The survivors keep their order.  One in-place pass (tiles write once the
  * earlier tiles with sources in their range have read them; no scratch for the
- * items), or, for p below 2^22 and n / 8, a gather into context scratch (p
- * items) and a copy back. */
+ * items), or, for p below 2^22 and n / 8 and for 4-byte lists with p a little
+ * below 2^22 (6 p + n from 25 to 40 million), a gather into context scratch
+ * (p items) and a copy back. */
 rz_status rz_gather_preserve(rz_ctx* ctx, void* d_data, int64_t n, uint32_t elem_bytes, const int32_t* d_keep,
                              int64_t p, uint32_t flags, void* stream);
 /* The mark step alone, into a caller-owned tail bitmap (zero beforehand),

@@ -7,10 +7,11 @@
 //    in its output range has read them.  At most two tiles do: the sources in
 //    T positions are at most T consecutive entries of P.  A tile finds them
 //    with a search over the tiles' first entries.
-//  - two passes (gather_sparse below): gather into context scratch with no ordering
+//  - two passes (gather_two_passes): gather into context scratch with no ordering
 //    between workgroups, then a device copy back to the front of the list.
 #include "rz_ctx.hpp"
 #include "rz_device.hpp"
+#include "rz_rules.hpp"
 
 namespace rz {
 
@@ -139,12 +140,7 @@ static rz_status gather_inplace_launch(rz_ctx* ctx, T* A, uint32_t n, const int3
   if ((st = ensure(ctx, ctx->ploaded, (size_t)tiles * kFlagStride * 4, s)) != RZ_OK) return st;
   if ((st = ensure(ctx, ctx->pgcnt, (size_t)groups * 4, s)) != RZ_OK) return st;
   uint32_t* ctrl = (uint32_t*)ctx->ctrl.ptr;
-  // Fewer than half of many 8- or 16-byte items kept: sources and outputs are
-  // far apart, and tiles that follow each other read and write them in longer
-  // stretches (2^24.5 of 2.5 p 16-byte items 258 us, 270 each on its own; 8-byte
-  // 146 and 149).  Dense and 4-byte lists lose by it (8-byte, 95% kept 104
-  // against 97).
-  const uint32_t follow = sizeof(T) >= 8 && p >= 1u << 22 && (uint64_t)p * 2 < n ? 32u : 0u;
+  const uint32_t follow = gather_follow(sizeof(T), n, p);
   hipLaunchKernelGGL((rz_gather_inplace<T, WG, IPT>), dim3(tiles), dim3(WG), 0, s, A, n, P, p,
                      (uint32_t*)ctx->ploaded.ptr, (uint32_t*)ctx->pgcnt.ptr, tiles, follow, ctrl);
   RZ_HIP(hipGetLastError());
@@ -164,17 +160,9 @@ static rz_status gather_launch(rz_ctx* ctx, T* A, uint32_t n, const int32_t* P, 
   return RZ_OK;
 }
 
-// Fewer than an eighth of the items kept, and fewer than 2^22: every item
-// comes from a page of its own, and many small workgroups with nothing to
-// wait for hide that better (p = 2^19 of 50 p 4-byte items: 11.2 us two passes,
-// 12.8-14 one; 500 p: 14.3 and 21).  From an eighth up one launch in place is
-// the faster one: 2^17 of 2.5 p 9.4 -> 7.0 us, 2^22 of 8-byte items
-// 25.5 -> 22.7 at 95% kept.
-static bool gather_sparse(int64_t n, int64_t p) { return p * 8 < n && p < ((int64_t)1 << 22); }
-
 template <typename T, int IPT>
 static rz_status gather_form(rz_ctx* ctx, void* A, int64_t n, const int32_t* P, int64_t p, hipStream_t s) {
-  if (gather_sparse(n, p)) return gather_launch<T, IPT>(ctx, (T*)A, (uint32_t)n, P, (uint32_t)p, s);
+  if (gather_two_passes(sizeof(T), n, p)) return gather_launch<T, IPT>(ctx, (T*)A, (uint32_t)n, P, (uint32_t)p, s);
   // Big tiles: every workgroup pays for its dispatch, flags and exit (2^21 of
   // 5 M 8-byte items: 245 tiles of 1,024 x 8 14.6 us, 489 of 512 x 8 18.6).
   // With a quarter of the CUs or fewer at work, half tiles win (2^19 of 2.5 p

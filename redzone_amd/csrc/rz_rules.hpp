@@ -83,4 +83,38 @@ inline uint32_t dense_scatter_bins_log(uint32_t esz, int64_t n, int64_t k) {
   return esz == 4 ? 12 : esz == 8 && 16 * k >= n ? 11 : 9;
 }
 
+// ---------------------------------------------------------------------------
+// the gather of preserved items
+// ---------------------------------------------------------------------------
+// Two passes (through scratch) instead of one in place, for p below 2^22.
+// Fewer than an eighth of the items kept: every item comes from a page of its own,
+// and many small workgroups with nothing to wait for hide that better (p = 2^19 of
+// 50 p 4-byte items: 11.2 us two passes, 12.8-14 one; 500 p: 14.3 and 21).  From an
+// eighth up one launch in place is the faster one: 2^17 of 2.5 p 9.4 -> 7.0 us,
+// 2^22 of 8-byte items 25.5 -> 22.7 at 95% kept.
+// 4-byte lists have a band (6 p + n from 25 to 40 M) where the one pass is a single
+// round of one or two tiles per CU whose waits nothing hides, two passes / one, us,
+// n = 1.3 p / 2.5 p / 4 p / 6 p:
+//   p = 2,300,000  12.7 / 11.4  13.4 / 12.2  14.5 / 14.3  15.8 / 15.9
+//   p = 3,000,000  14.9 / 13.8  14.8 / 15.9  16.2 / 18.3  18.6 / 19.3
+//   p = 3,600,000  15.7 / 16.5  16.5 / 18.7  18.6 / 19.0  22.1 / 21.9
+//   p = 4,194,299  16.8 / 19.2  18.3 / 20.6  21.3 / 21.6  25.6 / 25.0
+//   p = 5,000,000  21.8 / 19.1  23.6 / 21.0  26.6 / 23.9  31.8 / 28.7
+inline bool gather_two_passes(uint32_t esz, int64_t n, int64_t p) {
+  if (p >= (int64_t)1 << 22) return false;
+  return p * 8 < n || (esz == 4 && 6 * p + n >= 25000000 && 6 * p + n <= 40000000);
+}
+
+// Earlier tiles that a tile of the one pass waits for beside the two it has to.
+// Where sources and outputs are far apart, tiles that follow each other read and
+// write them in longer stretches (fewer than half of 2^24.5 items kept: 16-byte 258
+// us with 32, 270 without; 8-byte 146 and 149).  Dense lists lose by it (8-byte, 95%
+// kept 104 against 97), and 4-byte ones unless fewer than a quarter of many are kept:
+// with 16 / without, 2^26 of 4 p 293 / 311, of 8 p 476 / 502, 2^25 of 6 p 200 / 208,
+// 2^24 of 4 p 78 / 77.
+inline uint32_t gather_follow(uint32_t esz, int64_t n, int64_t p) {
+  if (esz == 4) return p >= 3 << 23 && p * 4 <= n ? 16 : 0;
+  return p >= 1 << 22 && p * 2 < n ? 32 : 0;
+}
+
 }  // namespace rz

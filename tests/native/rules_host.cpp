@@ -1,6 +1,7 @@
 // The rules of rz_rules.hpp at the sizes on stdin, one question a line:
 //   part <n> <k>               ->  atomic | buckets | ranges <number of ranges>
-//   dense <elem_bytes> <n> <k> ->  windows | stores <log2 of the most bins>
+//   dense <elem_bytes> <n> <k> ->  windows | stores <log2 of the most bins>//   gather <elem_bytes> <n> <p> ->  two | one <tiles followed>
+
 #include <cstdio>
 #include <cstring>
 
@@ -25,6 +26,11 @@ int main() {
       if (scanf("%lld %lld %lld", &e, &n, &k) != 3) return 1;
       if (rz::dense_scatter((uint32_t)e, n, k)) printf("stores %u\n", rz::dense_scatter_bins_log((uint32_t)e, n, k));
       else printf("windows\n");
+    } else if (!strcmp(what, "gather")) {
+      long long e, n, p;
+      if (scanf("%lld %lld %lld", &e, &n, &p) != 3) return 1;
+      if (rz::gather_two_passes((uint32_t)e, n, p)) printf("two\n");
+      else printf("one %u\n", rz::gather_follow((uint32_t)e, n, p));
     } else {
       return 1;
     }

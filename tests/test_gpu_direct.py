@@ -146,6 +146,24 @@ def test_gather_tiles(ctx, esz, p):
     assert ctx.check_errors() == 0
 
 
+@pytest.mark.parametrize("n,p", [(4000000, 3499999), (4000000, 3500000), (22000000, 3000000), (22000001, 3000000),
+                                 ((1 << 27) + 3, 3 << 23)])
+def test_gather_forms(ctx, n, p):
+    """4-byte gathers at the edges of the band that takes two passes, and a large
+    sparse one whose tiles follow each other."""
+    announce("gather forms", n, p)
+    A = torch.empty(n, dtype=torch.int32, device="cuda")
+    ctx.gen_payload(A, p)
+    R = torch.empty(p, dtype=torch.int32, device="cuda")
+    ctx.gen_uniform_removals(R, n, p + 1)
+    P = torch.sort(R).values.contiguous()
+    want = A[P.long()]
+    rest = A[p:].clone()
+    assert ctx.gather_preserve(A, P) == p
+    assert torch.equal(A[:p], want) and torch.equal(A[p:], rest)
+    assert ctx.check_errors() == 0
+
+
 @pytest.mark.parametrize("given", [False, True])
 def test_calls_run_on_the_stream_they_name(ctx, given):
     """The caller's current stream, or the stream it passes, on every call (not

@@ -63,3 +63,16 @@ def test_dense_lists_that_windows_would_read_too_often(ask):
                 assert a.startswith("stores"), (e, n, k)
             if (n - k) * e <= 1 << 29:
                 assert a == "windows", (e, n, k)
+
+
+def test_gather_forms(ask):
+    """Two passes for fewer than an eighth kept and in the band of 4-byte lists, never
+    from 2^22 kept items on."""
+    M = 1000000
+    assert ask([("gather", 4, 8 * 1000, 1000), ("gather", 4, 8 * 1000 + 1, 1000), ("gather", 4, 4 * M, 3500000 - 1),
+                ("gather", 4, 4 * M, 3500000), ("gather", 8, 4 * M, 3500000), ("gather", 4, 22 * M, 3 * M),
+                ("gather", 4, 22 * M + 1, 3 * M), ("gather", 4, 10 * M, 1 << 22), ("gather", 4, 10 * M, (1 << 22) - 1),
+                ("gather", 16, 1 << 26, 1 << 22), ("gather", 8, 1 << 23, 1 << 22), ("gather", 4, 1 << 28, 1 << 26),
+                ("gather", 4, (1 << 28) - 1, 1 << 26), ("gather", 4, 1 << 28, (3 << 23) - 1)]) == \
+        ["one 0", "two", "one 0", "two", "one 0", "two", "one 0", "one 0", "two", "one 32", "one 0", "one 16", "one 0",
+         "one 0"]

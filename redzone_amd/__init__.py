@@ -267,7 +267,7 @@ class Context:
 
     def last_stages(self):
         """Stage timeline (us from the first workgroup's start) of the last
-        fused-form call made with RZ_PROFILE (see rz_last_stages)."""
+        fused or direct call made with RZ_PROFILE (see rz_last_stages)."""
         out = (ctypes.c_float * 16)()
         self._call("rz_last_stages", self._h, out)
         return dict(zip(self.STAGE_NAMES, [round(v, 3) for v in out]))

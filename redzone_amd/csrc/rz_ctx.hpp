@@ -55,7 +55,7 @@ __device__ __forceinline__ bool stalled(const uint32_t* ctrl) {
 enum StampIndex : int {
   kStampStart = 0,     // the workgroup started
   kStampReady = 1,     // slice: the marks of this launch are in (one-launch form)
-  kStampLookback = 2,  // slice: the look-back (in the last step) has the earlier slices' orphan counts
+  kStampLookback = 2,  // slice: the look-back (in the last step) has the earlier slices' orphan counts; direct form: the maps
   kStampMoves = 3,     // slice: every step's moves issued
   kStampExchange = 4,  // slice: every orphan of the slice went through its exchange word
   kStampExit = 5,      // slice: left (after clearing its bitmap words and counting its exit)
@@ -123,7 +123,7 @@ struct rz_ctx {
   rz_tile_config table[3][33];    // [element size 4/8/16][floor(log2 k)]
   hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};  // RZ_PROFILE marks
   bool ev_recorded = false;
-  rz::DeviceBuffer stamps;     // RZ_PROFILE: stage stamps of the last fused call (StampIndex rows)
+  rz::DeviceBuffer stamps;     // RZ_PROFILE: stage stamps of the last fused or direct call (StampIndex rows)
   uint32_t stamp_groups = 0;   // rows written by that call (0: the last call had none)
   uint32_t stamp_marks = 0;    // of which mark workgroups (one-launch form)
   std::mutex mu;

@@ -323,10 +323,13 @@ __device__ __forceinline__ uint32_t select_bit(uint64_t m, uint32_t r) {
   return pos;
 }
 
-template <typename T, int WG, int IPT>
+// PROF: thread 0 stamps the wall clock (a kernel of its own: a test for the
+// stamps' address costs every other call 0.05 to 0.1 us).
+template <typename T, int WG, int IPT, bool PROF>
 __global__ __launch_bounds__(WG) void rz_direct(T* __restrict__ A, const int32_t* __restrict__ R, uint32_t k,
                                                  uint32_t sZ, const T* __restrict__ add, uint32_t split,
-                                                 uint32_t* __restrict__ ctrl, int stats) {
+                                                 uint32_t* __restrict__ ctrl, int stats,
+                                                 uint64_t* __restrict__ stamps) {
   extern __shared__ uint64_t s_direct[];
   __shared__ uint64_t s_tmp[WG / kWave + 1];
   const uint32_t W = (k + 63u) >> 6;
@@ -334,6 +337,10 @@ __global__ __launch_bounds__(WG) void rz_direct(T* __restrict__ A, const int32_t
   uint64_t* const dead = hole + W;       // bit i: red-zone item i was removed
   uint64_t* const pre = dead + W;        // orphans before a word: dest | source << 32
   const uint32_t tid = threadIdx.x;
+  auto stamp = [&](StampIndex at) {
+    if (PROF && tid == 0) stamps[(size_t)blockIdx.x * kStampsPerGroup + at] = wall_clock64();
+  };
+  stamp(kStampStart);
   const RedZone<T> Z{A + sZ, add, split};
   const uint32_t base = blockIdx.x * (WG * IPT);
   // this slice's pairs, loaded ahead of the maps
@@ -407,6 +414,7 @@ __global__ __launch_bounds__(WG) void rz_direct(T* __restrict__ A, const int32_t
     }
   }
   __syncthreads();
+  stamp(kStampLookback);
   // the dest orphans' sources first: a load after the moves would wait for them to drain
 #pragma unroll
   for (int j = 0; j < IPT; ++j) {
@@ -426,6 +434,9 @@ __global__ __launch_bounds__(WG) void rz_direct(T* __restrict__ A, const int32_t
 #pragma unroll
   for (int j = 0; j < IPT; ++j)
     if (d[j] < sZ) A[d[j]] = z[j];
+  stamp(kStampMoves);
+  if (PROF) wait_all_memory();
+  stamp(kStampExit);
 }
 
 // ---------------------------------------------------------------------------
@@ -593,13 +604,14 @@ static bool dispatch_move_pair(int wg, int ipt, hipStream_t s, T* A, const int32
 
 template <typename T>
 static bool dispatch_direct(int wg, int ipt, hipStream_t s, T* A, const int32_t* R, uint32_t k, uint32_t sZ,
-                            const T* add, uint32_t split, uint32_t* ctrl, int stats) {
+                            const T* add, uint32_t split, uint32_t* ctrl, int stats, uint64_t* stamps) {
   const size_t lds = (size_t)((k + 63) / 64) * 24;
   const uint32_t grid = (k + wg * ipt - 1) / (wg * ipt);
-#define RZ_DIRECT_CASE(W, I)                                                                                   \
-  if (wg == W && ipt == I) {                                                                                   \
-    hipLaunchKernelGGL((rz_direct<T, W, I>), dim3(grid), dim3(W), lds, s, A, R, k, sZ, add, split, ctrl, stats); \
-    return true;                                                                                               \
+#define RZ_DIRECT_CASE(W, I)                                                                                     \
+  if (wg == W && ipt == I) {                                                                                     \
+    auto* kern = stamps ? rz_direct<T, W, I, true> : rz_direct<T, W, I, false>;                                  \
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(W), lds, s, A, R, k, sZ, add, split, ctrl, stats, stamps);         \
+    return true;                                                                                                 \
   }
   RZ_DIRECT_CASE(256, 1) RZ_DIRECT_CASE(256, 2) RZ_DIRECT_CASE(256, 4)
   RZ_DIRECT_CASE(512, 1) RZ_DIRECT_CASE(512, 2) RZ_DIRECT_CASE(512, 4)
@@ -744,6 +756,17 @@ static rz_status dispatch_coop(int wg, int ipt, rz_ctx* ctx, T* A, int32_t* R, i
   return RZ_EINVAL;
 }
 
+// RZ_PROFILE: a zeroed row of stamps for each of `groups` workgroups, the first `marks` of them mark workgroups.
+static rz_status stamp_rows(rz_ctx* ctx, uint32_t groups, uint32_t marks, hipStream_t s, uint64_t** out) {
+  rz_status st;
+  if ((st = ensure(ctx, ctx->stamps, (size_t)groups * kStampsPerGroup * 8, s)) != RZ_OK) return st;
+  *out = (uint64_t*)ctx->stamps.ptr;
+  if ((st = fill_u32((uint32_t*)*out, 0u, (size_t)groups * kStampsPerGroup * 2, s)) != RZ_OK) return st;
+  ctx->stamp_groups = groups;
+  ctx->stamp_marks = marks;
+  return RZ_OK;
+}
+
 template <typename T>
 static rz_status plain_impl(rz_ctx* ctx, T* A, int64_t n, int32_t* R, int64_t k, uint32_t flags,
                             const rz_tile_config& cfg, bool coop, hipStream_t s, uint32_t* ext_bits, const T* add,
@@ -757,9 +780,14 @@ static rz_status plain_impl(rz_ctx* ctx, T* A, int64_t n, int32_t* R, int64_t k,
     uint32_t* ctrl = (uint32_t*)ctx->ctrl.ptr;
     const int stats = (flags & RZ_STATS) ? 1 : 0;
     if (stats && (st = fill_u32(ctrl + kCtrlStatTail, 0u, 2, s)) != RZ_OK) return st;
+    uint64_t* stamps = nullptr;
+    if ((flags & RZ_PROFILE) &&
+        (st = stamp_rows(ctx, (uint32_t)((k + cfg.wg_size * cfg.items - 1) / (cfg.wg_size * cfg.items)), 0u, s,
+                         &stamps)) != RZ_OK)
+      return st;
     if ((st = prof_mark(ctx, flags, 0, s)) != RZ_OK) return st;
     if ((st = prof_mark(ctx, flags, 1, s)) != RZ_OK) return st;
-    if (!dispatch_direct<T>(cfg.wg_size, cfg.items, s, A, R, (uint32_t)k, sZ, add, split, ctrl, stats))
+    if (!dispatch_direct<T>(cfg.wg_size, cfg.items, s, A, R, (uint32_t)k, sZ, add, split, ctrl, stats, stamps))
       return RZ_EINVAL;
     RZ_HIP(hipGetLastError());
     if ((st = prof_mark(ctx, flags, 2, s)) != RZ_OK) return st;
@@ -825,12 +853,7 @@ static rz_status plain_impl(rz_ctx* ctx, T* A, int64_t n, int32_t* R, int64_t k,
   if (fused && (flags & RZ_PROFILE)) {
     const uint32_t marks =
         one_launch ? mark_plan(n, k, L, cfg.slice_steps, (flags & RZ_SORTED) != 0).nm : 0u;
-    const uint32_t groups = ns + marks;
-    if ((st = ensure(ctx, ctx->stamps, (size_t)groups * kStampsPerGroup * 8, s)) != RZ_OK) return st;
-    stamps = (uint64_t*)ctx->stamps.ptr;
-    if ((st = fill_u32((uint32_t*)stamps, 0u, (size_t)groups * kStampsPerGroup * 2, s)) != RZ_OK) return st;
-    ctx->stamp_groups = groups;
-    ctx->stamp_marks = marks;
+    if ((st = stamp_rows(ctx, ns + marks, marks, s, &stamps)) != RZ_OK) return st;
   }
   if (one_launch) {
     if (!dispatch_mark_move_pair<T>(cfg.wg_size, cfg.items, s, A, R, (uint32_t)k, sZ, L, ns, bits,

@@ -80,6 +80,21 @@ def test_direct_flags(ctx, oracle):
             ctx.remove(dA, dR, config=bad)
 
 
+@pytest.mark.parametrize("k", [1, 97, 5000, 20001])
+def test_direct_stages(ctx, oracle, k):
+    """RZ_PROFILE on small removals through the tuned table: the slices' timeline,
+    without the stages that the direct form does not have."""
+    n = 3 * k + 40
+    A, R = W.payload(4, n, seed=k), W.uniform_removals(n, k, seed=k + 1)
+    announce("direct stages", k)
+    gpu_remove_parity(ctx, oracle, A, R, flags=rz.RZ_PROFILE)
+    st = ctx.last_stages()
+    assert st["slices"] == (k + 511) // 512 and st["mark_groups"] == 0
+    assert 0 <= st["first_slice_start"] <= st["last_slice_start"]
+    assert 0 < st["lookback_end"] <= st["moves_end"] <= st["exit"] < 10_000
+    assert st["marks_done"] == st["ready_raised"] == st["ready_wait_end"] == st["exchange_end"] == 0
+
+
 @pytest.mark.parametrize("esz", [4, 8, 16])
 @pytest.mark.parametrize("k,variant", [(300, 7), (5000, 7), (70001, 6), (70001, 4), (70001, 0)])
 def test_add_remove_sources(oracle, esz, k, variant):

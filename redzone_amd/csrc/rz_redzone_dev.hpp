@@ -55,7 +55,8 @@ __device__ __forceinline__ uint32_t next_word(uint32_t w) {
 // its runs of one word together, and one lane of a run makes the atomic.  (Equal words that are
 // not neighbours may be merged as well, which changes nothing.)  2^20 removals in a
 // row of 2.2 times as many items: partition 48.6 -> 26.3 us, removal 47.0 -> 30.7.
-// On every removal it costs random lists 1 us of 12, so a round asks first.
+// A kernel of many rows per thread asks first (below); rz_mark_all, one row at a
+// time, does without: random lists take 9.6 us of marks either way (k = 2^17).
 template <bool LDS>
 __device__ __forceinline__ void set_runs(uint32_t* __restrict__ bits, uint32_t z, bool hit) {
   const uint32_t w = hit ? z >> 5 : 0xffffffffu;
@@ -99,8 +100,13 @@ __device__ __forceinline__ void mark_body(const int32_t* __restrict__ R, uint32_
       most = max(most, (uint32_t)__popcll(ballot(r[u] - sZ < k)));
       if (STATS) hits += r[u] - sZ < k ? 1u : 0u;
     }
-    // Random lists stay below 32 of 64 (they mark one by one up to k / n = 0.24).  One
-    // question a round: a branch per removal cost 0.4 us of 133.
+    // One question a round (a branch per removal cost 0.4 us of 133): random lists
+    // stay below 32 hits of 64 up to k / n = 0.24 and mark one by one.  Denser random
+    // lists and sorted ones without neighbours in a word pay for the row shifts (12.8
+    // -> 13.2 us for k = 20,000 of 30,000, 8.1 -> 9.2 for 25,000 of 2^22 with
+    // RZ_SORTED); asking in addition whether neighbours share words, in all rows or
+    // in five, cost sorted dense and clustered lists as much (11.1 -> 11.5, 17.3 ->
+    // 20.3) as it gave those.
     if (__builtin_expect(most >= 32u, 0)) {
 #pragma unroll
       for (int u = 0; u < U; ++u) set_runs<false>(bits, r[u] - sZ, r[u] - sZ < k);

@@ -118,7 +118,8 @@ rz_status rz_remove_premarked(rz_ctx* ctx, void* d_data, int64_t n, uint32_t ele
  * zone lies inside the appended items, so every removal is a plain move of an
  * added item into its hole.  Added items that fall into the red zone are read
  * from d_add where the launch form allows it and then never written to the
- * list's end, which is scratch like every red zone. */
+ * list's end, which is scratch like every red zone.  When the removals are
+ * refused (RZ_VALIDATE), all g items have been appended and none removed. */
 rz_status rz_add_remove(rz_ctx* ctx, void* d_data, int64_t n, int64_t capacity, uint32_t elem_bytes,
                         const void* d_add, int64_t g, int32_t* d_removals, int64_t k, uint32_t flags, void* stream);
 /* In-place gather by a preserve list (paper p.14, eq. 3): A'[i] = A[P[i]] for

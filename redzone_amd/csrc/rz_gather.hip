@@ -232,11 +232,15 @@ rz_status rz_add_remove(rz_ctx* ctx, void* d_data, int64_t n, int64_t capacity, 
     if (copied > 0)
       RZ_HIP(hipMemcpyAsync(dst, add, (size_t)copied * elem_bytes, hipMemcpyDeviceToDevice, s));
     if (direct) {
-      rz_status st;
-      if ((flags & RZ_VALIDATE) && (st = launch_validate(ctx, d_removals, m, k, flags, s)) != RZ_OK) return st;
-      st = launch_plain(ctx, d_data, m, elem_bytes, d_removals, k, flags, cfg, s, nullptr,
-                        add + (size_t)copied * elem_bytes, (uint32_t)(g < k ? k - g : 0));
-      return st != RZ_OK ? st : finish_call(ctx, flags, s);
+      const size_t done = (size_t)copied * elem_bytes;
+      rz_status st = flags & RZ_VALIDATE ? launch_validate(ctx, d_removals, m, k, flags, s) : RZ_OK;
+      if (st == RZ_OK)
+        st = launch_plain(ctx, d_data, m, elem_bytes, d_removals, k, flags, cfg, s, nullptr, add + done,
+                          (uint32_t)(g < k ? k - g : 0));
+      if (st == RZ_OK) return finish_call(ctx, flags, s);
+      // refused: nothing is removed, and the items are appended all the same
+      if (done < bytes) (void)hipMemcpyAsync(dst + done, add + done, bytes - done, hipMemcpyDeviceToDevice, s);
+      return st;
     }
   }
   return rz_remove(ctx, d_data, m, elem_bytes, d_removals, k, flags, stream);

@@ -135,6 +135,31 @@ def test_add_remove_sources(oracle, esz, k, variant):
     ctx.close()
 
 
+@pytest.mark.parametrize("k", [500, 40000])
+@pytest.mark.parametrize("share", [0.4, 1, 2.5])
+@pytest.mark.parametrize("bad", ["duplicate", "range"])
+def test_add_remove_refused(oracle, k, share, bad):
+    """Removals that RZ_VALIDATE refuses: the added items are in the list behind the
+    others, and the corrected removals work on them."""
+    ctx = rz.Context(0)
+    n, g = 3 * k, int(share * k)
+    m = n + g
+    full, R = W.payload(8, m, seed=31), W.uniform_removals(m, k, seed=32)
+    cap = torch.zeros((m, 2), dtype=torch.int32, device="cuda")
+    cap[:n] = full[:n].cuda()
+    wrong = R.clone()
+    wrong[k // 2] = m if bad == "range" else wrong[3]
+    announce("add refused", k, share, bad)
+    with pytest.raises(rz.RedzoneError) as e:
+        ctx.add_remove(cap, n, full[n:].cuda(), wrong.cuda(), flags=rz.RZ_VALIDATE)
+    assert e.value.status == (2 if bad == "range" else 3)
+    assert torch.equal(cap.cpu(), full)
+    want = expected_canonical(oracle, full.numpy(), R.numpy())
+    assert ctx.remove(cap, R.cuda(), flags=rz.RZ_VALIDATE) == m - k
+    assert first_mismatch(cap[: m - k].cpu().numpy(), want[: m - k]) < 0
+    ctx.close()
+
+
 @pytest.mark.parametrize("esz", [4, 8, 16])
 @pytest.mark.parametrize("p", [1, 1000, 8192, 8193, 64 * 8192, 64 * 8192 + 1, 65 * 4096 + 3, (1 << 22) + 17])
 def test_gather_tiles(ctx, esz, p):

@@ -40,6 +40,7 @@
 #include "../../include/redzone_device.h"
 #include "rz_fused_dev.hpp"
 #include "rz_redzone_dev.hpp"
+#include "rz_rules.hpp"
 
 namespace rz {
 
@@ -306,8 +307,6 @@ __global__ __launch_bounds__(WG) void rz_mark_move_pair_sized(T* __restrict__ A,
 // 8.2 against 8.5 and 7.5 against 13.1; k = 2^15.5 (1024 x 1) 11.2 against
 // 8.8 and 10.1 against 13.5.  So the tuned table has it up to 2^15 removals.
 // ---------------------------------------------------------------------------
-constexpr uint32_t kDirectMaxK = 1u << 17;  // 24 bytes of LDS per 64 removals: 48 KiB
-
 // position of the r-th set bit of m (r below its count)
 __device__ __forceinline__ uint32_t select_bit(uint64_t m, uint32_t r) {
   uint32_t pos = 0;
@@ -956,7 +955,7 @@ static bool plain_shape_ok(const rz_ctx* ctx, const rz_tile_config& cfg, uint32_
     case 2: return wg_ok && (cfg.items == 4 || cfg.items == 8);
     case 5: return dense_shape_ok(ctx, cfg, esz, n, k, flags);
     case 7:
-      return k <= (int64_t)kDirectMaxK &&
+      return k <= kDirectMaxK &&
              (cfg.items == 1 || cfg.items == 2 ? wg_ok || cfg.wg_size == 1024 : wg_ok && cfg.items == 4);
     default: return false;
   }

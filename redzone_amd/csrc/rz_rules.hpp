@@ -55,6 +55,18 @@ inline uint32_t part_range_span(int64_t n) {
 }
 
 // ---------------------------------------------------------------------------
+// small removals: the direct form
+// ---------------------------------------------------------------------------
+constexpr int64_t kDirectMaxK = 1 << 17;  // 24 bytes of LDS per 64 removals: 48 KiB
+
+// Whether every k of the table's bucket of k, [2^b, 2^(b+1)), fits the form.
+inline bool direct_covers_bucket(int64_t k) {
+  int64_t top = 1;
+  while (top <= k) top *= 2;
+  return top - 1 <= kDirectMaxK;
+}
+
+// ---------------------------------------------------------------------------
 // the dense form's last step
 // ---------------------------------------------------------------------------
 // Whether a bin's entries are written one store per entry instead of through

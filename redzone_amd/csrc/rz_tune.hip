@@ -17,6 +17,7 @@
 
 #include "rz_ctx.hpp"
 #include "rz_device.hpp"
+#include "rz_rules.hpp"
 
 namespace rz {
 
@@ -92,9 +93,10 @@ static const rz_tile_config kCandidates[] = {
     {256, 4, 512, 4, 0, 1},   {256, 4, 2048, 4, 0, 1},  {256, 8, 512, 4, 0, 1},  {512, 8, 4096, 4, 0, 1},   // fused
     {256, 2, 4096, 4, 0, 1},  {256, 8, 4096, 4, 0, 1},
     {256, 4, 512, 6, 10, 1},  {256, 2, 4096, 6, 10, 1}, {256, 4, 512, 6, 12, 1}, {256, 8, 512, 6, 14, 1},  // one launch
-    {512, 4, 512, 6, 10, 1},  {512, 4, 512, 6, 12, 1},  {256, 4, 1024, 6, 11, 1},
-    {1024, 8, 1024, 5, 11, 2}, {1024, 8, 1024, 5, 12, 2}, {1024, 4, 1024, 5, 11, 2}, {512, 8, 2048, 5, 11, 2},  // dense
-    {1024, 8, 1024, 5, 11, 0},
+    {512, 4, 512, 6, 10, 1},  {512, 4, 512, 6, 12, 1},  {256, 4, 1024, 6, 11, 1}, {512, 8, 512, 6, 12, 1},
+    {512, 4, 768, 4, 0, 1},   {512, 8, 768, 4, 0, 1},   {512, 4, 512, 4, 0, 1},  // fused, slices in one round of workgroups
+    {1024, 8, 1024, 5, 11, 2}, {1024, 8, 1024, 5, 12, 2}, {1024, 4, 1024, 5, 11, 2}, {1024, 4, 1024, 5, 12, 2},  // dense
+    {512, 8, 2048, 5, 11, 2}, {1024, 8, 1024, 5, 11, 0},
     {512, 1, 0, 7, 0, 1},     {1024, 1, 0, 7, 0, 1},                                                        // direct
 };
 
@@ -105,7 +107,7 @@ static const rz_tile_config kBatchCandidates[] = {
     // fused items (a list's slices pair their orphans through look-back and exchange words)
     {256, 4, 0, 4, 4, 1}, {256, 8, 0, 4, 1, 1}, {256, 8, 0, 4, 2, 1}, {512, 8, 0, 4, 1, 1},
     {512, 8, 0, 4, 2, 1}, {512, 4, 0, 4, 2, 1}, {512, 8, 0, 4, 1, 2},
-    // bucketed tail marks for lists of 2^17 removals and more
+    // bucketed tail marks for lists of 2^19 removals and more
     {512, 8, 0, 5, 1, 1}, {512, 8, 0, 5, 2, 1}, {256, 8, 0, 5, 1, 1}, {512, 4, 0, 5, 2, 1},
 };
 
@@ -248,6 +250,11 @@ rz_status rz_tune(rz_ctx* ctx, uint32_t elem_bytes, int64_t n, int64_t k, const 
   int best_i = -1;
   float best_t = 0.f;
   for (int32_t c = 0; c < ncand && st == RZ_OK; ++c) {
+    // the winner stands for its whole bucket: not a form that refuses some of it
+    if (cands[c].variant == 7 && !direct_covers_bucket(k)) {
+      if (all_ms) all_ms[c] = -1.f;
+      continue;
+    }
     std::vector<float> ts;
     for (int32_t r = 0; r <= reps && st == RZ_OK; ++r) {
       if (hipMemcpyAsync(data, pristine, bytes, hipMemcpyDeviceToDevice, s) != hipSuccess ||

@@ -94,3 +94,24 @@ def test_committed_table_loads():
     ctx = rz.Context(0)
     assert ctx.tuned_table == _native.TUNED_TABLE
     ctx.close()
+
+
+def test_tuned_shape_covers_its_bucket(oracle):
+    """The direct form ends within the bucket of 2^17 removals: it is not installed for
+    it, whatever k of the bucket was timed."""
+    ctx = rz.Context(0)
+    before = ctx.table(4, 17).as_tuple()
+    n, k = 1 << 19, 1 << 17
+    direct, fused = rz.TileConfig(1024, 1, 0, 7, 0, 1), rz.TileConfig(256, 4, 512, 6, 12, 1)
+    announce("tune bucket 17")
+    with pytest.raises(rz.RedzoneError):
+        ctx.tune(4, n, k, candidates=[direct], reps=1, cold=False)
+    assert ctx.table(4, 17).as_tuple() == before
+    best, _, results = ctx.tune(4, n, k, candidates=[direct, fused], reps=1, cold=False)
+    assert best.as_tuple() == fused.as_tuple() and results[0][1] == -1
+    A, R = W.unique_u32_payload(n, seed=5), W.uniform_removals(n, k + 77, seed=6)
+    gpu_remove_parity(ctx, oracle, A, R)
+    best, _, _ = ctx.tune(4, n, (1 << 16) + 9, candidates=[direct], reps=1, cold=False)
+    assert best.as_tuple() == direct.as_tuple()
+    gpu_remove_parity(ctx, oracle, A, W.uniform_removals(n, (1 << 17) - 1, seed=7))
+    ctx.close()

@@ -76,3 +76,18 @@ def test_gather_forms(ask):
                 ("gather", 4, (1 << 28) - 1, 1 << 26), ("gather", 4, 1 << 28, (3 << 23) - 1)]) == \
         ["one 0", "two", "one 0", "two", "one 0", "two", "one 0", "one 0", "two", "one 32", "one 0", "one 16", "one 0",
          "one 0"]
+
+
+def test_installed_shapes_are_the_tuners():
+    """Every shape of the installed table is one that the tuner times, so tuning a
+    context again can find it."""
+    import redzone_amd as rz
+
+    plain = {c.as_tuple() for c in rz.Context.candidates()}
+    batch = {c.as_tuple() for c in rz.Context.candidates(batch=True)}
+    for line in open(os.path.join(ROOT, "redzone_amd", "tuned_gfx950.txt")):
+        words = line.split()
+        if words and words[0] == "plain":
+            assert tuple(map(int, words[3:])) in plain, line
+        elif words and words[0] == "batch":
+            assert tuple(map(int, words[1:])) in batch, line

@@ -610,7 +610,7 @@ bool dense_bucket_marks(const rz_tile_config& cfg, int64_t k, uint32_t flags) {
 static uint32_t min_windows_log(uint32_t esz) { return esz == 16 ? 3 : 2; }
 
 // The dense form's bins for (cfg, n, k); RZ_EINVAL when the shape cannot be
-// launched (LDS above the device's, or a workgroup shape with no kernel).  No
+// launched (some kernel's LDS above the device's, or a workgroup shape with none).  No
 // side effect, so a caller can check before it launches anything.
 static rz_status dense_shape(const rz_ctx* ctx, const rz_tile_config& cfg, uint32_t esz, int64_t n, int64_t k,
                              bool bucket_marks, DenseShape* out) {
@@ -632,8 +632,7 @@ static rz_status dense_shape(const rz_ctx* ctx, const rz_tile_config& cfg, uint3
   if (d.wlog > d.bsf) d.wlog = d.bsf;
   d.G = d.scatter ? (uint32_t)std::max(1, ctx->cu_count / 8) : 1u << (d.bsf - d.wlog);
   if (d.NBf > (uint32_t)kFineMax) return RZ_EINVAL;
-  const size_t lds = (size_t)cfg.wg_size * cfg.items * (esz + 6) + 48 * 1024;  // the largest stage, and static LDS
-  if (lds > (size_t)ctx->lds_max) return RZ_EINVAL;
+  if (dense_lds_bytes(esz, cfg.wg_size, cfg.items, d.scatter, d.wlog) > ctx->lds_max) return RZ_EINVAL;
   const bool kernel = (cfg.wg_size == 256 || cfg.wg_size == 512 || cfg.wg_size == 1024) &&
                       (cfg.items == 4 || cfg.items == 8);
   return kernel ? RZ_OK : RZ_EINVAL;

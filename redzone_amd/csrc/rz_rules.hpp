@@ -95,6 +95,14 @@ inline uint32_t dense_scatter_bins_log(uint32_t esz, int64_t n, int64_t k) {
   return esz == 4 ? 12 : esz == 8 && 16 * k >= n ? 11 : 9;
 }
 
+// LDS of the dense form's largest kernel: the split's and the bin kernel's stage with
+// their static part, or a window of 2^wlog positions and a bit for each.
+inline int64_t dense_lds_bytes(uint32_t esz, int wg, int items, bool scatter, uint32_t wlog) {
+  const int64_t stage = (int64_t)wg * items * (esz + 6) + 48 * 1024;
+  const int64_t window = scatter ? 0 : ((int64_t)esz << wlog) + ((int64_t)4 << wlog) / 32;
+  return stage > window ? stage : window;
+}
+
 // ---------------------------------------------------------------------------
 // the gather of preserved items
 // ---------------------------------------------------------------------------

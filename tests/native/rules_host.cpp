@@ -1,6 +1,7 @@
 // The rules of rz_rules.hpp at the sizes on stdin, one question a line:
 //   part <n> <k>               ->  atomic | buckets | ranges <number of ranges>
 //   dense <elem_bytes> <n> <k> ->  windows | stores <log2 of the most bins>//   gather <elem_bytes> <n> <p> ->  two | one <tiles followed>
+//   lds <elem_bytes> <wg> <items> <stores> <log2 of a window's positions>  ->  bytes
 
 #include <cstdio>
 #include <cstring>
@@ -31,6 +32,10 @@ int main() {
       if (scanf("%lld %lld %lld", &e, &n, &p) != 3) return 1;
       if (rz::gather_two_passes((uint32_t)e, n, p)) printf("two\n");
       else printf("one %u\n", rz::gather_follow((uint32_t)e, n, p));
+    } else if (!strcmp(what, "lds")) {
+      int e, wg, items, stores, wlog;
+      if (scanf("%d %d %d %d %d", &e, &wg, &items, &stores, &wlog) != 5) return 1;
+      printf("%lld\n", (long long)rz::dense_lds_bytes((uint32_t)e, wg, items, stores != 0, (uint32_t)wlog));
     } else {
       return 1;
     }

@@ -65,6 +65,19 @@ def test_dense_lists_that_windows_would_read_too_often(ask):
                 assert a == "windows", (e, n, k)
 
 
+def test_dense_shapes_count_every_kernels_lds(ask):
+    """A shape is refused before anything is launched where one of its kernels does
+    not fit: with 64 KiB a workgroup, every shape that writes whole windows.  All
+    installed and candidate shapes fit 160 KiB."""
+    small = [("lds", e, 256, 4, s, (1 << 17).bit_length() - 1 - {4: 2, 8: 3, 16: 4}[e]) for e in (4, 8, 16) for s in (0, 1)]
+    assert [int(a) > 65536 for a in ask(small)] == [True, False, True, False, True, True]
+    full = [("lds", e, wg, it, s, 17 - {4: 2, 8: 3, 16: 4}[e]) for e, wg, it in
+            ((4, 1024, 8), (8, 1024, 8), (16, 1024, 4), (16, 512, 8), (4, 512, 8)) for s in (0, 1)]
+    assert all(int(a) <= 163840 for a in ask(full))
+    assert int(ask([("lds", 16, 1024, 8, 0, 13)])[0]) > 163840  # refused, as it was
+    assert ask([("lds", 4, 256, 4, 0, 10), ("lds", 4, 256, 4, 0, 15)]) == ["59392", "135168"]
+
+
 def test_gather_forms(ask):
     """Two passes for fewer than an eighth kept and in the band of 4-byte lists, never
     from 2^22 kept items on."""

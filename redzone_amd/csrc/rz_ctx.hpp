@@ -84,7 +84,8 @@ struct rz_ctx {
   int max_wg_per_cu_256 = 0;  // occupancy of the cooperative kernel at 256 threads
   int lds_per_block = 65536;  // LDS bytes the fused form's orphan list may use (capped at 64 KiB)
   int lds_max = 65536;        // LDS bytes one workgroup may use on this device
-  // scratch, all zero-initialised on allocation and kept zero by the kernels
+  // scratch, zero-initialised on allocation; what has to be zero between calls is
+  // kept zero by the kernels, and reset_scratch clears it after a failed check
   rz::DeviceBuffer tail_bits;  // k bits: tail removals of the plain path
   rz::DeviceBuffer list_bits;  // n bits: removals of the O(n) path and validation
   rz::DeviceBuffer counts;     // per-slice orphan counts (uint64: dest | src << 32)
@@ -93,17 +94,19 @@ struct rz_ctx {
   rz::DeviceBuffer ploaded;    // partition and gather: per tile, the epoch once its items are loaded
   rz::DeviceBuffer pgcnt;      // gather: per 64 tiles, the number of them done (zero between calls)
   rz::DeviceBuffer ptrem;      // partition: removals per bin, then per tile (written by the bucketed marks)
-  rz::DeviceBuffer pent;       // partition's bucketed marks: per 2^19-position bin, its removals
-  rz::DeviceBuffer pcur;       // partition's bucketed marks: per bin its count, then per bin a done counter (zero between calls)
+  rz::DeviceBuffer pent;       // partition's bucketed marks: per bin of 2^15 to 2^20 positions, its removals (refilled by each call)
+  rz::DeviceBuffer pcur;       // partition's bucketed marks: per bin its count, then per bin a done counter (zero between calls), and a
+                               // place written by removals that have no bin
   rz::DeviceBuffer ctrl;       // control block (rz::CtrlWord)
   rz::DeviceBuffer queue;      // ticket / exit / done words of the single-list queue launch
   rz::DeviceBuffer mstatus;    // fused form: two halves of kMaxSlices look-back words, used alternately
   rz::DeviceBuffer slots;      // fused form: one exchange word per orphan rank (epoch | position + 1)
-  rz::DeviceBuffer dense_cnt;    // dense form: per-tile bin counts, then their per-bin prefixes
-  rz::DeviceBuffer dense_small;  // dense form: bin totals / bases, per-tile orphan counts / ranks
-  rz::DeviceBuffer dense_ent;    // dense form: coarse-bin head writes (positions, then values)
-  rz::DeviceBuffer dense_fine;   // dense form: fine-bin head writes (fixed capacity per bin)
-  rz::DeviceBuffer dense_src;    // dense form: source orphan values by rank
+  // dense form; every word is refilled by each call
+  rz::DeviceBuffer dense_cnt;    // look-back words of the split's tiles
+  rz::DeviceBuffer dense_small;  // move cursors per XCD, the number of orphan pairs, bin cursors
+  rz::DeviceBuffer dense_ent;    // moves as (position, value) entries, a region per XCD
+  rz::DeviceBuffer dense_fine;   // entries by destination bin (fixed capacity per bin)
+  rz::DeviceBuffer dense_src;    // source orphan values by rank, then dest orphan positions by rank
   rz::DeviceBuffer gstatus;    // preserve-list gather: the gathered items before they are copied back
   rz::DeviceBuffer dispatch;   // network parameters
   bool dispatch_ready = false; // parameters installed (else the k < n/2 rule)

@@ -65,9 +65,10 @@ rz_status scratch_address(int dev, unsigned char** out) {
   return RZ_OK;
 }
 
-// Launch shape by k (the tuned table's choice for 4-byte items): the one-launch
-// fused form for small k, the mark kernel then the fused move-and-pair kernel
-// from 2^19 removals on.
+// Launch shape by k: the one-launch fused form for small k, the mark kernel then
+// the fused move-and-pair kernel from 2^19 removals on.  One shape each for all
+// item sizes: the context's table has shapes by item size and bucket, and its direct
+// form below 2^15.
 rz_tile_config noalloc_shape(int64_t k) {
   rz_tile_config c;
   c.wg_size = 256;

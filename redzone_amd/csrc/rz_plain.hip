@@ -305,7 +305,11 @@ __global__ __launch_bounds__(WG) void rz_mark_move_pair_sized(T* __restrict__ A,
 // tuned fused shape, 4- and 16-byte items alike, us: k = 2^14 at k/n = 1% 7.2
 // (the caller's own rate) against 8.5, at 50% 7.3 against 12.5; k = 2^14.5
 // 8.2 against 8.5 and 7.5 against 13.1; k = 2^15.5 (1024 x 1) 11.2 against
-// 8.8 and 10.1 against 13.5.  So the tuned table has it up to 2^15 removals.
+// 8.8 and 10.1 against 13.5.  So the tuned table has it up to 2^15 removals.  From
+// a fourth round of 8,192 removals on (k above 24,576) it is 0.4 to 0.8 us slower
+// than a fused shape for random lists of 10 k items and more (k = 32,767 of 2^22:
+// 9.3 against 8.4), and 4 us faster for tail-heavy ones (8.7 against 12.8), which
+// the sizes do not tell apart.
 // ---------------------------------------------------------------------------
 // position of the r-th set bit of m (r below its count)
 __device__ __forceinline__ uint32_t select_bit(uint64_t m, uint32_t r) {
@@ -640,6 +644,8 @@ static int clamp_tile_log(int tile_log) {
 //   k = 2^23.3    388 -> 214 / 324 -> 283 / 276 -> 315 / 273 -> 332 / 302 -> 393
 // and much the same for 8- and 16-byte items.  The two meet at n = 4.3 k for
 // 2^19.5 and 2^20.5 and later for the others; the direct form has k below 2^15.
+// From 2^23 on the line lies elsewhere (between n = 2.2 k and 4 k at 2^23.3) and the
+// marks stay single: the table's shapes of 2^24 and up group them in buckets.
 static bool range_marks(int64_t n, int64_t k) { return k >= 1 << 15 && k < 1 << 23 && 4 * n <= 17 * k; }
 
 // The mark workgroups of a call: tiles of removals, or (ranges > 0) ranges of

@@ -1,6 +1,7 @@
 // The rules of rz_rules.hpp at the sizes on stdin, one question a line:
 //   part <n> <k>               ->  atomic | buckets | ranges <number of ranges>
-//   dense <elem_bytes> <n> <k> ->  windows | stores <log2 of the most bins>//   gather <elem_bytes> <n> <p> ->  two | one <tiles followed>
+//   dense <elem_bytes> <n> <k> ->  windows | stores <log2 of the most bins>
+//   gather <elem_bytes> <n> <p> ->  two | one <tiles followed>
 //   lds <elem_bytes> <wg> <items> <stores> <log2 of a window's positions>  ->  bytes
 
 #include <cstdio>
